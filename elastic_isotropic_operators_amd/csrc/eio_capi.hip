@@ -31,6 +31,7 @@
 #include "eio_step2.h"
 #include "eio_step2q.h"
 #include "eio_step3.h"
+#include "eio_resident.h"
 #include "eio_abc.h"
 #include "eio_abc_train.h"
 
@@ -217,6 +218,8 @@ struct Ctx {
     hipEvent_t fork = nullptr, join = nullptr;
     int persistent = 0;  // two-step NL forward in one persistent launch: 0 off, 1 on, 2 when it fits
     int spin_limit = 1 << 20;  // polls per neighbour wait of the persistent launch before it aborts
+    bool resident = true;      // false while a call is repeated with the launched kernels
+    int ncu = 0;               // compute units of the device
     std::map<int, FwiStore> fwi;
     int next_fwi = 1;
     bool fwi_ws_busy = false;  // a store holds the workspace's "fwi_ring" / "fwi_ck" buffers
@@ -509,7 +512,8 @@ void build_entries3(const ModelBase& m, const int* const pos[4], const int nreg[
 // entries on the step-1 region, receivers owned-only) and the two-step adjoint (56 x TX
 // tiles, receiver entries on the step-1 region: they are injected in both steps; source
 // entries owned-only: the NL adjoint reads them in both steps).
-enum class PlanKind { ONE, FWD2, ADJ2, FWD3 };
+// NONE: the shots' order and step counts only (resident loops build their own tiles).
+enum class PlanKind { ONE, FWD2, ADJ2, FWD3, NONE };
 
 template <typename T>
 Plan make_plan(Ctx* c, int nshot, const eio_shot* shots, Op op, PlanKind kind = PlanKind::ONE, int v2 = 0) {
@@ -528,6 +532,10 @@ Plan make_plan(Ctx* c, int nshot, const eio_shot* shots, Op op, PlanKind kind = 
     for (int oi = 0; oi < nshot; ++oi) {
         const eio_shot& s = shots[p.order[oi]];
         const ModelBase& m = get_model(c, s.model);
+        if (kind == PlanKind::NONE) {
+            p.nsteps.push_back(m.ntw - 1);
+            continue;
+        }
         const int nbz = (m.g.nz - 2 * eio::FAT + TZ - 1) / TZ;
         const int nbx = (m.g.nx - 2 * eio::FAT + TX - 1) / TX;
         std::vector<std::vector<eio::Entry>> src_t(size_t(nbz) * nbx), rec_t(size_t(nbz) * nbx);
@@ -666,7 +674,8 @@ bool nl_grouped(Ctx* c, int nshot, const eio_shot* shots, long long per_cell, lo
 template <typename T>
 Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
                const void* const dm_fwd[5], T* ring = nullptr, int wcap = 0, bool two_step = false,
-               bool adj2 = false, bool src2 = false, bool three_step = false, bool grouped = false) {
+               bool adj2 = false, bool src2 = false, bool three_step = false, bool grouped = false,
+               bool resident = false) {
     if (nshot <= 0) fail("nshot must be > 0");
     if (!shots) fail("shots is NULL");
     // the learned boundary is part of the NL forward only: the adjoint, Born and FWI passes
@@ -682,11 +691,13 @@ Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
     run.v2 = variant2_for(c, nshot, shots, grouped);
     run.v2a = variant2a_for(c, nshot, shots);
     run.v3 = variant3_for(c, nshot, shots);
-    run.plan = three_step ? make_plan<T>(c, nshot, shots, op, PlanKind::FWD3, run.v3)
+    run.plan = resident     ? make_plan<T>(c, nshot, shots, op, PlanKind::NONE)
+               : three_step ? make_plan<T>(c, nshot, shots, op, PlanKind::FWD3, run.v3)
                           : make_plan<T>(c, nshot, shots, op, two_step ? PlanKind::FWD2 : PlanKind::ONE, run.v2);
     if (adj2) run.plan2 = make_plan<T>(c, nshot, shots, op, PlanKind::ADJ2, run.v2a);
     if (src2) run.plan3 = make_plan<T>(c, nshot, shots, op, PlanKind::FWD2, run.v2);
-    const int nlev = (two_step || three_step || adj2 || src2) ? 4 : 2;  // state levels per shot
+    // state levels per shot (a resident loop from rest keeps its state on the chip)
+    const int nlev = resident ? 0 : (two_step || three_step || adj2 || src2) ? 4 : 2;
     const bool born = (op == Op::BORN_FWD || op == Op::BORN_ADJ);
     const bool fwi = (op == Op::FWI_FWD || op == Op::FWI_GRAD);
     const bool has_ss = born || op == Op::FWI_GRAD;
@@ -717,7 +728,7 @@ Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
             }
         }
     }
-    T* state = static_cast<T*>(ws_get(c, "state", state_elems * sizeof(T)));
+    T* state = state_elems ? static_cast<T*>(ws_get(c, "state", state_elems * sizeof(T))) : nullptr;
     T* trbuf = tr_elems ? static_cast<T*>(ws_get(c, "traces", tr_elems * sizeof(T))) : nullptr;
     T* ssbuf = ss_elems ? static_cast<T*>(ws_get(c, "ss", ss_elems * sizeof(T))) : nullptr;
     T* wbuf = w_elems ? static_cast<T*>(ws_get(c, "W", w_elems * sizeof(T))) : nullptr;
@@ -735,8 +746,10 @@ Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
         d.nz = m.g.nz; d.nx = m.g.nx; d.nts = m.g.nts; d.sub = m.g.sub_fd; d.h = m.h;
         d.ntw = m.ntw; d.minPad = m.g.minPad; d.surface = m.g.surface;
         for (int k = 0; k < 4; ++k) { d.cz[k] = T(m.cz[k]); d.cx[k] = T(m.cx[k]); }
-        d.A = state + so;
-        d.B = state + so + 5 * size_t(m.n);
+        if (nlev > 0) {
+            d.A = state + so;
+            d.B = state + so + 5 * size_t(m.n);
+        }
         if (two_step || three_step || adj2 || src2) {
             d.C = state + so + 10 * size_t(m.n);
             d.D = state + so + 15 * size_t(m.n);
@@ -802,9 +815,10 @@ Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
     }
     // ---- tables
     run.d_shots = static_cast<eio::ShotDev<T>*>(ws_get(c, "shots", sizeof(eio::ShotDev<T>) * nshot));
+    EIO_CHECK_HIP(hipMemcpyAsync(run.d_shots, run.sd.data(), sizeof(eio::ShotDev<T>) * nshot, h2d, c->stream));
+    if (resident) return run;
     run.d_tiles = static_cast<eio::TileDev*>(ws_get(c, "tiles", sizeof(eio::TileDev) * run.plan.tiles.size()));
     run.d_ents = static_cast<eio::Entry*>(ws_get(c, "ents", sizeof(eio::Entry) * std::max<size_t>(1, run.plan.ents.size())));
-    EIO_CHECK_HIP(hipMemcpyAsync(run.d_shots, run.sd.data(), sizeof(eio::ShotDev<T>) * nshot, h2d, c->stream));
     EIO_CHECK_HIP(hipMemcpyAsync(run.d_tiles, run.plan.tiles.data(), sizeof(eio::TileDev) * run.plan.tiles.size(), h2d, c->stream));
     if (!run.plan.ents.empty())
         EIO_CHECK_HIP(hipMemcpyAsync(run.d_ents, run.plan.ents.data(), sizeof(eio::Entry) * run.plan.ents.size(), h2d, c->stream));
@@ -1393,6 +1407,199 @@ void launch_persistent(Run<float>& run, const eio_shot* shots, int kmax) {
                                         "neighbour; the launch was abandoned (outputs are incomplete)"};
 }
 
+// ------------------------------------------------------------------ resident loops
+// Time loops of shots whose whole state stays on the chip (eio_resident.h): the shots of a call
+// (in plan order: decreasing step count) are split into consecutive groups, each one cooperative
+// launch whose tiles (64 x RES_WX*R cells, one workgroup per CU) fit the device.
+using eio::RES_WX;
+template <typename T>
+constexpr int res_max_r() { return sizeof(T) == 4 ? 5 : 2; }
+
+struct ResGroup {
+    int s0, s1;       // shots, in plan order
+    int R;            // columns per wave
+    int tile0, ntile;
+};
+struct ResPlan {
+    std::vector<ResGroup> groups;
+    std::vector<eio::ResTile> tiles;
+    std::vector<eio::Entry> ents;
+    eio::ResTile* d_tiles = nullptr;
+    eio::Entry* d_ents = nullptr;
+    void* inbox = nullptr;
+    size_t inbox_bytes = 0;
+    int* abort_flag = nullptr;
+    int* xcd = nullptr;     // the XCD each workgroup of a launch runs on
+};
+
+inline int res_tiles(const ModelBase& m, int R) {
+    return ((m.g.nz - 2 * eio::FAT + eio::TZ - 1) / eio::TZ) *
+           ((m.g.nx - 2 * eio::FAT + RES_WX * R - 1) / (RES_WX * R));
+}
+
+// Measured time of one fine step of a launch with R columns per wave [us] (every CU busy; the
+// halo exchange and the barriers are about 2.5 us of it, so wide tiles do the most work per
+// time, and narrow ones finish a call that cannot fill the device soonest).
+template <typename T>
+double res_step_us(int R) {
+    constexpr double f32[] = {3.4, 3.85, 5.05, 5.65, 7.0}, f64[] = {5.1, 6.15};
+    return sizeof(T) == 4 ? f32[R - 1] : f64[R - 1];
+}
+
+// The groups of a call, or none when a shot does not fit the device.
+template <typename T>
+std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots) {
+    const int n = int(plan.order.size());
+    std::vector<ResGroup> out;
+    int tile0 = 0;
+    for (int s0 = 0; s0 < n;) {
+        ResGroup best{s0, s0, 0, tile0, 0};
+        double cost = 0.0;
+        for (int R = 1; R <= res_max_r<T>(); ++R) {
+            int nt = 0, s1 = s0;
+            double work = 0.0;
+            while (s1 < n) {
+                const ModelBase& m = get_model(c, shots[plan.order[s1]].model);
+                const int k = res_tiles(m, R);
+                if (nt + k > c->ncu) break;
+                nt += k;
+                work += double(m.n) * plan.nsteps[s1];
+                ++s1;
+            }
+            if (s1 == s0) continue;
+            const double t = res_step_us<T>(R) * plan.nsteps[s0] / work;  // time per cell-update
+            if (!best.R || t < cost) {
+                best = {s0, s1, R, tile0, nt};
+                cost = t;
+            }
+        }
+        if (!best.R) return {};
+        out.push_back(best);
+        tile0 += best.ntile;
+        s0 = best.s1;
+    }
+    return out;
+}
+
+// Tiles and entries of the groups, their device tables and the exchange buffers.
+template <typename T>
+void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp) {
+    Ctx* c = run.c;
+    int maxR = 1;
+    for (const ResGroup& g : rp.groups) {
+        const int TX = RES_WX * g.R;
+        maxR = std::max(maxR, g.R);
+        // a tile's entries, grouped by the wave that owns their columns
+        auto by_wave = [&](std::vector<eio::Entry>& es, int* off) {
+            std::stable_sort(es.begin(), es.end(),
+                             [&](const eio::Entry& a, const eio::Entry& b) { return (a.lcell >> 8) / g.R < (b.lcell >> 8) / g.R; });
+            size_t i = 0;
+            for (int w = 0; w <= RES_WX; ++w) {
+                while (i < es.size() && (es[i].lcell >> 8) / g.R < w) ++i;
+                off[w] = int(rp.ents.size() + i);
+            }
+            rp.ents.insert(rp.ents.end(), es.begin(), es.end());
+        };
+        int base = 0;
+        for (int oi = g.s0; oi < g.s1; ++oi) {
+            const eio_shot& s = shots[run.plan.order[oi]];
+            const ModelBase& m = get_model(c, s.model);
+            const int nbz = (m.g.nz - 2 * eio::FAT + eio::TZ - 1) / eio::TZ;
+            const int nbx = (m.g.nx - 2 * eio::FAT + TX - 1) / TX;
+            std::vector<std::vector<eio::Entry>> src_t(size_t(nbz) * nbx), rec_t(size_t(nbz) * nbx);
+            build_entries<T>(m, s.src_pos, s.n_src, TX, src_t, nbz, "source");
+            build_entries<T>(m, s.rec_pos, s.n_rec, TX, rec_t, nbz, "receiver");
+            for (int bx = 0; bx < nbx; ++bx)
+                for (int bz = 0; bz < nbz; ++bz) {
+                    const int i = bx * nbz + bz;
+                    eio::ResTile t;
+                    t.shot = oi;
+                    t.z0 = eio::FAT + bz * eio::TZ;
+                    t.x0 = eio::FAT + bx * TX;
+                    t.up = bz > 0 ? base + i - 1 : -1;
+                    t.down = bz + 1 < nbz ? base + i + 1 : -1;
+                    t.left = bx > 0 ? base + i - nbz : -1;
+                    t.right = bx + 1 < nbx ? base + i + nbz : -1;
+                    by_wave(src_t[i], t.src);
+                    by_wave(rec_t[i], t.rec);
+                    rp.tiles.push_back(t);
+                }
+            base += nbz * nbx;
+        }
+    }
+    const hipMemcpyKind h2d = hipMemcpyHostToDevice;
+    rp.d_tiles = static_cast<eio::ResTile*>(ws_get(c, "res_tiles", sizeof(eio::ResTile) * rp.tiles.size()));
+    rp.d_ents = static_cast<eio::Entry*>(ws_get(c, "res_ents", sizeof(eio::Entry) * std::max<size_t>(1, rp.ents.size())));
+    EIO_CHECK_HIP(hipMemcpyAsync(rp.d_tiles, rp.tiles.data(), sizeof(eio::ResTile) * rp.tiles.size(), h2d, c->stream));
+    if (!rp.ents.empty())
+        EIO_CHECK_HIP(hipMemcpyAsync(rp.d_ents, rp.ents.data(), sizeof(eio::Entry) * rp.ents.size(), h2d, c->stream));
+    const size_t per_tile = 2 * (32 * size_t(RES_WX * maxR) + 2048);  // Inbox<TX>::TILE
+    int ntile = 0;
+    for (const ResGroup& g : rp.groups) ntile = std::max(ntile, g.ntile);
+    rp.inbox_bytes = size_t(ntile) * per_tile * eio::Packet<T>::BYTES;
+    rp.inbox = ws_get(c, "res_inbox", rp.inbox_bytes);
+    rp.abort_flag = static_cast<int*>(ws_get(c, "res_abort", 256));
+    rp.xcd = static_cast<int*>(ws_get(c, "res_xcd", size_t(c->ncu) * sizeof(int)));
+    fill0<int>(c, rp.abort_flag, 1);
+}
+
+// One launch of a group's fine steps [k0, k1).
+template <typename T, int MODE, bool FSURF>
+void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save,
+                    int dlo = 0, int dhi = -1) {
+    Ctx* c = run.c;
+    if (from_rest) {  // levels and inboxes of another group or call
+        fill0<T>(c, static_cast<T*>(rp.inbox), long(rp.inbox_bytes / sizeof(T)));
+    }
+    fill0<int>(c, rp.xcd, c->ncu);
+    const eio::ShotDev<T>* sh = run.d_shots;
+    const eio::ResTile* tt = rp.d_tiles + g.tile0;
+    const eio::Entry* te = rp.d_ents;
+    T* inbox = static_cast<T*>(rp.inbox);
+    unsigned ib = unsigned(rp.inbox_bytes);
+    int* ab = rp.abort_flag;
+    int* xc = rp.xcd;
+    int nt = g.ntile, fr = from_rest, sv = save, sl = c->spin_limit;
+    void* args[] = {&sh, &tt, &te, &inbox, &ib, &ab, &xc, &nt, &k0, &k1, &fr, &sv, &dlo, &dhi, &sl};
+    const void* fn = nullptr;
+    switch (g.R) {
+        case 1: fn = reinterpret_cast<const void*>(eio::k_res_fwd<T, 1, MODE, FSURF>); break;
+        case 2: fn = reinterpret_cast<const void*>(eio::k_res_fwd<T, 2, MODE, FSURF>); break;
+        default:
+            if constexpr (res_max_r<T>() > 2) {
+                fn = g.R == 3   ? reinterpret_cast<const void*>(eio::k_res_fwd<T, 3, MODE, FSURF>)
+                     : g.R == 4 ? reinterpret_cast<const void*>(eio::k_res_fwd<T, 4, MODE, FSURF>)
+                                : reinterpret_cast<const void*>(eio::k_res_fwd<T, 5, MODE, FSURF>);
+            }
+    }
+    EIO_CHECK_HIP(hipLaunchCooperativeKernel(fn, dim3(nt), dim3(64 * RES_WX), args, 0, c->stream));
+}
+
+// Whether the resident launches of this call gave up a wait (the call then repeats launched).
+inline bool res_aborted(Ctx* c, const ResPlan& rp) {
+    int aborted = 0;
+    EIO_CHECK_HIP(hipMemcpyAsync(&aborted, rp.abort_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    EIO_CHECK_HIP(hipStreamSynchronize(c->stream));
+    return aborted != 0;
+}
+
+// A context that leaves the launch form to the library, outside graphs, the persistent launch
+// and the no-allocation call; and a loop long enough for the set-up of a resident launch (tables,
+// cleared inboxes, a cooperative launch: some 60 us).  Whole calls, resident against launched:
+// 280 x 472 (45 tiles of 56 x 32) 396 against 373 us at 64 fine steps, 622 against 635 at 128;
+// 600 x 1592 (550 tiles) 262 against 249 us at 10, 310 against 352 at 18.
+constexpr int RES_MIN_STEPS = 96, RES_MIN_STEPS_WIDE = 16, RES_WIDE_TILES = 256;
+template <typename T>
+bool res_allowed(Ctx* c, int nshot, const eio_shot* shots) {
+    if (!c->resident || c->use_graph || c->persistent || c->bump || nshot <= 0 || !shots) return false;
+    if (sizeof(T) == 4 &&
+        (c->time_block != 2 || c->variant2 != EIO_VARIANT_AUTO || c->group_bytes != EIO_GROUP_AUTO))
+        return false;
+    int steps = 0;
+    for (int i = 0; i < nshot; ++i) steps = std::max(steps, get_model(c, shots[i].model).ntw - 1);
+    return steps >= RES_MIN_STEPS || (steps >= RES_MIN_STEPS_WIDE && wide_tiles(c, nshot, shots) >= RES_WIDE_TILES);
+}
+
 // Fine-step snapshots of one shot: after step steps[i] (after the boundary correction) the
 // older then the newer level, [nsnap][2][5][nx*nz].
 template <typename T>
@@ -1402,6 +1609,30 @@ struct Snap {
     T* out = nullptr;
 };
 
+// The NL forward with every shot resident; false when a shot does not fit or a wait was given up.
+template <typename T>
+bool nl_forward_resident(Ctx* c, int nshot, const eio_shot* shots, int flags, bool any_fs) {
+    ResPlan rp;
+    rp.groups = res_groups<T>(c, make_plan<T>(c, nshot, shots, Op::NL_FWD, PlanKind::NONE), shots);
+    if (rp.groups.empty()) return false;
+    Run<T> run = prepare<T>(c, nshot, shots, Op::NL_FWD, flags, nullptr, nullptr, 0, false, false, false, false, false, true);
+    res_build(run, shots, rp);
+    c->last_groups = int(rp.groups.size());
+    timing_begin<T>(c);
+    EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
+    for (const ResGroup& g : rp.groups) {
+        int kmax = run.plan.nsteps[g.s0];
+        if (c->step_limit > 0) kmax = std::min(kmax, c->step_limit);
+        if (any_fs) res_launch_fwd<T, eio::M_NL, true>(run, rp, g, 0, kmax, true, false);
+        else res_launch_fwd<T, eio::M_NL, false>(run, rp, g, 0, kmax, true, false);
+    }
+    EIO_CHECK_HIP(hipEventRecord(c->ev[3], c->stream));
+    timing_end<T>(c, (long long)rp.groups.size());
+    if (res_aborted(c, rp)) return false;
+    finish(run);
+    return true;
+}
+
 template <typename T>
 void nl_forward(Ctx* c, int nshot, const eio_shot* shots, int flags, int wshot = -1, void* wfld = nullptr,
                 int snap_shot = -1, int nsnap = 0, const int* snap_steps = nullptr, void* snap_out = nullptr) {
@@ -1410,6 +1641,9 @@ void nl_forward(Ctx* c, int nshot, const eio_shot* shots, int flags, int wshot =
     bool any_fs = false;
     for (int i = 0; i < nshot && shots; ++i) any_fs = any_fs || get_model(c, shots[i].model).g.surface;
     const bool abc = any_abc(c, nshot, shots);
+    if (res_allowed<T>(c, nshot, shots) && !wfld && !abc && nsnap == 0 &&
+        nl_forward_resident<T>(c, nshot, shots, flags, any_fs))
+        return;
     const bool plain = sizeof(T) == 4 && !wfld && !any_fs && !abc && nsnap == 0;
     const bool three = plain && c->time_block == 3;
     const bool two = plain && c->time_block == 2;
@@ -2114,6 +2348,7 @@ int eio_ctx_create(int device, int precision, eio_ctx** out) {
         c->prec = precision;
         try {
             c->scratch_dev = scratch_address(device);
+            EIO_CHECK_HIP(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device));
         } catch (...) {
             delete c;
             throw;

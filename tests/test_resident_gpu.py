@@ -1,0 +1,141 @@
+"""Resident time loops (csrc/eio_resident.h: one cooperative launch, the state on the chip) against
+the FP64 oracle, at the sizes where their tiles can go wrong: 64 rows by 16 R columns, R = 1..5,
+with remainders of one to four rows and columns, tiles that end on the grid's edge, more devices than
+a wave keeps in registers, uneven batches, and the repeat with launched kernels after a wait is given up.
+Bars: those of the launched kernels, FP32 1e-5 and FP64 1e-11 relative L2."""
+import numpy as np
+import pytest
+
+import oracle as O
+from elastic_isotropic_operators_amd import _capi
+from elastic_isotropic_operators_amd import workloads as W
+
+from helpers import GRID_OF_COMP, random_traces, rel_l2, scattered_positions
+
+pytestmark = pytest.mark.gpu
+
+TOL = {np.float32: 1e-5, np.float64: 1e-11}
+
+
+def _ctx(dtype):
+    ctx = _capi.Context(0, dtype)
+    if dtype == np.float32:
+        ctx.set_time_block(2, _capi.VARIANT_AUTO)
+        ctx.set_adjoint_time_block(2, _capi.VARIANT_AUTO)
+    return ctx
+
+
+def _model(ctx, nz, nx, nts, sub, seed, surface=0, pad=12):
+    """A padded grid of exactly nz x nx cells; (model id, oracle grid, media)."""
+    rng = np.random.default_rng(seed)
+    vp = 2200.0 + 900.0 * rng.random((1, nz)) + 60.0 * rng.random((nx, nz))
+    vs = vp / 1.8
+    rho = 1800.0 + 300.0 * rng.random((nx, 1)) + 0.0 * vp
+    g = O.grid(nz, nx, nts, sub, 10.0, 10.0, 0.0008 * sub / 2, pad, surface=surface)
+    med = O.media(g, np.stack([rho, rho * (vp * vp - 2 * vs * vs), rho * vs * vs]), np.float64)
+    mid = ctx.model_add(nz, nx, nts, sub, g.dz, g.dx, g.dts, pad, med, g.alphaCos, surface=surface)
+    return mid, g, med
+
+
+def _positions(rng, g, n, below=4):
+    p = scattered_positions(rng, g.nz, g.nx, n)
+    return [q[q % g.nz >= below] for q in p]
+
+
+def _forward_case(ctx, mid, g, med, rng, dtype, nsrc, nrec, below=4):
+    spos, rpos = _positions(rng, g, nsrc, below), _positions(rng, g, nrec, below)
+    src = random_traces(rng, spos, g.nts, np.float64)
+    ref = O.nl_fwd_reg(g, med, spos, src, rpos, np.float64)
+    rec = [np.zeros((rpos[GRID_OF_COMP[k]].size, g.nts), dtype) for k in range(5)]
+    shot, keep = ctx.make_shot(mid, spos, rpos, [np.ascontiguousarray(s, dtype) for s in src], rec)
+    return shot, keep, rec, ref
+
+
+def _check(rec, ref, dtype):
+    for k in range(5):
+        assert np.linalg.norm(ref[k]) > 0
+        assert rel_l2(rec[k], ref[k]) < TOL[dtype], (k, rel_l2(rec[k], ref[k]))
+
+
+@pytest.mark.parametrize("dtype,nz,nx,nsrc,nrec", [
+    (np.float32, 72, 24, 10, 20),       # one full tile of R = 1
+    (np.float32, 73, 25, 10, 20),       # one row and one column over
+    (np.float32, 76, 28, 10, 20),       # the four halo rows and columns exactly
+    (np.float32, 40, 90, 300, 700),     # more entries than a wave keeps in registers
+    (np.float32, 139, 61, 20, 40),
+    (np.float32, 281, 967, 40, 60),     # R = 2
+    (np.float32, 563, 1103, 40, 60),    # R = 3
+    (np.float32, 601, 1593, 40, 60),    # R = 4
+    (np.float32, 683, 1503, 40, 60),    # R = 5
+    (np.float64, 73, 25, 10, 20),
+    (np.float64, 40, 90, 300, 700),
+    (np.float64, 281, 967, 40, 60),     # R = 2
+])
+def test_forward_tiles(dtype, nz, nx, nsrc, nrec):
+    ctx = _ctx(dtype)
+    mid, g, med = _model(ctx, nz, nx, 51, 2, nz + nx)
+    rng = np.random.default_rng(nz * nx)
+    shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, dtype, nsrc, nrec)
+    ctx.nl_forward([shot])
+    assert ctx.last_timing()[1] == 1          # one launch
+    _check(rec, ref, dtype)
+    first = [r.copy() for r in rec]
+    ctx.nl_forward([shot])                     # the buffers of the first call are reused
+    for k in range(5):
+        assert np.array_equal(first[k], rec[k]), k
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_forward_uneven_batch(dtype):
+    """Shots of several grids, lengths and sub-samplings in one launch, odd counts among them."""
+    ctx = _ctx(dtype)
+    rng = np.random.default_rng(5)
+    cases = []
+    for i, (nz, nx, nts, sub) in enumerate([(90, 130, 50, 2), (150, 90, 27, 4), (61, 200, 33, 3), (75, 75, 90, 1)]):
+        mid, g, med = _model(ctx, nz, nx, nts, sub, 50 + i)
+        cases.append(_forward_case(ctx, mid, g, med, rng, dtype, 8, 20))
+    ctx.nl_forward([c[0] for c in cases])
+    for _, _, rec, ref in cases:
+        _check(rec, ref, dtype)
+    ctx.close()
+
+
+def test_forward_many_groups():
+    """More tiles than compute units: groups one after the other, each with its own inboxes."""
+    ctx = _ctx(np.float32)
+    rng = np.random.default_rng(6)
+    models = [_model(ctx, 200 + 3 * i, 700 + 50 * i, 50 + i, 2, 60 + i) for i in range(3)]
+    cases = [_forward_case(ctx, *models[i % 3], rng, np.float32, 5, 15) for i in range(9)]
+    ctx.nl_forward([c[0] for c in cases])
+    assert ctx.last_shot_groups() >= 2
+    for _, _, rec, ref in cases:
+        _check(rec, ref, np.float32)
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype,nz,nx", [(np.float32, 73, 25), (np.float32, 330, 601), (np.float64, 139, 90)])
+def test_forward_free_surface(dtype, nz, nx):
+    ctx = _ctx(dtype)
+    mid, g, med = _model(ctx, nz, nx, 51, 2, 7, surface=1)
+    rng = np.random.default_rng(8)
+    shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, dtype, 20, 40, below=9)
+    ctx.nl_forward([shot])
+    assert ctx.last_timing()[1] == 1
+    _check(rec, ref, dtype)
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_given_up_wait_repeats_with_launched_kernels(dtype):
+    """A spin limit of one poll ends the resident launch (every workgroup leaves at its next wait); the
+    call then runs its loop with launched kernels."""
+    ctx = _ctx(dtype)
+    ctx.set_persistent(0, 1)
+    mid, g, med = _model(ctx, 281, 301, 51, 2, 9)
+    rng = np.random.default_rng(10)
+    shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, dtype, 20, 40)
+    ctx.nl_forward([shot])
+    assert ctx.last_timing()[1] > 1
+    _check(rec, ref, dtype)
+    ctx.close()
