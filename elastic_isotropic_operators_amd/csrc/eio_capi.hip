@@ -160,6 +160,7 @@ struct FwiStore {
     void* ck = nullptr;          // (nseg-1) batch states
     void* ring = nullptr;        // per ordered shot: Vx then Vz, wcap slices each
     bool ring_fresh = false;     // the ring holds the last segment (true right after the forward)
+    bool resident = false;       // made by resident loops, which recompute its segments too
     bool ws = false;             // ring and checkpoints borrowed from the context workspace
     size_t bytes = 0;
 };
@@ -675,7 +676,7 @@ template <typename T>
 Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
                const void* const dm_fwd[5], T* ring = nullptr, int wcap = 0, bool two_step = false,
                bool adj2 = false, bool src2 = false, bool three_step = false, bool grouped = false,
-               bool resident = false) {
+               int resident = 0) {
     if (nshot <= 0) fail("nshot must be > 0");
     if (!shots) fail("shots is NULL");
     // the learned boundary is part of the NL forward only: the adjoint, Born and FWI passes
@@ -696,8 +697,9 @@ Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
                           : make_plan<T>(c, nshot, shots, op, two_step ? PlanKind::FWD2 : PlanKind::ONE, run.v2);
     if (adj2) run.plan2 = make_plan<T>(c, nshot, shots, op, PlanKind::ADJ2, run.v2a);
     if (src2) run.plan3 = make_plan<T>(c, nshot, shots, op, PlanKind::FWD2, run.v2);
-    // state levels per shot (a resident loop from rest keeps its state on the chip)
-    const int nlev = resident ? 0 : (two_step || three_step || adj2 || src2) ? 4 : 2;
+    // state levels per shot (resident = 1: none, the loop starts from rest and keeps its state
+    // on the chip; resident = 2: two, saved between launches)
+    const int nlev = resident == 1 ? 0 : resident == 2 ? 2 : (two_step || three_step || adj2 || src2) ? 4 : 2;
     const bool born = (op == Op::BORN_FWD || op == Op::BORN_ADJ);
     const bool fwi = (op == Op::FWI_FWD || op == Op::FWI_GRAD);
     const bool has_ss = born || op == Op::FWI_GRAD;
@@ -816,6 +818,7 @@ Run<T> prepare(Ctx* c, int nshot, const eio_shot* shots, Op op, int flags,
     // ---- tables
     run.d_shots = static_cast<eio::ShotDev<T>*>(ws_get(c, "shots", sizeof(eio::ShotDev<T>) * nshot));
     EIO_CHECK_HIP(hipMemcpyAsync(run.d_shots, run.sd.data(), sizeof(eio::ShotDev<T>) * nshot, h2d, c->stream));
+    if (state_elems && resident) fill0<T>(c, state, long(state_elems));
     if (resident) return run;
     run.d_tiles = static_cast<eio::TileDev*>(ws_get(c, "tiles", sizeof(eio::TileDev) * run.plan.tiles.size()));
     run.d_ents = static_cast<eio::Entry*>(ws_get(c, "ents", sizeof(eio::Entry) * std::max<size_t>(1, run.plan.ents.size())));
@@ -1412,9 +1415,6 @@ void launch_persistent(Run<float>& run, const eio_shot* shots, int kmax) {
 // (in plan order: decreasing step count) are split into consecutive groups, each one cooperative
 // launch whose tiles (64 x RES_WX*R cells, one workgroup per CU) fit the device.
 using eio::RES_WX;
-template <typename T>
-constexpr int res_max_r() { return sizeof(T) == 4 ? 5 : 2; }
-
 struct ResGroup {
     int s0, s1;       // shots, in plan order
     int R;            // columns per wave
@@ -1437,25 +1437,31 @@ inline int res_tiles(const ModelBase& m, int R) {
            ((m.g.nx - 2 * eio::FAT + RES_WX * R - 1) / (RES_WX * R));
 }
 
+// The passes that run resident and the widest tiles (columns per wave) their registers allow.
+enum class ResKind { NL, DEC };
+template <typename T>
+constexpr int res_max_r(ResKind k) {
+    return sizeof(T) == 8 ? 2 : k == ResKind::NL ? 6 : 5;
+}
 // Measured time of one fine step of a launch with R columns per wave [us] (every CU busy; the
 // halo exchange and the barriers are about 2.5 us of it, so wide tiles do the most work per
 // time, and narrow ones finish a call that cannot fill the device soonest).
 template <typename T>
-double res_step_us(int R) {
-    constexpr double f32[] = {3.4, 3.85, 5.05, 5.65, 7.0}, f64[] = {5.1, 6.15};
-    return sizeof(T) == 4 ? f32[R - 1] : f64[R - 1];
+double res_step_us(ResKind k, int R) {
+    constexpr double nl[] = {3.4, 3.85, 5.05, 5.65, 7.0, 8.7}, dec[] = {3.5, 4.0, 5.2, 5.8, 8.2}, f64[] = {5.1, 6.15};
+    return sizeof(T) == 8 ? f64[R - 1] : k == ResKind::NL ? nl[R - 1] : dec[R - 1];
 }
 
 // The groups of a call, or none when a shot does not fit the device.
 template <typename T>
-std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots) {
+std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) {
     const int n = int(plan.order.size());
     std::vector<ResGroup> out;
     int tile0 = 0;
     for (int s0 = 0; s0 < n;) {
         ResGroup best{s0, s0, 0, tile0, 0};
         double cost = 0.0;
-        for (int R = 1; R <= res_max_r<T>(); ++R) {
+        for (int R = 1; R <= res_max_r<T>(kind); ++R) {
             int nt = 0, s1 = s0;
             double work = 0.0;
             while (s1 < n) {
@@ -1467,7 +1473,7 @@ std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots
                 ++s1;
             }
             if (s1 == s0) continue;
-            const double t = res_step_us<T>(R) * plan.nsteps[s0] / work;  // time per cell-update
+            const double t = res_step_us<T>(kind, R) * plan.nsteps[s0] / work;  // time per cell-update
             if (!best.R || t < cost) {
                 best = {s0, s1, R, tile0, nt};
                 cost = t;
@@ -1543,16 +1549,16 @@ void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp) {
     fill0<int>(c, rp.abort_flag, 1);
 }
 
-// One launch of a group's fine steps [k0, k1).
-template <typename T, int MODE, bool FSURF>
+// One launch of a group's fine steps [k0, k1).  `dsh` replaces the run's shot table.
+template <typename T, int MODE, bool FSURF = false>
 void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save,
-                    int dlo = 0, int dhi = -1) {
+                    int dlo = 0, int dhi = -1, const eio::ShotDev<T>* dsh = nullptr) {
     Ctx* c = run.c;
-    if (from_rest) {  // levels and inboxes of another group or call
-        fill0<T>(c, static_cast<T*>(rp.inbox), long(rp.inbox_bytes / sizeof(T)));
-    }
+    constexpr int RMAX = res_max_r<T>((MODE & eio::F_DEC) ? ResKind::DEC : ResKind::NL);
+    // packets of another group, call or segment may carry the levels of this one
+    fill0<T>(c, static_cast<T*>(rp.inbox), long(rp.inbox_bytes / sizeof(T)));
     fill0<int>(c, rp.xcd, c->ncu);
-    const eio::ShotDev<T>* sh = run.d_shots;
+    const eio::ShotDev<T>* sh = dsh ? dsh : run.d_shots;
     const eio::ResTile* tt = rp.d_tiles + g.tile0;
     const eio::Entry* te = rp.d_ents;
     T* inbox = static_cast<T*>(rp.inbox);
@@ -1562,16 +1568,17 @@ void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, i
     int nt = g.ntile, fr = from_rest, sv = save, sl = c->spin_limit;
     void* args[] = {&sh, &tt, &te, &inbox, &ib, &ab, &xc, &nt, &k0, &k1, &fr, &sv, &dlo, &dhi, &sl};
     const void* fn = nullptr;
-    switch (g.R) {
-        case 1: fn = reinterpret_cast<const void*>(eio::k_res_fwd<T, 1, MODE, FSURF>); break;
-        case 2: fn = reinterpret_cast<const void*>(eio::k_res_fwd<T, 2, MODE, FSURF>); break;
-        default:
-            if constexpr (res_max_r<T>() > 2) {
-                fn = g.R == 3   ? reinterpret_cast<const void*>(eio::k_res_fwd<T, 3, MODE, FSURF>)
-                     : g.R == 4 ? reinterpret_cast<const void*>(eio::k_res_fwd<T, 4, MODE, FSURF>)
-                                : reinterpret_cast<const void*>(eio::k_res_fwd<T, 5, MODE, FSURF>);
-            }
-    }
+    auto pick = [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        if constexpr (R <= RMAX)
+            if (g.R == R) fn = reinterpret_cast<const void*>(eio::k_res_fwd<T, R, MODE, FSURF>);
+    };
+    pick(std::integral_constant<int, 1>{});
+    pick(std::integral_constant<int, 2>{});
+    pick(std::integral_constant<int, 3>{});
+    pick(std::integral_constant<int, 4>{});
+    pick(std::integral_constant<int, 5>{});
+    pick(std::integral_constant<int, 6>{});
     EIO_CHECK_HIP(hipLaunchCooperativeKernel(fn, dim3(nt), dim3(64 * RES_WX), args, 0, c->stream));
 }
 
@@ -1583,21 +1590,49 @@ inline bool res_aborted(Ctx* c, const ResPlan& rp) {
     return aborted != 0;
 }
 
+// While a call is repeated with the launched kernels.
+struct ResidentOff {
+    Ctx* c;
+    bool was;
+    explicit ResidentOff(Ctx* c_) : c(c_), was(c_->resident) { c->resident = false; }
+    ~ResidentOff() { c->resident = was; }
+};
+
 // A context that leaves the launch form to the library, outside graphs, the persistent launch
-// and the no-allocation call; and a loop long enough for the set-up of a resident launch (tables,
-// cleared inboxes, a cooperative launch: some 60 us).  Whole calls, resident against launched:
-// 280 x 472 (45 tiles of 56 x 32) 396 against 373 us at 64 fine steps, 622 against 635 at 128;
-// 600 x 1592 (550 tiles) 262 against 249 us at 10, 310 against 352 at 18.
-constexpr int RES_MIN_STEPS = 96, RES_MIN_STEPS_WIDE = 16, RES_WIDE_TILES = 256;
+// and the no-allocation call.
 template <typename T>
-bool res_allowed(Ctx* c, int nshot, const eio_shot* shots) {
-    if (!c->resident || c->use_graph || c->persistent || c->bump || nshot <= 0 || !shots) return false;
-    if (sizeof(T) == 4 &&
-        (c->time_block != 2 || c->variant2 != EIO_VARIANT_AUTO || c->group_bytes != EIO_GROUP_AUTO))
-        return false;
-    int steps = 0;
-    for (int i = 0; i < nshot; ++i) steps = std::max(steps, get_model(c, shots[i].model).ntw - 1);
-    return steps >= RES_MIN_STEPS || (steps >= RES_MIN_STEPS_WIDE && wide_tiles(c, nshot, shots) >= RES_WIDE_TILES);
+bool res_allowed(Ctx* c) {
+    if (!c->resident || c->use_graph || c->persistent || c->bump) return false;
+    return sizeof(T) == 8 ||
+           (c->time_block == 2 && c->variant2 == EIO_VARIANT_AUTO && c->group_bytes == EIO_GROUP_AUTO);
+}
+
+// The groups of a pass of `per_launch` fine steps a launch (0: each group's own steps), or none
+// where the launched kernels are the faster form.  Launched, a step takes (FP32, two per launch) 2.6
+// us and its cells at 100 GCell/s, 4.2 us at least; (FP64, one per launch) its cells at 22 GCell/s, 6
+// us at least.  A resident launch takes its steps and a set-up: cleared inboxes, a cooperative launch
+// and the state's first load, some 60 us, and 160 where the state comes from and goes back to memory
+// between segments.  Whole calls, resident against launched: 280 x 472, 396 against 373 us at 64 fine
+// steps, 622 against 635 at 128; 600 x 1592, 262 against 249 us at 10, 310 against 352 at 18; a
+// checkpointed gradient of four shots of 280 x 472 in segments of 46 steps, 43.7 against 37.4 ms.
+constexpr double RES_SETUP_US = 60.0, RES_SEGMENT_US = 160.0;
+template <typename T>
+std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
+    if (!res_allowed<T>(c)) return {};
+    std::vector<ResGroup> groups = res_groups<T>(c, plan, shots, kind);
+    double res = 0.0, work = 0.0;
+    int longest = 0;
+    for (const ResGroup& g : groups) {
+        const int steps = per_launch ? per_launch : plan.nsteps[g.s0];
+        res += (per_launch ? RES_SEGMENT_US : RES_SETUP_US) + steps * res_step_us<T>(kind, g.R);
+        longest = std::max(longest, steps);
+        for (int i = g.s0; i < g.s1; ++i)
+            work += double(get_model(c, shots[plan.order[i]].model).n) * (per_launch ? per_launch : plan.nsteps[i]);
+    }
+    const double launched = sizeof(T) == 4 ? std::max(4.2 * longest, 2.6 * longest + work / 100e3)
+                                           : std::max(6.0 * longest, work / 22e3);
+    if (res >= launched) groups.clear();
+    return groups;
 }
 
 // Fine-step snapshots of one shot: after step steps[i] (after the boundary correction) the
@@ -1613,9 +1648,9 @@ struct Snap {
 template <typename T>
 bool nl_forward_resident(Ctx* c, int nshot, const eio_shot* shots, int flags, bool any_fs) {
     ResPlan rp;
-    rp.groups = res_groups<T>(c, make_plan<T>(c, nshot, shots, Op::NL_FWD, PlanKind::NONE), shots);
+    rp.groups = res_choose<T>(c, make_plan<T>(c, nshot, shots, Op::NL_FWD, PlanKind::NONE), shots, ResKind::NL);
     if (rp.groups.empty()) return false;
-    Run<T> run = prepare<T>(c, nshot, shots, Op::NL_FWD, flags, nullptr, nullptr, 0, false, false, false, false, false, true);
+    Run<T> run = prepare<T>(c, nshot, shots, Op::NL_FWD, flags, nullptr, nullptr, 0, false, false, false, false, false, 1);
     res_build(run, shots, rp);
     c->last_groups = int(rp.groups.size());
     timing_begin<T>(c);
@@ -1641,7 +1676,7 @@ void nl_forward(Ctx* c, int nshot, const eio_shot* shots, int flags, int wshot =
     bool any_fs = false;
     for (int i = 0; i < nshot && shots; ++i) any_fs = any_fs || get_model(c, shots[i].model).g.surface;
     const bool abc = any_abc(c, nshot, shots);
-    if (res_allowed<T>(c, nshot, shots) && !wfld && !abc && nsnap == 0 &&
+    if (nshot > 0 && shots && !wfld && !abc && nsnap == 0 &&
         nl_forward_resident<T>(c, nshot, shots, flags, any_fs))
         return;
     const bool plain = sizeof(T) == 4 && !wfld && !any_fs && !abc && nsnap == 0;
@@ -1955,6 +1990,20 @@ void born_source_pass(Run<T>& run, int ntile, int kmax) {
     for (int k = 0; k < kmax; ++k) launch_fwd<T, eio::M_BSRC>(run, ntile, k, 0, 0, -1);
 }
 
+// The Born source pass with every shot resident; false when a shot does not fit or a wait was
+// given up (the launched pass then overwrites the record).
+template <typename T>
+bool born_source_resident(Run<T>& run, int nshot, const eio_shot* shots) {
+    Ctx* c = run.c;
+    ResPlan rp;
+    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::DEC);
+    if (rp.groups.empty()) return false;
+    res_build(run, shots, rp);
+    for (const ResGroup& g : rp.groups)
+        res_launch_fwd<T, eio::M_BSRC>(run, rp, g, 0, run.plan.nsteps[g.s0], true, false, 0, -1);
+    return !res_aborted(c, rp);
+}
+
 template <typename T>
 void born_forward(Ctx* c, int nshot, const eio_shot* shots, const void* const dm[5], int flags) {
     if (!dm) fail("dm is NULL");
@@ -1977,7 +2026,7 @@ void born_forward(Ctx* c, int nshot, const eio_shot* shots, const void* const dm
     timing_begin<T>(c);
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
     run_loop(c, [&]() {
-        born_source_pass(run, ntile, kmax);
+        if (!born_source_resident(run, nshot, shots)) born_source_pass(run, ntile, kmax);
         // scattered pass restarts from a zero state (BornElasticGpuFunctions.cu:773-774)
         for (int oi = 0; oi < nshot; ++oi) {
             fill0<T>(c, run.sd[oi].A, 5 * m.n);
@@ -2017,7 +2066,7 @@ void born_adjoint(Ctx* c, int nshot, const eio_shot* shots, void* const dm[5], i
     timing_begin<T>(c);
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
     run_loop(c, [&]() {
-        born_source_pass(run, ntile, kmax);
+        if (!born_source_resident(run, nshot, shots)) born_source_pass(run, ntile, kmax);
         for (int oi = 0; oi < nshot; ++oi) {
             fill0<T>(c, run.sd[oi].A, 5 * m.n);
             fill0<T>(c, run.sd[oi].B, 5 * m.n);
@@ -2117,6 +2166,38 @@ void copy_dev(Ctx* c, T* dst, const T* src, size_t n) {
 inline int seg_begin(const FwiStore& f, int j) { return j * f.L; }
 inline int seg_end(const FwiStore& f, int j) { return std::min((j + 1) * f.L, f.nts - 1); }
 
+// The forward of a store with every shot resident, segment by segment with the state saved in
+// between; false when a shot does not fit or a wait was given up.
+template <typename T>
+bool fwi_forward_resident(Ctx* c, int nshot, const eio_shot* shots, int flags, FwiStore& f) {
+    ResPlan rp;
+    rp.groups = res_choose<T>(c, make_plan<T>(c, nshot, shots, Op::FWI_FWD, PlanKind::NONE), shots, ResKind::DEC,
+                              std::min(f.L, f.nts - 1) * f.sub);
+    if (rp.groups.empty()) return false;
+    Run<T> run = prepare<T>(c, nshot, shots, Op::FWI_FWD, flags, nullptr, static_cast<T*>(f.ring), f.wcap, false, false,
+                            false, false, false, f.nseg > 1 ? 2 : 1);
+    res_build(run, shots, rp);
+    const size_t n10 = 10 * size_t(run.sd[0].nz) * run.sd[0].nx;
+    timing_begin<T>(c);
+    EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
+    for (const ResGroup& g : rp.groups)
+        for (int j = 0; j < f.nseg; ++j) {
+            // the batch state is one contiguous buffer in plan order, levels A, B of each shot
+            if (j > 0)
+                copy_dev<T>(c, static_cast<T*>(f.ck) + size_t(j - 1) * f.state_elems + g.s0 * n10, run.sd[g.s0].A,
+                            (g.s1 - g.s0) * n10);
+            const int k0 = seg_begin(f, j) * f.sub, k1 = seg_end(f, j) * f.sub;
+            if (j + 1 < f.nseg) res_launch_fwd<T, eio::M_NL>(run, rp, g, k0, k1, j == 0, true);
+            else res_launch_fwd<T, eio::M_NL | eio::F_DEC>(run, rp, g, k0, k1, j == 0, false, seg_begin(f, j), -1);
+        }
+    EIO_CHECK_HIP(hipEventRecord(c->ev[3], c->stream));
+    timing_end<T>(c, (long long)(f.nts - 1) * f.sub);
+    if (res_aborted(c, rp)) return false;
+    finish(run);
+    f.ring_fresh = f.resident = true;
+    return true;
+}
+
 template <typename T>
 int fwi_forward(Ctx* c, int nshot, const eio_shot* shots, int flags, int segment) {
     if (nshot <= 0 || !shots) fail("no shots");
@@ -2163,6 +2244,11 @@ int fwi_forward(Ctx* c, int nshot, const eio_shot* shots, int flags, int segment
         // steps stay inside one coarse interval because the fine sub-sampling is even, and
         // segments start at even fine steps
         const bool two = sizeof(T) == 4 && c->time_block >= 2 && sub % 2 == 0;
+        if (fwi_forward_resident<T>(c, nshot, shots, flags, f)) {
+            const int id = c->next_fwi++;
+            c->fwi[id] = f;
+            return id;
+        }
         Run<T> run = prepare<T>(c, nshot, shots, Op::FWI_FWD, flags, nullptr, static_cast<T*>(f.ring), f.wcap, two);
         const int ntile = int(run.plan.tiles.size());
         T* state = run.sd[0].A;  // the batch state is one contiguous buffer in plan order
@@ -2229,7 +2315,8 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
     const bool two = sizeof(T) == 4 && c->adj_time_block == 2 && f.sub % 2 == 0;
     // FP32: segments are recomputed two fine steps per launch (four levels per shot), the
     // kernel of the forward, so that a recomputed ring equals the forward's bit for bit
-    const bool rtwo = sizeof(T) == 4 && c->time_block >= 2 && f.sub % 2 == 0;
+    const bool rres = f.resident && c->resident && !c->use_graph;
+    const bool rtwo = !rres && sizeof(T) == 4 && c->time_block >= 2 && f.sub % 2 == 0;
     Run<T> run = prepare<T>(c, nshot, shots, Op::FWI_GRAD, flags, nullptr, static_cast<T*>(f.ring), f.wcap,
                             false, two, rtwo);
     const int ntile = int(run.plan.tiles.size());
@@ -2250,6 +2337,12 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
     auto* d_sdf = static_cast<eio::ShotDev<T>*>(ws_get(c, "shots_f", sizeof(eio::ShotDev<T>) * nshot));
     EIO_CHECK_HIP(hipMemcpyAsync(d_sdf, sdf.data(), sizeof(eio::ShotDev<T>) * nshot, hipMemcpyHostToDevice,
                                  c->stream));
+    ResPlan rp;
+    if (rres) {
+        rp.groups = res_groups<T>(c, make_plan<T>(c, nshot, shots, Op::FWI_GRAD, PlanKind::NONE), shots, ResKind::DEC);
+        if (rp.groups.empty()) throw EioError{EIO_ERR_STATE, "the device no longer takes the resident loop of this store"};
+        res_build(run, shots, rp);
+    }
     long long nrecomp = 0;
     for (int j = 0; j + 1 < f.nseg; ++j) nrecomp += (long long)(seg_end(f, j) - seg_begin(f, j)) * sub;
     timing_begin<T>(c);
@@ -2278,6 +2371,12 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
                 return;
             }
         }
+        if (rres) {
+            if (j > 0) copy_dev<T>(c, fstate, static_cast<const T*>(f.ck) + size_t(j - 1) * f.state_elems, f.state_elems);
+            for (const ResGroup& g : rp.groups)
+                res_launch_fwd<T, eio::M_RECOMP>(run, rp, g, k0, k1, j == 0, false, seg_begin(f, j), dhi, d_sdf);
+            return;
+        }
         if (j == 0) fill0<T>(c, fstate, long(f.state_elems));
         else copy_dev<T>(c, fstate, static_cast<const T*>(f.ck) + size_t(j - 1) * f.state_elems, f.state_elems);
         for (int k = k0; k < k1; ++k) launch_fwd<T, eio::M_RECOMP>(run, ntile, k, 0, seg_begin(f, j), dhi, d_sdf);
@@ -2305,6 +2404,11 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
     });
     EIO_CHECK_HIP(hipEventRecord(c->ev[3], c->stream));
     timing_end<T>(c, (long long)(nts - 1) * sub + nrecomp);
+    if (rres && res_aborted(c, rp)) {  // a wait was given up: the whole sweep again, launched
+        ResidentOff off(c);
+        fwi_gradient<T>(c, handle, nshot, shots, dm, flags);
+        return;
+    }
     stack_into(run, m, nshot, dm, flags);
     finish(run);
 }

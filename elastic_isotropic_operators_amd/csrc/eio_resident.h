@@ -341,6 +341,10 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
     constexpr bool DEC = (MODE & F_DEC) != 0;
     constexpr bool PAIR = sizeof(T) == 4 && !FSURF;
     constexpr bool PIN = sizeof(T) == 8 || FSURF || R >= 4;
+    // the widest tiles read the media again each step (20 B a cell, from L2) where registers end
+    // (R = 5: 7.0 us a step with the media in registers and 10 spilled ones, 7.8 without them)
+    constexpr bool MEML2 = sizeof(T) == 4 && (R >= 6 || (R >= 5 && DEC));
+    constexpr int RM = MEML2 ? 1 : R;
     __shared__ __attribute__((aligned(16))) T L[5][TXH][ZH];
     __shared__ int s_stop;
 
@@ -365,17 +369,18 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
     const T* filt = S.filt;
 
     if (tid == 0) s_stop = 0;
-    T o[5][R], m[5][R], d[R];
+    T o[5][R], m[5][RM], d[R];
+    const rsrc_t rmed = make_rsrc(S.med, 5 * fbytes);
 #pragma unroll
     for (int r = 0; r < R; ++r) d[r] = zok && r < ncol ? damp_at(S, iz, ix0 + r) : T(1);
     {
-        const rsrc_t rold = make_rsrc(S.A, 5 * fbytes), rcur = make_rsrc(S.B, 5 * fbytes), rmed = make_rsrc(S.med, 5 * fbytes);
+        const rsrc_t rold = make_rsrc(S.A, 5 * fbytes), rcur = make_rsrc(S.B, 5 * fbytes);
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
             for (int f = 0; f < 5; ++f) {
                 const unsigned so = unsigned(r) * colb + unsigned(f) * fbytes;
-                m[f][r] = zok && r < ncol ? bld<T>(rmed, voff, so) : T(0);
+                if (!MEML2) m[f][MEML2 ? 0 : r] = zok && r < ncol ? bld<T>(rmed, voff, so) : T(0);
                 o[f][r] = !from_rest && zok && r < ncol ? bld<T>(rold, voff, so) : T(0);
             }
         for (int e = tid; e < TXH * ZH; e += NT) {
@@ -502,28 +507,37 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
         }
     };
     // z derivatives and the update: the next level into o
+    T mnext[5];
+    auto load_media = [&](int r) {
+#pragma unroll
+        for (int f = 0; f < 5; ++f) mnext[f] = zok && r < ncol ? bld<T>(rmed, voff, unsigned(r) * colb + unsigned(f) * fbytes) : T(0);
+    };
     auto update = [&](bool odd) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
+            T mm[5];
+#pragma unroll
+            for (int f = 0; f < 5; ++f) mm[f] = MEML2 ? mnext[f] : m[f][MEML2 ? 0 : r];
+            if (MEML2 && r + 1 < R) load_media(r + 1);
             const T s0 = dxx[r] + dp_l(lds_at<T>(laz, 4 * FS + r * ZH), cz);
             const T s1 = dm_l(lds_at<T>(laz, 3 * FS + r * ZH), cz) + dxz[r];
             const T vzz = dp_l(lds_at<T>(laz, FS + r * ZH), cz);
             const T sh = dm_l(lds_at<T>(laz, r * ZH), cz) + vzx[r];
             T a0, a1, a2, a3, a4;
             if (!FSURF || !fs_top) {
-                a0 = upd_velocity<T, PAIR>(d[r], o[0][r], m[0][r], s0);
-                a1 = upd_velocity<T, PAIR>(d[r], o[1][r], m[1][r], s1);
-                a2 = upd_normal<T, PAIR>(d[r], o[2][r], m[2][r], vxx[r], m[3][r], vzz);
-                a3 = upd_normal<T, PAIR>(d[r], o[3][r], m[3][r], vxx[r], m[2][r], vzz);
-                a4 = upd_shear<T, PAIR>(odd, d[r], o[4][r], m[4][r], sh);
+                a0 = upd_velocity<T, PAIR>(d[r], o[0][r], mm[0], s0);
+                a1 = upd_velocity<T, PAIR>(d[r], o[1][r], mm[1], s1);
+                a2 = upd_normal<T, PAIR>(d[r], o[2][r], mm[2], vxx[r], mm[3], vzz);
+                a3 = upd_normal<T, PAIR>(d[r], o[3][r], mm[3], vxx[r], mm[2], vzz);
+                a4 = upd_shear<T, PAIR>(odd, d[r], o[4][r], mm[4], sh);
             } else {  // kernelsGpuElastic.cu:589-776, as in k_step_fwd
                 const bool on = iz == SURF, below = iz > SURF;
-                a0 = d[r] * o[0][r] + ((on || below) ? m[0][r] * s0 : T(0));
-                a1 = d[r] * o[1][r] + (below ? m[1][r] * s1 : T(0));
-                a2 = d[r] * o[2][r] + (below ? (m[2][r] * vxx[r] + m[3][r] * vzz)
-                                             : (on ? (m[2][r] - m[3][r] * m[3][r] / m[2][r]) * vxx[r] : T(0)));
-                a3 = d[r] * o[3][r] + (below ? (m[3][r] * vxx[r] + m[2][r] * vzz) : T(0));
-                a4 = d[r] * o[4][r] + (below ? m[4][r] * sh : T(0));
+                a0 = d[r] * o[0][r] + ((on || below) ? mm[0] * s0 : T(0));
+                a1 = d[r] * o[1][r] + (below ? mm[1] * s1 : T(0));
+                a2 = d[r] * o[2][r] + (below ? (mm[2] * vxx[r] + mm[3] * vzz)
+                                             : (on ? (mm[2] - mm[3] * mm[3] / mm[2]) * vxx[r] : T(0)));
+                a3 = d[r] * o[3][r] + (below ? (mm[3] * vxx[r] + mm[2] * vzz) : T(0));
+                a4 = d[r] * o[4][r] + (below ? mm[4] * sh : T(0));
             }
             o[0][r] = d[r] * a0;
             o[1][r] = d[r] * a1;
@@ -554,6 +568,7 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
         }
         __syncthreads();  // the halos are staged
         if (s_stop) return;
+        if (MEML2) load_media(0);
         if (edge) dx_all(js, j2);
         update(k & 1);
         __syncthreads();  // every read of level k is done

@@ -139,3 +139,40 @@ def test_given_up_wait_repeats_with_launched_kernels(dtype):
     assert ctx.last_timing()[1] > 1
     _check(rec, ref, dtype)
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype,nz,nx,segment", [(np.float32, 139, 90, 0), (np.float32, 281, 967, 0), (np.float32, 563, 1103, 26),
+                                                 (np.float64, 139, 90, 0), (np.float64, 281, 967, 26)])
+def test_fwi_record_and_checkpoints(dtype, nz, nx, segment):
+    """FWI forward and gradient with the forward (whole record, or checkpoints whose segments are long enough
+    for a resident launch) and the recompute resident: data and gradient against the oracle, a second gradient
+    (which recomputes every segment) bit for bit, and both again after a given-up wait."""
+    ctx = _ctx(dtype)
+    nts, sub = 80, 4
+    mid, g, med = _model(ctx, nz, nx, nts, sub, 11)
+    rng = np.random.default_rng(12)
+    spos, rpos = _positions(rng, g, 10), _positions(rng, g, 30)
+    src = random_traces(rng, spos, nts, np.float64)
+    dat = random_traces(rng, rpos, nts, np.float64)
+    fine = [O.time_interp(s, g.dts, sub) for s in src]
+    ref = O.nl_fwd_reg(g, med, spos, src, rpos, np.float64)
+    ref_dm = O.born_adj_reg(g, med, spos, fine, rpos, dat, np.float64)
+    srcd = [np.ascontiguousarray(s, dtype) for s in src]
+    datd = [np.ascontiguousarray(s, dtype) for s in dat]
+    grads = []
+    for limit in (0, 1):
+        if limit:
+            ctx.set_persistent(0, limit)
+        rec = [np.zeros((rpos[GRID_OF_COMP[k]].size, nts), dtype) for k in range(5)]
+        shot, keep = ctx.make_shot(mid, spos, rpos, srcd, rec)
+        h = ctx.fwi_forward([shot], segment if segment else nts - 1)
+        _check(rec, ref, dtype)
+        for _ in range(2):
+            shot, keep2 = ctx.make_shot(mid, spos, rpos, srcd, datd)
+            dm = np.zeros((5, nx, nz), dtype)
+            ctx.fwi_gradient(h, [shot], dm)
+            assert rel_l2(dm, ref_dm) < (2e-5 if dtype == np.float32 else 1e-10), rel_l2(dm, ref_dm)
+            grads.append(dm)
+        ctx.fwi_release(h)
+    assert np.array_equal(grads[0], grads[1])
+    ctx.close()
