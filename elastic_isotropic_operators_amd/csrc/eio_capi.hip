@@ -1438,7 +1438,7 @@ inline int res_tiles(const ModelBase& m, int R) {
 }
 
 // The passes that run resident and the widest tiles (columns per wave) their registers allow.
-enum class ResKind { NL, DEC };
+enum class ResKind { NL, DEC, ADJ };
 template <typename T>
 constexpr int res_max_r(ResKind k) {
     return sizeof(T) == 8 ? 2 : k == ResKind::NL ? 6 : 5;
@@ -1449,6 +1449,8 @@ constexpr int res_max_r(ResKind k) {
 template <typename T>
 double res_step_us(ResKind k, int R) {
     constexpr double nl[] = {3.4, 3.85, 5.05, 5.65, 7.0, 8.7}, dec[] = {3.5, 4.0, 5.2, 5.8, 8.2}, f64[] = {5.1, 6.15};
+    constexpr double adj[] = {3.35, 4.1, 5.35, 6.0, 8.4}, adj64[] = {5.15, 7.65};
+    if (k == ResKind::ADJ) return sizeof(T) == 8 ? adj64[R - 1] : adj[R - 1];
     return sizeof(T) == 8 ? f64[R - 1] : k == ResKind::NL ? nl[R - 1] : dec[R - 1];
 }
 
@@ -1549,29 +1551,26 @@ void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp) {
     fill0<int>(c, rp.abort_flag, 1);
 }
 
-// One launch of a group's fine steps [k0, k1).  `dsh` replaces the run's shot table.
-template <typename T, int MODE, bool FSURF = false>
-void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save,
-                    int dlo = 0, int dhi = -1, const eio::ShotDev<T>* dsh = nullptr) {
+// One cooperative launch of a group, over kernels k_res_*<T, R, ..> by the group's R (at most
+// RMAX): `pick(integral_constant R)` names the kernel, `extra` its arguments after the tile count.
+template <typename T, int RMAX, typename Pick, typename... A>
+void res_launch(Run<T>& run, const ResPlan& rp, const ResGroup& g, const eio::ShotDev<T>* sh, Pick&& kernel, A... extra) {
     Ctx* c = run.c;
-    constexpr int RMAX = res_max_r<T>((MODE & eio::F_DEC) ? ResKind::DEC : ResKind::NL);
     // packets of another group, call or segment may carry the levels of this one
     fill0<T>(c, static_cast<T*>(rp.inbox), long(rp.inbox_bytes / sizeof(T)));
     fill0<int>(c, rp.xcd, c->ncu);
-    const eio::ShotDev<T>* sh = dsh ? dsh : run.d_shots;
     const eio::ResTile* tt = rp.d_tiles + g.tile0;
     const eio::Entry* te = rp.d_ents;
     T* inbox = static_cast<T*>(rp.inbox);
     unsigned ib = unsigned(rp.inbox_bytes);
     int* ab = rp.abort_flag;
     int* xc = rp.xcd;
-    int nt = g.ntile, fr = from_rest, sv = save, sl = c->spin_limit;
-    void* args[] = {&sh, &tt, &te, &inbox, &ib, &ab, &xc, &nt, &k0, &k1, &fr, &sv, &dlo, &dhi, &sl};
+    int nt = g.ntile;
+    void* args[] = {&sh, &tt, &te, &inbox, &ib, &ab, &xc, &nt, &extra...};
     const void* fn = nullptr;
     auto pick = [&](auto r) {
-        constexpr int R = decltype(r)::value;
-        if constexpr (R <= RMAX)
-            if (g.R == R) fn = reinterpret_cast<const void*>(eio::k_res_fwd<T, R, MODE, FSURF>);
+        if constexpr (decltype(r)::value <= RMAX)
+            if (g.R == decltype(r)::value) fn = kernel(r);
     };
     pick(std::integral_constant<int, 1>{});
     pick(std::integral_constant<int, 2>{});
@@ -1580,6 +1579,25 @@ void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, i
     pick(std::integral_constant<int, 5>{});
     pick(std::integral_constant<int, 6>{});
     EIO_CHECK_HIP(hipLaunchCooperativeKernel(fn, dim3(nt), dim3(64 * RES_WX), args, 0, c->stream));
+}
+
+// Fine steps [k0, k1) of a group's forward loop.  `dsh` replaces the run's shot table.
+template <typename T, int MODE, bool FSURF = false>
+void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save,
+                    int dlo = 0, int dhi = -1, const eio::ShotDev<T>* dsh = nullptr) {
+    res_launch<T, res_max_r<T>((MODE & eio::F_DEC) ? ResKind::DEC : ResKind::NL)>(
+        run, rp, g, dsh ? dsh : run.d_shots,
+        [](auto r) { return reinterpret_cast<const void*>(eio::k_res_fwd<T, decltype(r)::value, MODE, FSURF>); }, k0, k1,
+        int(from_rest), int(save), dlo, dhi, run.c->spin_limit);
+}
+
+// Reverse fine steps [k0, k1) of a group's adjoint loop.
+template <typename T, int MODE>
+void res_launch_adj(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save) {
+    res_launch<T, res_max_r<T>(ResKind::ADJ)>(
+        run, rp, g, run.d_shots,
+        [](auto r) { return reinterpret_cast<const void*>(eio::k_res_adj<T, decltype(r)::value, MODE>); }, k0, k1,
+        int(from_rest), int(save), run.c->spin_limit);
 }
 
 // Whether the resident launches of this call gave up a wait (the call then repeats launched).
@@ -1601,16 +1619,19 @@ struct ResidentOff {
 // A context that leaves the launch form to the library, outside graphs, the persistent launch
 // and the no-allocation call.
 template <typename T>
-bool res_allowed(Ctx* c) {
+bool res_allowed(Ctx* c, ResKind kind) {
     if (!c->resident || c->use_graph || c->persistent || c->bump) return false;
-    return sizeof(T) == 8 ||
-           (c->time_block == 2 && c->variant2 == EIO_VARIANT_AUTO && c->group_bytes == EIO_GROUP_AUTO);
+    if (sizeof(T) == 8) return true;
+    if (kind == ResKind::ADJ) return c->adj_time_block == 2 && c->variant2a == EIO_VARIANT_AUTO;
+    return c->time_block == 2 && c->variant2 == EIO_VARIANT_AUTO && c->group_bytes == EIO_GROUP_AUTO;
 }
 
 // The groups of a pass of `per_launch` fine steps a launch (0: each group's own steps), or none
 // where the launched kernels are the faster form.  Launched, a step takes (FP32, two per launch) 2.6
 // us and its cells at 100 GCell/s, 4.2 us at least; (FP64, one per launch) its cells at 22 GCell/s, 6
-// us at least.  A resident launch takes its steps and a set-up: cleared inboxes, a cooperative launch
+// us at least; an adjoint step 3 us and its cells at 75 GCell/s, FP64 5 us and 38 GCell/s.  (Adjoint, us
+// a step, launched and resident: 280 x 472, 4.7 and 3.35; 600 x 1592, 15.2 and 5.9; two of 520 x
+// 1000, 17.2 and 5.9; FP64, two of 280 x 472, 12.0 and 7.65.)  A resident launch takes its steps and a set-up: cleared inboxes, a cooperative launch
 // and the state's first load, some 60 us, and 160 where the state comes from and goes back to memory
 // between segments.  Whole calls, resident against launched: 280 x 472, 396 against 373 us at 64 fine
 // steps, 622 against 635 at 128; 600 x 1592, 262 against 249 us at 10, 310 against 352 at 18; a
@@ -1618,7 +1639,7 @@ bool res_allowed(Ctx* c) {
 constexpr double RES_SETUP_US = 60.0, RES_SEGMENT_US = 160.0;
 template <typename T>
 std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
-    if (!res_allowed<T>(c)) return {};
+    if (!res_allowed<T>(c, kind)) return {};
     std::vector<ResGroup> groups = res_groups<T>(c, plan, shots, kind);
     double res = 0.0, work = 0.0;
     int longest = 0;
@@ -1629,8 +1650,9 @@ std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots
         for (int i = g.s0; i < g.s1; ++i)
             work += double(get_model(c, shots[plan.order[i]].model).n) * (per_launch ? per_launch : plan.nsteps[i]);
     }
-    const double launched = sizeof(T) == 4 ? std::max(4.2 * longest, 2.6 * longest + work / 100e3)
-                                           : std::max(6.0 * longest, work / 22e3);
+    const double launched =
+        sizeof(T) == 4 ? std::max(4.2 * longest, kind == ResKind::ADJ ? 3.0 * longest + work / 75e3 : 2.6 * longest + work / 100e3)
+                       : std::max(6.0 * longest, kind == ResKind::ADJ ? 5.0 * longest + work / 38e3 : work / 22e3);
     if (res >= launched) groups.clear();
     return groups;
 }
@@ -1923,6 +1945,26 @@ void set_abc(Ctx* c, int model, int on, const float* w, const float* scale) {
     m.abc_depth = depth;
 }
 
+// The NL adjoint with every shot resident; false when a shot does not fit or a wait was given up.
+template <typename T>
+bool nl_adjoint_resident(Ctx* c, int nshot, const eio_shot* shots, int flags) {
+    ResPlan rp;
+    rp.groups = res_choose<T>(c, make_plan<T>(c, nshot, shots, Op::NL_ADJ, PlanKind::NONE), shots, ResKind::ADJ);
+    if (rp.groups.empty()) return false;
+    Run<T> run = prepare<T>(c, nshot, shots, Op::NL_ADJ, flags, nullptr, nullptr, 0, false, false, false, false, false, 1);
+    res_build(run, shots, rp);
+    int kmax = run.plan.nsteps[0];
+    if (c->step_limit > 0) kmax = std::min(kmax, c->step_limit);
+    timing_begin<T>(c);
+    EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
+    for (const ResGroup& g : rp.groups) res_launch_adj<T, eio::M_NLADJ>(run, rp, g, 0, kmax, true, false);
+    EIO_CHECK_HIP(hipEventRecord(c->ev[3], c->stream));
+    timing_end<T>(c, kmax);
+    if (res_aborted(c, rp)) return false;
+    finish(run);
+    return true;
+}
+
 template <typename T>
 void nl_adjoint(Ctx* c, int nshot, const eio_shot* shots, int flags, int wshot = -1, void* wfld = nullptr) {
     if (nshot <= 0 || !shots) fail("no shots");
@@ -1930,7 +1972,10 @@ void nl_adjoint(Ctx* c, int nshot, const eio_shot* shots, int flags, int wshot =
     bool any_fs = false;
     for (int i = 0; i < nshot; ++i) any_fs = any_fs || get_model(c, shots[i].model).g.surface;
     int kmax0 = get_model(c, shots[0].model).ntw - 1;
+    bool same = true;  // all shots of a call share their step count (checked below)
+    for (int i = 1; i < nshot; ++i) same = same && get_model(c, shots[i].model).ntw == kmax0 + 1;
     if (c->step_limit > 0) kmax0 = std::min(kmax0, c->step_limit);
+    if (!wfld && !any_fs && same && nl_adjoint_resident<T>(c, nshot, shots, flags)) return;
     const bool two = sizeof(T) == 4 && c->adj_time_block == 2 && !wfld && !any_fs && kmax0 % 2 == 0;
     Run<T> run = prepare<T>(c, nshot, shots, Op::NL_ADJ, flags, nullptr, nullptr, 0, false, two);
     if (wfld) attach_wavefield(run, wshot, wfld, flags);

@@ -75,7 +75,8 @@ struct ShotDev {
     T* Wvx;                // Born coarse storage: wcap slices of nz*nx, coarse index its in slot its % wcap
     T* Wvz;
     int wcap;              // nts for full storage, segment length + 3 for the checkpointed gradient
-    int pad1;
+    int sscap;             // resident passes: coarse samples in the ring of secondary sources / adjoint
+                           // fields at ss[0] (else ss is the ping-pong of two)
     T* dm;                 // Born perturbation (forward) or per-shot imaging accumulator (adjoint)
     T* wfld;               // saved coarse-sampled wavefield [nts][5][nz*nx] of this shot, or NULL
 };

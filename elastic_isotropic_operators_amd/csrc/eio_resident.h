@@ -685,4 +685,476 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
     }
 }
 
+// Reverse fine steps [k0, k1) of the adjoint loop.  MODE M_NLADJ: the NL adjoint (source traces
+// extracted); M_BADJ: the Born receiver pass, whose adjoint fields of a coarse sample are summed in
+// registers and stored once, complete, into the ring of S.sscap samples at S.ss[0] (sample j at j %
+// sscap); a launch that ends above sample 0 leaves the open sample there for the next one.  k0 and,
+// for M_BADJ, k1 are multiples of the sub-sampling.  The stage holds the media-scaled level (as
+// k_step_adj), so the current level itself stays in registers with the older one.  Bound as the
+// forward loop is (a step of R = 4 with the media from L2 where registers end); two shots of 520 x
+// 1000, R = 4, 5.9 us a reverse step against 17.2 with two steps per launch, 280 x 472, R = 1, 3.35
+// against 4.7, and FP64, two of 280 x 472, R = 2, 7.65 against 12.0.
+template <typename T, int R, int MODE>
+__global__ __launch_bounds__(64 * RES_WX) __attribute__((amdgpu_waves_per_eu(RES_WX / 4, RES_WX / 4)))
+void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__ tiles,
+               const Entry* __restrict__ ents, T* inbox, unsigned inbox_bytes, int* abort_flag, int* xcd,
+               int ntiles, int k0, int k1, int from_rest, int save, int spin_limit) {
+    constexpr int WX = RES_WX;
+    constexpr int NT = 64 * WX;
+    constexpr int TX = WX * R;
+    constexpr int TXH = TX + 2 * FAT;
+    constexpr int FS = TXH * ZH;
+    constexpr unsigned SZ = sizeof(T);
+    constexpr bool BORN = MODE == M_BADJ;
+    constexpr bool MEML2 = sizeof(T) == 4 && R >= (BORN ? 4 : 5);
+    constexpr int RM = MEML2 ? 1 : R;
+    constexpr int RB = BORN ? R : 1;
+    constexpr bool PIN = sizeof(T) == 8 || R >= 3;
+    __shared__ __attribute__((aligned(16))) T L[5][TXH][ZH];
+    __shared__ int s_stop;
+
+    const int tile = xcd_remap(blockIdx.x, ntiles);
+    const ResTile& t = tiles[tile];
+    const ShotDev<T>& S = shots[t.shot];
+    const int nz = S.nz, nx = S.nx, sub = S.sub, h = S.h, nts = S.nts;
+    const unsigned n = unsigned(nz) * unsigned(nx);
+    const unsigned fbytes = n * SZ, colb = unsigned(nz) * SZ;
+    const int kend = min(k1, S.ntw - 1);
+    if (k0 >= kend) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int z0 = t.z0, x0 = t.x0;
+    const int iz = z0 + lane, zz = lane + FAT;
+    const int c0 = FAT + w * R, ix0 = x0 + w * R;
+    const unsigned voff = (unsigned(ix0) * unsigned(nz) + unsigned(iz)) * SZ;
+    const bool zok = iz < nz - FAT;
+    const int ncol = nx - FAT - ix0;
+    T cz[4], cx[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cz[i] = S.cz[i], cx[i] = S.cx[i];
+    const T* filt = S.filt;
+
+    if (tid == 0) s_stop = 0;
+    T o[5][R], c[5][R], m[5][RM], d[R];   // older and current level, media, sponge of the own cells
+    const rsrc_t rmed = make_rsrc(S.med, 5 * fbytes);
+#pragma unroll
+    for (int r = 0; r < R; ++r) d[r] = zok && r < ncol ? damp_at(S, iz, ix0 + r) : T(1);
+    {
+        const rsrc_t rold = make_rsrc(S.A, 5 * fbytes), rcur = make_rsrc(S.B, 5 * fbytes);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+                const unsigned so = unsigned(r) * colb + unsigned(f) * fbytes;
+                const bool ok = zok && r < ncol;
+                if (!MEML2) m[f][MEML2 ? 0 : r] = ok ? bld<T>(rmed, voff, so) : T(0);
+                o[f][r] = !from_rest && ok ? bld<T>(rold, voff, so) : T(0);
+                c[f][r] = !from_rest && ok ? bld<T>(rcur, voff, so) : T(0);
+            }
+        for (int e = tid; e < TXH * ZH; e += NT) {
+            const int cc = e / ZH, z = e - cc * ZH;
+            const int gx = x0 - FAT + cc, gz = z0 - FAT + z;
+            const bool in = !from_rest && gx < nx && gz < nz;
+            const unsigned vo = in ? (unsigned(gx) * unsigned(nz) + unsigned(gz)) * SZ : 0u;
+            T u[5], g[5];
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+                u[f] = in ? bld<T>(rcur, vo, unsigned(f) * fbytes) : T(0);
+                g[f] = in ? bld<T>(rmed, vo, unsigned(f) * fbytes) : T(0);
+            }
+            L[0][cc][z] = g[0] * u[0];
+            L[1][cc][z] = g[1] * u[1];
+            L[2][cc][z] = g[2] * u[2] + g[3] * u[3];
+            L[3][cc][z] = g[3] * u[2] + g[2] * u[3];
+            L[4][cc][z] = g[4] * u[4];
+        }
+    }
+    ResComm<T, R> cm;
+    cm.init(t, tile, w, lane, nz, nx, inbox, inbox_bytes, abort_flag, xcd, spin_limit);
+    const bool edge = (w * R < FAT && t.left >= 0) || (w * R + R > TX - FAT && t.right >= 0);
+    const unsigned lax = unsigned(reinterpret_cast<uintptr_t>((LdsT<T>*)&L[0][c0 - FAT][zz]));
+    const unsigned laz = unsigned(reinterpret_cast<uintptr_t>((LdsT<T>*)&L[0][c0][zz - FAT]));
+
+    // the wave's entries (data to inject, source cells to read), the first 64 of each in registers
+    const int rb0 = t.rec[w], re0 = t.rec[w + 1];
+    const int sb0 = BORN ? 0 : t.src[w], se0 = BORN ? 0 : t.src[w + 1];
+    const bool entries = rb0 < re0 || sb0 < se0;
+    int its = nts - 2 - k0 / sub, it2 = sub - 1;   // as adj_time; k0 is a multiple of sub
+    T* const Lf = &L[0][0][0];
+    auto sample = [&](int row, int j) -> T {
+        return j >= 0 ? S.rec_tr[row >> 24][long(row & 0xffffff) * nts + j] : T(0);
+    };
+    T ra = T(0), rb = T(0), rd = T(0);   // data samples its, its+1, sponge factor
+    int rcell = 0, rrow = -1;
+    if (rb0 + lane < re0) {
+        const Entry en = ents[rb0 + lane];
+        const int lz = en.lcell & 255, lx = en.lcell >> 8;
+        rcell = ((en.crow >> 24) * TXH + FAT + lx) * ZH + FAT + lz;
+        rd = damp_at(S, z0 + lz, x0 + lx);
+        rrow = en.crow;
+        ra = sample(rrow, its);
+        rb = sample(rrow, its + 1);
+    }
+    T sa = T(0), sb = T(0);              // source-trace sums of samples its, its+1
+    int scell = 0, srow = -1;
+    auto strace = [&](int row) -> T* { return S.src_tr[row >> 24] + long(row & 0xffffff) * nts; };
+    if (!BORN && sb0 + lane < se0) {
+        const Entry en = ents[sb0 + lane];
+        scell = ((en.crow >> 24) * TXH + FAT + (en.lcell >> 8)) * ZH + FAT + (en.lcell & 255);
+        srow = en.crow;
+        sb = strace(srow)[its + 1];
+    }
+    // adjoint fields of the own cells: coarse samples its+1 (ax) and its (ay)
+    T ax[5][RB], ay[5][RB];
+    auto slot = [&](int j) { return make_rsrc(S.ss[0] + size_t(j % S.sscap) * 5 * n, 5 * fbytes); };
+    auto store_slot = [&](int j) {
+        const rsrc_t rs = slot(j);
+        if (zok) {
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+                if (r < ncol) {
+#pragma unroll
+                    for (int f = 0; f < 5; ++f) bst(rs, ax[f][r], voff, unsigned(r) * colb + unsigned(f) * fbytes);
+                }
+        }
+    };
+    if constexpr (BORN) {
+        const rsrc_t rs = slot(its + 1);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+                ax[f][r] = !from_rest && zok && r < ncol ? bld<T>(rs, voff, unsigned(r) * colb + unsigned(f) * fbytes) : T(0);
+                ay[f][r] = T(0);
+            }
+    }
+    constexpr int XG = sizeof(T) == 4 ? 4 : 2;
+    auto dx = [&](int f, bool plus, T (&out)[R]) {
+        T q[R + 8];
+        const LdsT<T>* p = nullptr;
+#pragma unroll
+        for (int j = 0; j < R + 8; ++j) {
+            if (j % XG == 0) p = lds_at<T>(lax, f * FS + j * ZH);
+            q[j] = p[(j % XG) * ZH];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) out[r] = plus ? dp_q(q, r + 4, cx) : dm_q(q, r + 4, cx);
+#pragma unroll
+        for (int r = 0; r < R; ++r) asm volatile("" : "+v"(out[r]));
+        if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
+    };
+    T dxa[R], dx6[R], dx0[R], dx1[R];   // x derivatives of the stage's fields 2, 4, 0, 1
+    auto dx_all = [&]() {
+        dx(2, false, dxa);
+        dx(4, true, dx6);
+        dx(0, true, dx0);
+        dx(1, false, dx1);
+    };
+    T mnext[5];
+    auto load_media = [&](int r) {
+#pragma unroll
+        for (int f = 0; f < 5; ++f) mnext[f] = zok && r < ncol ? bld<T>(rmed, voff, unsigned(r) * colb + unsigned(f) * fbytes) : T(0);
+    };
+    __syncthreads();
+
+    constexpr unsigned PARITY = Inbox<TX>::PARITY * Packet<T>::BYTES;
+    for (int k = k0; k < kend; ++k) {
+        const unsigned pr = (unsigned(k) & 1u) * PARITY;
+        Quad<T> q[ResComm<T, R>::NQ];
+        if (k > k0) cm.send_x(Lf, k, pr);
+        if (!edge) dx_all();
+        if (k > k0) {
+            cm.request(q, pr);
+            if (!cm.receive(q, Lf, k, pr)) s_stop = 1;
+        }
+        __syncthreads();  // the halos are staged
+        if (s_stop) return;
+        if (edge) dx_all();
+        // the next level into o, which trades places with the current one
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const T d6 = dp_l(lds_at<T>(laz, 4 * FS + r * ZH), cz);
+            const T db = dm_l(lds_at<T>(laz, 3 * FS + r * ZH), cz);
+            const T d1 = dp_l(lds_at<T>(laz, FS + r * ZH), cz);
+            const T d0 = dm_l(lds_at<T>(laz, r * ZH), cz);
+            T v[5];
+            v[0] = d[r] * (d[r] * o[0][r] - (dxa[r] + d6));
+            v[1] = d[r] * (d[r] * o[1][r] - (db + dx6[r]));
+            v[2] = d[r] * (d[r] * o[2][r] - dx0[r]);
+            v[3] = d[r] * (d[r] * o[3][r] - d1);
+            v[4] = d[r] * (d[r] * o[4][r] - (d0 + dx1[r]));
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+                o[f][r] = c[f][r];
+                c[f][r] = v[f];
+            }
+            if constexpr (PIN) {
+#pragma unroll
+                for (int f = 0; f < 5; ++f) asm volatile("" : "+v"(c[f][r]), "+v"(o[f][r]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (MEML2) load_media(0);
+        __syncthreads();  // every read of level k is done
+        if (entries) {  // through the wave's own columns: data into the new level, source cells out of it
+            if (zok) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (r < ncol) {
+                        LdsT<T>* p = const_cast<LdsT<T>*>(lds_at<T>(laz, r * ZH + FAT));
+#pragma unroll
+                        for (int f = 0; f < 5; ++f) p[f * FS] = c[f][r];
+                    }
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (rb0 < re0) {
+                const T fa = filt[it2 + 1], fb = filt[h + it2 + 1];
+                if (rrow >= 0) {
+                    Lf[rcell] += rd * (ra * fa + rb * fb);
+                    if (it2 == 0) {
+                        rb = ra;
+                        ra = sample(rrow, its - 1);
+                    }
+                }
+                for (int e = rb0 + 64 + lane; e < re0; e += 64) {
+                    const Entry en = ents[e];
+                    const int lz = en.lcell & 255, lx = en.lcell >> 8;
+                    const T s = sample(en.crow, its) * fa + sample(en.crow, its + 1) * fb;
+                    L[en.crow >> 24][FAT + lx][FAT + lz] += damp_at(S, z0 + lz, x0 + lx) * s;
+                }
+                __builtin_amdgcn_wave_barrier();
+                if (zok) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (r < ncol) {
+                            const LdsT<T>* p = lds_at<T>(laz, r * ZH + FAT);
+#pragma unroll
+                            for (int f = 0; f < 5; ++f) c[f][r] = p[f * FS];
+                        }
+                }
+            }
+            if (!BORN && sb0 < se0) {
+                const T fa = filt[it2], fb = filt[h + it2];
+                if (srow >= 0) {
+                    const T v = Lf[scell];
+                    sa += v * fa;
+                    sb += v * fb;
+                    if (it2 == 0) {
+                        strace(srow)[its + 1] = sb;
+                        sb = sa;
+                        sa = T(0);
+                    }
+                }
+                for (int e = sb0 + 64 + lane; e < se0; e += 64) {
+                    const Entry en = ents[e];
+                    const T v = L[en.crow >> 24][FAT + (en.lcell >> 8)][FAT + (en.lcell & 255)];
+                    T* tr = strace(en.crow) + its;
+                    tr[0] += v * fa;
+                    tr[1] += v * fb;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        // the scaled next level is staged
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            T g[5];
+#pragma unroll
+            for (int f = 0; f < 5; ++f) g[f] = MEML2 ? mnext[f] : m[f][MEML2 ? 0 : r];
+            if (MEML2 && r + 1 < R) load_media(r + 1);
+            if (zok && r < ncol) {
+                LdsT<T>* p = const_cast<LdsT<T>*>(lds_at<T>(laz, r * ZH + FAT));
+                p[0] = g[0] * c[0][r];
+                p[FS] = g[1] * c[1][r];
+                p[2 * FS] = g[2] * c[2][r] + g[3] * c[3][r];
+                p[3 * FS] = g[3] * c[2][r] + g[2] * c[3][r];
+                p[4 * FS] = g[4] * c[4][r];
+            }
+            if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (k + 1 < kend) cm.send_z(Lf, k + 1, PARITY - pr);
+        if constexpr (BORN) {
+            const T ea = filt[it2], eb = filt[h + it2];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int f = 0; f < 5; ++f) {
+                    ay[f][r] += c[f][r] * ea;
+                    ax[f][r] += c[f][r] * eb;
+                }
+            if (it2 == 0) {
+                store_slot(its + 1);
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int f = 0; f < 5; ++f) {
+                        ax[f][r] = ay[f][r];
+                        ay[f][r] = T(0);
+                    }
+            }
+        }
+        if (--it2 < 0) {
+            it2 = sub - 1;
+            --its;
+        }
+        __syncthreads();  // the next level is staged
+    }
+    // the open sums and the state (its, it2: the step after the last one)
+    if (!BORN && srow >= 0) {
+        T* tr = strace(srow);
+        tr[its + 1] = sb;
+        if (it2 != sub - 1) tr[its] = sa;
+    }
+    if constexpr (BORN) store_slot(its + 1);
+    if (save) {
+        const rsrc_t rold = make_rsrc(S.A, 5 * fbytes), rcur = make_rsrc(S.B, 5 * fbytes);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (zok && r < ncol) {
+#pragma unroll
+                for (int f = 0; f < 5; ++f) {
+                    const unsigned so = unsigned(r) * colb + unsigned(f) * fbytes;
+                    bst(rold, o[f][r], voff, so);
+                    bst(rcur, c[f][r], voff, so);
+                }
+            }
+    }
+}
+
+// ------------------------------------------------------------------ imaging over many coarse samples
+// k_imaging for coarse samples j0, j0 - 1, .., j1 (ADJ: the imaging condition with the ring's adjoint
+// fields) or j0, j0 + 1, .., j1 (forward: the secondary sources into the ring), sample j at j % sscap
+// of S.ss[0].  The perturbation or the accumulators stay in registers over the samples, and the
+// slices next to a sample are in L2 from its neighbours' turn: 31 B a cell and sample instead of 104 (ADJ).
+template <typename T, int R, int WX, bool ADJ>
+__global__ __launch_bounds__(64 * WX) void k_imaging_many(const ShotDev<T>* __restrict__ shots,
+                                                          const TileDev* __restrict__ tiles, int ntiles, int j0, int j1) {
+    constexpr int NT = 64 * WX;
+    constexpr int TX = WX * R;
+    constexpr int TXH = TX + 2 * FAT;
+    constexpr unsigned SZ = sizeof(T);
+    constexpr int NFILL = (TXH * ZH + NT - 1) / NT;
+    __shared__ T lds[2][TXH][ZH];
+
+    const TileDev t = tiles[xcd_remap(blockIdx.x, ntiles)];
+    const ShotDev<T>& S = shots[t.shot];
+    const int nz = S.nz, nx = S.nx, nts = S.nts, wcap = S.wcap;
+    const unsigned n = unsigned(nz) * unsigned(nx);
+    const unsigned fbytes = n * SZ, colb = unsigned(nz) * SZ;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int iz = t.z0 + lane, zz = lane + FAT;
+    const int c0 = FAT + w * R, ix0 = t.x0 + w * R;
+    const unsigned voff = (unsigned(ix0) * unsigned(nz) + unsigned(iz)) * SZ;
+    const bool zok = iz < nz - FAT;
+    T cz[4], cx[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cz[i] = S.cz[i], cx[i] = S.cx[i];
+    const T dinv = S.filt[2 * S.h];  // 1/(2 dts)
+    const unsigned hbase = (unsigned(t.x0 - FAT) * unsigned(nz) + unsigned(t.z0 - FAT)) * SZ;
+    // halo fill: cells outside the update region are zero, as in k_imaging
+    unsigned hv[NFILL];
+#pragma unroll
+    for (int it = 0; it < NFILL; ++it) {
+        const int e = threadIdx.x + it * NT;
+        const int c = e / ZH, z = e - c * ZH;
+        const int hz = t.z0 - FAT + z, hx = t.x0 - FAT + c;
+        const bool upd = e < TXH * ZH && hz >= FAT && hz < nz - FAT && hx >= FAT && hx < nx - FAT;
+        hv[it] = upd ? hbase + unsigned(c) * colb + unsigned(z) * SZ : 0xfffffff0u;  // past the end: reads 0
+    }
+    auto slice = [&](const T* W, int j) { return make_rsrc(W + size_t(j % wcap) * n, fbytes); };
+    const rsrc_t rdm = make_rsrc(S.dm, 5 * fbytes);
+    T dm[5][R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int f = 0; f < 5; ++f)
+            dm[f][r] = zok && ix0 + r < nx - FAT ? bld<T>(rdm, voff, unsigned(r) * colb + unsigned(f) * fbytes) : T(0);
+
+    const int step = ADJ ? -1 : 1;
+    T fx[NFILL], fz[NFILL];   // the next sample's slice, in flight while this one is used
+    auto prefetch = [&](int j) {
+        const rsrc_t rwx = slice(S.Wvx, j), rwz = slice(S.Wvz, j);
+#pragma unroll
+        for (int it = 0; it < NFILL; ++it) {
+            fx[it] = bld<T>(rwx, hv[it], 0u);
+            fz[it] = bld<T>(rwz, hv[it], 0u);
+        }
+    };
+    prefetch(j0);
+    for (int j = j0;; j += step) {
+        __syncthreads();
+#pragma unroll
+        for (int it = 0; it < NFILL; ++it) {
+            const int e = threadIdx.x + it * NT;
+            if (e < TXH * ZH) {
+                (&lds[0][0][0])[e] = fx[it];
+                (&lds[1][0][0])[e] = fz[it];
+            }
+        }
+        __syncthreads();
+        const bool more = j != j1;
+        const rsrc_t rxm = slice(S.Wvx, j > 0 ? j - 1 : j), rzm = slice(S.Wvz, j > 0 ? j - 1 : j);
+        const rsrc_t rxp = slice(S.Wvx, j < nts - 1 ? j + 1 : j), rzp = slice(S.Wvz, j < nts - 1 ? j + 1 : j);
+        const rsrc_t rss = make_rsrc(S.ss[0] + size_t(j % S.sscap) * 5 * n, 5 * fbytes);
+        T wxm[R], wzm[R], wxp[R], wzp[R], a[5][R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const unsigned so = unsigned(r) * colb;
+            const bool ok = zok && ix0 + r < nx - FAT;
+            wxm[r] = ok && j > 0 ? bld<T>(rxm, voff, so) : T(0);
+            wzm[r] = ok && j > 0 ? bld<T>(rzm, voff, so) : T(0);
+            wxp[r] = ok && j < nts - 1 ? bld<T>(rxp, voff, so) : T(0);
+            wzp[r] = ok && j < nts - 1 ? bld<T>(rzp, voff, so) : T(0);
+            if (ADJ) {
+#pragma unroll
+                for (int f = 0; f < 5; ++f) a[f][r] = ok ? bld<T>(rss, voff, so + unsigned(f) * fbytes) : T(0);
+            }
+        }
+        if (more) prefetch(j + step);
+        T xx[R], zxm[R];
+        {
+            T q[R + 8];
+#pragma unroll
+            for (int i = 0; i < R + 8; ++i) q[i] = lds[0][c0 - 4 + i][zz];
+#pragma unroll
+            for (int r = 0; r < R; ++r) xx[r] = dp_q(q, r + 4, cx);
+#pragma unroll
+            for (int i = 0; i < R + 8; ++i) q[i] = lds[1][c0 - 4 + i][zz];
+#pragma unroll
+            for (int r = 0; r < R; ++r) zxm[r] = dm_q(q, r + 4, cx);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const T zv = dp_q(&lds[1][c0 + r][zz], 0, cz);
+            const T xz = dm_q(&lds[0][c0 + r][zz], 0, cz) + zxm[r];
+            const T tx = j == 0 ? -wxp[r] : j == nts - 1 ? wxm[r] : wxm[r] - wxp[r];
+            const T tz = j == 0 ? -wzp[r] : j == nts - 1 ? wzm[r] : wzm[r] - wzp[r];
+            if (ADJ) {
+                dm[0][r] = dm[0][r] + a[0][r] * tx * dinv;
+                dm[1][r] = dm[1][r] + a[1][r] * tz * dinv;
+                dm[2][r] = dm[2][r] + (a[2][r] + a[3][r]) * (xx[r] + zv);
+                dm[3][r] = dm[3][r] + T(2) * (xx[r] * a[2][r] + zv * a[3][r]);
+                dm[4][r] = dm[4][r] + a[4][r] * xz;
+            } else if (zok && ix0 + r < nx - FAT) {
+                const unsigned so = unsigned(r) * colb;
+                const T dl = dm[2][r] * (xx[r] + zv);
+                bst(rss, dm[0][r] * tx * dinv, voff, so);
+                bst(rss, dm[1][r] * tz * dinv, voff, so + fbytes);
+                bst(rss, dl + T(2) * dm[3][r] * xx[r], voff, so + 2 * fbytes);
+                bst(rss, dl + T(2) * dm[3][r] * zv, voff, so + 3 * fbytes);
+                bst(rss, dm[4][r] * xz, voff, so + 4 * fbytes);
+            }
+        }
+        if (!more) break;
+    }
+    if (ADJ) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (zok && ix0 + r < nx - FAT) {
+#pragma unroll
+                for (int f = 0; f < 5; ++f) bst(rdm, dm[f][r], voff, unsigned(r) * colb + unsigned(f) * fbytes);
+            }
+    }
+}
+
 }  // namespace eio

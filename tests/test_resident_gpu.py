@@ -176,3 +176,71 @@ def test_fwi_record_and_checkpoints(dtype, nz, nx, segment):
         ctx.fwi_release(h)
     assert np.array_equal(grads[0], grads[1])
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype,nz,nx,nts,sub,nsrc,nrec", [
+    (np.float32, 72, 24, 51, 2, 10, 20),       # one full tile of R = 1
+    (np.float32, 73, 25, 50, 3, 10, 20),       # one row and one column over, an odd sub-sampling
+    (np.float32, 76, 28, 90, 1, 10, 20),
+    (np.float32, 40, 90, 51, 2, 700, 700),     # more entries than a wave keeps in registers
+    (np.float32, 281, 967, 51, 2, 40, 60),     # R = 2
+    (np.float32, 563, 1103, 51, 2, 40, 60),    # R = 3
+    (np.float32, 601, 1593, 51, 2, 40, 60),    # R = 4
+    (np.float32, 683, 1503, 51, 2, 40, 60),    # R = 5
+    (np.float64, 73, 25, 50, 3, 10, 20),
+    (np.float64, 40, 90, 51, 2, 700, 700),
+    (np.float64, 281, 967, 51, 2, 40, 60),     # R = 2
+])
+def test_adjoint_tiles(dtype, nz, nx, nts, sub, nsrc, nrec):
+    """The NL adjoint, then again with its waits given up (launched kernels): both against the oracle, and
+    the resident one again into buffers of the call before."""
+    ctx = _ctx(dtype)
+    mid, g, med = _model(ctx, nz, nx, nts, sub, nz + nx)
+    rng = np.random.default_rng(nz * nx + 1)
+    spos, rpos = _positions(rng, g, nsrc), _positions(rng, g, nrec)
+    dat = random_traces(rng, rpos, nts, np.float64)
+    ref = O.nl_adj_reg(g, med, spos, rpos, dat, np.float64)
+    datd = [np.ascontiguousarray(s, dtype) for s in dat]
+    out = []
+    for limit in (0, 0, 1):
+        if limit:
+            ctx.set_persistent(0, limit)
+        src = [np.full((spos[GRID_OF_COMP[k]].size, nts), 7, dtype) for k in range(5)]
+        shot, keep = ctx.make_shot(mid, spos, rpos, src, datd)
+        ctx.nl_adjoint([shot])
+        _check(src, ref, dtype)
+        out.append(src)
+    for k in range(5):
+        assert np.array_equal(out[0][k], out[1][k]), k
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_adjoint_batch(dtype):
+    """Shots of several grids (one step count) in one launch, and a step limit that ends inside a coarse
+    sample: the same as the launched kernels."""
+    ctx = _ctx(dtype)
+    rng = np.random.default_rng(15)
+    shots, outs, refs, keeps = [], [], [], []
+    for i, (nz, nx) in enumerate([(90, 130), (150, 90), (61, 200)]):
+        mid, g, med = _model(ctx, nz, nx, 50, 4, 70 + i)
+        spos, rpos = _positions(rng, g, 8), _positions(rng, g, 20)
+        dat = random_traces(rng, rpos, g.nts, np.float64)
+        refs.append(O.nl_adj_reg(g, med, spos, rpos, dat, np.float64))
+        src = [np.zeros((spos[GRID_OF_COMP[k]].size, g.nts), dtype) for k in range(5)]
+        shot, keep = ctx.make_shot(mid, spos, rpos, src, [np.ascontiguousarray(s, dtype) for s in dat])
+        shots.append(shot)
+        outs.append(src)
+        keeps.append(keep)
+    ctx.nl_adjoint(shots)
+    for src, ref in zip(outs, refs):
+        _check(src, ref, dtype)
+    ctx.set_step_limit(186)
+    ctx.nl_adjoint(shots)
+    part = [[s.copy() for s in src] for src in outs]
+    ctx.set_persistent(0, 1)
+    ctx.nl_adjoint(shots)
+    for src, p in zip(outs, part):
+        for k in range(5):
+            assert np.any(p[k]) and rel_l2(p[k], src[k]) < TOL[dtype], k
+    ctx.close()
