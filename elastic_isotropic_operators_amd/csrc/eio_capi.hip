@@ -1438,10 +1438,10 @@ inline int res_tiles(const ModelBase& m, int R) {
 }
 
 // The passes that run resident and the widest tiles (columns per wave) their registers allow.
-enum class ResKind { NL, DEC, ADJ };
+enum class ResKind { NL, DEC, ADJ, BADJ };
 template <typename T>
 constexpr int res_max_r(ResKind k) {
-    return sizeof(T) == 8 ? 2 : k == ResKind::NL ? 6 : 5;
+    return sizeof(T) == 8 ? 2 : k == ResKind::NL ? 6 : k == ResKind::BADJ ? 4 : 5;
 }
 // Measured time of one fine step of a launch with R columns per wave [us] (every CU busy; the
 // halo exchange and the barriers are about 2.5 us of it, so wide tiles do the most work per
@@ -1450,48 +1450,57 @@ template <typename T>
 double res_step_us(ResKind k, int R) {
     constexpr double nl[] = {3.4, 3.85, 5.05, 5.65, 7.0, 8.7}, dec[] = {3.5, 4.0, 5.2, 5.8, 8.2}, f64[] = {5.1, 6.15};
     constexpr double adj[] = {3.35, 4.1, 5.35, 6.0, 8.4}, adj64[] = {5.15, 7.65};
+    constexpr double badj[] = {3.6, 4.5, 6.0, 7.2}, badj64[] = {5.5, 9.0};
     if (k == ResKind::ADJ) return sizeof(T) == 8 ? adj64[R - 1] : adj[R - 1];
+    if (k == ResKind::BADJ) return sizeof(T) == 8 ? badj64[R - 1] : badj[R - 1];
     return sizeof(T) == 8 ? f64[R - 1] : k == ResKind::NL ? nl[R - 1] : dec[R - 1];
 }
 
-// The groups of a call, or none when a shot does not fit the device.
+// The groups of a call that take the least time in all, or none when a shot does not fit the device.
+// A group of a given R holds as many shots as fit (steps decrease along the plan, so fewer would
+// leave the later groups no less); over R and over the groups' ends the best split is exact: eight shots
+// of 280 x 472 take one launch of R = 5 (8.4 us an adjoint step), not six shots of R = 4 and two of
+// R = 2 (6.0 + 4.1), which do the most work per time first.
+constexpr double RES_SETUP_US = 60.0;   // of one launch, see res_choose
 template <typename T>
 std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) {
-    const int n = int(plan.order.size());
-    std::vector<ResGroup> out;
-    int tile0 = 0;
-    for (int s0 = 0; s0 < n;) {
-        ResGroup best{s0, s0, 0, tile0, 0};
-        double cost = 0.0;
-        for (int R = 1; R <= res_max_r<T>(kind); ++R) {
+    const int n = int(plan.order.size()), RM = res_max_r<T>(kind);
+    std::vector<ResGroup> best(n);
+    std::vector<double> cost(n + 1, 0.0);
+    for (int s0 = n - 1; s0 >= 0; --s0) {
+        best[s0] = ResGroup{s0, s0, 0, 0, 0};
+        cost[s0] = 1e30;
+        for (int R = 1; R <= RM; ++R) {
             int nt = 0, s1 = s0;
-            double work = 0.0;
             while (s1 < n) {
-                const ModelBase& m = get_model(c, shots[plan.order[s1]].model);
-                const int k = res_tiles(m, R);
+                const int k = res_tiles(get_model(c, shots[plan.order[s1]].model), R);
                 if (nt + k > c->ncu) break;
                 nt += k;
-                work += double(m.n) * plan.nsteps[s1];
                 ++s1;
             }
             if (s1 == s0) continue;
-            const double t = res_step_us<T>(kind, R) * plan.nsteps[s0] / work;  // time per cell-update
-            if (!best.R || t < cost) {
-                best = {s0, s1, R, tile0, nt};
-                cost = t;
+            const double t = RES_SETUP_US + res_step_us<T>(kind, R) * plan.nsteps[s0] + cost[s1];
+            if (t < cost[s0]) {
+                best[s0] = {s0, s1, R, 0, nt};
+                cost[s0] = t;
             }
         }
-        if (!best.R) return {};
-        out.push_back(best);
-        tile0 += best.ntile;
-        s0 = best.s1;
+        if (!best[s0].R) return {};
+    }
+    std::vector<ResGroup> out;
+    int tile0 = 0;
+    for (int s0 = 0; s0 < n; s0 = best[s0].s1) {
+        best[s0].tile0 = tile0;
+        tile0 += best[s0].ntile;
+        out.push_back(best[s0]);
     }
     return out;
 }
 
-// Tiles and entries of the groups, their device tables and the exchange buffers.
+// Tiles and entries of the groups, their device tables and the exchange buffers.  `tag` keeps the
+// buffers of two plans of one call apart.
 template <typename T>
-void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp) {
+void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp, const std::string& tag = "res_") {
     Ctx* c = run.c;
     int maxR = 1;
     for (const ResGroup& g : rp.groups) {
@@ -1536,8 +1545,8 @@ void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp) {
         }
     }
     const hipMemcpyKind h2d = hipMemcpyHostToDevice;
-    rp.d_tiles = static_cast<eio::ResTile*>(ws_get(c, "res_tiles", sizeof(eio::ResTile) * rp.tiles.size()));
-    rp.d_ents = static_cast<eio::Entry*>(ws_get(c, "res_ents", sizeof(eio::Entry) * std::max<size_t>(1, rp.ents.size())));
+    rp.d_tiles = static_cast<eio::ResTile*>(ws_get(c, tag + "tiles", sizeof(eio::ResTile) * rp.tiles.size()));
+    rp.d_ents = static_cast<eio::Entry*>(ws_get(c, tag + "ents", sizeof(eio::Entry) * std::max<size_t>(1, rp.ents.size())));
     EIO_CHECK_HIP(hipMemcpyAsync(rp.d_tiles, rp.tiles.data(), sizeof(eio::ResTile) * rp.tiles.size(), h2d, c->stream));
     if (!rp.ents.empty())
         EIO_CHECK_HIP(hipMemcpyAsync(rp.d_ents, rp.ents.data(), sizeof(eio::Entry) * rp.ents.size(), h2d, c->stream));
@@ -1545,9 +1554,9 @@ void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp) {
     int ntile = 0;
     for (const ResGroup& g : rp.groups) ntile = std::max(ntile, g.ntile);
     rp.inbox_bytes = size_t(ntile) * per_tile * eio::Packet<T>::BYTES;
-    rp.inbox = ws_get(c, "res_inbox", rp.inbox_bytes);
-    rp.abort_flag = static_cast<int*>(ws_get(c, "res_abort", 256));
-    rp.xcd = static_cast<int*>(ws_get(c, "res_xcd", size_t(c->ncu) * sizeof(int)));
+    rp.inbox = ws_get(c, tag + "inbox", rp.inbox_bytes);
+    rp.abort_flag = static_cast<int*>(ws_get(c, tag + "abort", 256));
+    rp.xcd = static_cast<int*>(ws_get(c, tag + "xcd", size_t(c->ncu) * sizeof(int)));
     fill0<int>(c, rp.abort_flag, 1);
 }
 
@@ -1593,9 +1602,10 @@ void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, i
 
 // Reverse fine steps [k0, k1) of a group's adjoint loop.
 template <typename T, int MODE>
-void res_launch_adj(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save) {
-    res_launch<T, res_max_r<T>(ResKind::ADJ)>(
-        run, rp, g, run.d_shots,
+void res_launch_adj(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save,
+                    const eio::ShotDev<T>* dsh = nullptr) {
+    res_launch<T, res_max_r<T>(MODE == eio::M_BADJ ? ResKind::BADJ : ResKind::ADJ)>(
+        run, rp, g, dsh ? dsh : run.d_shots,
         [](auto r) { return reinterpret_cast<const void*>(eio::k_res_adj<T, decltype(r)::value, MODE>); }, k0, k1,
         int(from_rest), int(save), run.c->spin_limit);
 }
@@ -1622,7 +1632,7 @@ template <typename T>
 bool res_allowed(Ctx* c, ResKind kind) {
     if (!c->resident || c->use_graph || c->persistent || c->bump) return false;
     if (sizeof(T) == 8) return true;
-    if (kind == ResKind::ADJ) return c->adj_time_block == 2 && c->variant2a == EIO_VARIANT_AUTO;
+    if (kind == ResKind::ADJ || kind == ResKind::BADJ) return c->adj_time_block == 2 && c->variant2a == EIO_VARIANT_AUTO;
     return c->time_block == 2 && c->variant2 == EIO_VARIANT_AUTO && c->group_bytes == EIO_GROUP_AUTO;
 }
 
@@ -1636,7 +1646,7 @@ bool res_allowed(Ctx* c, ResKind kind) {
 // between segments.  Whole calls, resident against launched: 280 x 472, 396 against 373 us at 64 fine
 // steps, 622 against 635 at 128; 600 x 1592, 262 against 249 us at 10, 310 against 352 at 18; a
 // checkpointed gradient of four shots of 280 x 472 in segments of 46 steps, 43.7 against 37.4 ms.
-constexpr double RES_SETUP_US = 60.0, RES_SEGMENT_US = 160.0;
+constexpr double RES_SEGMENT_US = 160.0;
 template <typename T>
 std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
     if (!res_allowed<T>(c, kind)) return {};
@@ -1650,9 +1660,10 @@ std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots
         for (int i = g.s0; i < g.s1; ++i)
             work += double(get_model(c, shots[plan.order[i]].model).n) * (per_launch ? per_launch : plan.nsteps[i]);
     }
+    const bool adj = kind == ResKind::ADJ || kind == ResKind::BADJ;
     const double launched =
-        sizeof(T) == 4 ? std::max(4.2 * longest, kind == ResKind::ADJ ? 3.0 * longest + work / 75e3 : 2.6 * longest + work / 100e3)
-                       : std::max(6.0 * longest, kind == ResKind::ADJ ? 5.0 * longest + work / 38e3 : work / 22e3);
+        sizeof(T) == 4 ? std::max(4.2 * longest, adj ? 3.0 * longest + work / 75e3 : 2.6 * longest + work / 100e3)
+                       : std::max(6.0 * longest, adj ? 5.0 * longest + work / 38e3 : work / 22e3);
     if (res >= launched) groups.clear();
     return groups;
 }
@@ -2049,6 +2060,98 @@ bool born_source_resident(Run<T>& run, int nshot, const eio_shot* shots) {
     return !res_aborted(c, rp);
 }
 
+// Coarse samples of one launch of a resident pass that trades them with k_imaging_many through a ring,
+// that kernel's tiles, and the shot table with the ring.
+constexpr int RES_RING = 32;
+template <typename T>
+struct ResRing {
+    static constexpr int R = 2, WX = sizeof(T) == 8 ? 4 : 8, TX = R * WX;
+    int K = 0;
+    std::vector<eio::TileDev> tiles;
+    std::vector<int> tile0;                       // first tile of each shot, and the end
+    eio::TileDev* d_tiles = nullptr;
+    std::vector<eio::ShotDev<T>> sd;
+    eio::ShotDev<T>* d_shots = nullptr;
+};
+
+// The ring of a plan's groups (one after the other in the same memory); false: no memory for it.
+template <typename T>
+bool ring_build(Run<T>& run, const ResPlan& rp, ResRing<T>& ring) {
+    Ctx* c = run.c;
+    const int nshot = int(run.sd.size()), nz = run.sd[0].nz, nx = run.sd[0].nx;
+    const size_t n5 = 5 * size_t(nz) * nx;
+    ring.K = std::min(RES_RING, run.sd[0].nts - 1);
+    int most = 0;
+    for (const ResGroup& g : rp.groups) most = std::max(most, g.s1 - g.s0);
+    // a ring is extra memory: only where it leaves plenty of what is free to the rest of the call
+    const size_t bytes = size_t(most) * (ring.K + 1) * n5 * sizeof(T);
+    size_t avail = 0, total = 0;
+    if (c->ws["res_ring"].bytes < bytes && (hipMemGetInfo(&avail, &total) != hipSuccess || bytes > avail / 4)) return false;
+    T* buf = static_cast<T*>(ws_get(c, "res_ring", bytes));
+    ring.sd = run.sd;
+    for (const ResGroup& g : rp.groups)
+        for (int oi = g.s0; oi < g.s1; ++oi) {
+            ring.sd[oi].ss[0] = buf + size_t(oi - g.s0) * (ring.K + 1) * n5;
+            ring.sd[oi].sscap = ring.K + 1;
+        }
+    for (int oi = 0; oi < nshot; ++oi) {
+        ring.tile0.push_back(int(ring.tiles.size()));
+        for (int x0 = eio::FAT; x0 < nx - eio::FAT; x0 += ring.TX)
+            for (int z0 = eio::FAT; z0 < nz - eio::FAT; z0 += eio::TZ) {
+                eio::TileDev t{};
+                t.shot = oi;
+                t.z0 = z0;
+                t.x0 = x0;
+                ring.tiles.push_back(t);
+            }
+    }
+    ring.tile0.push_back(int(ring.tiles.size()));
+    ring.d_tiles = static_cast<eio::TileDev*>(ws_get(c, "ring_tiles", sizeof(eio::TileDev) * ring.tiles.size()));
+    ring.d_shots = static_cast<eio::ShotDev<T>*>(ws_get(c, "ring_shots", sizeof(eio::ShotDev<T>) * nshot));
+    const hipMemcpyKind h2d = hipMemcpyHostToDevice;
+    EIO_CHECK_HIP(hipMemcpyAsync(ring.d_tiles, ring.tiles.data(), sizeof(eio::TileDev) * ring.tiles.size(), h2d, c->stream));
+    EIO_CHECK_HIP(hipMemcpyAsync(ring.d_shots, ring.sd.data(), sizeof(eio::ShotDev<T>) * nshot, h2d, c->stream));
+    return true;
+}
+
+// Imaging of the coarse samples j0 .. j1 of a group's shots, against the ring.
+template <typename T, bool ADJ>
+void launch_ring(Run<T>& run, const ResRing<T>& ring, const ResGroup& g, int j0, int j1) {
+    const int t0 = ring.tile0[g.s0], nt = ring.tile0[g.s1] - t0;
+    klaunch(run.c, eio::k_imaging_many<T, ResRing<T>::R, ResRing<T>::WX, ADJ>, dim3(nt), dim3(64 * ResRing<T>::WX),
+            ring.d_shots, ring.d_tiles + t0, nt, j0, j1);
+}
+
+// The Born receiver pass of a group: RES_RING coarse intervals a launch, then their imaging.
+// `before(j, flush)` runs before sample j is imaged; where it launches work, it calls flush first (the
+// imaging of the samples above j).
+template <typename T, typename F>
+void receiver_pass_resident(Run<T>& run, const ResPlan& rp, const ResRing<T>& ring, const ResGroup& g, F&& before) {
+    const int nts = run.sd[0].nts, sub = run.sd[0].sub;
+    for (int b = nts - 2; b >= 0; b -= ring.K) {   // intervals b .. a complete the samples b+1 .. a+1
+        const int a = std::max(0, b - ring.K + 1);
+        res_launch_adj<T, eio::M_BADJ>(run, rp, g, (nts - 2 - b) * sub, (nts - 1 - a) * sub, b == nts - 2, a > 0, ring.d_shots);
+        const int last = a > 0 ? a + 1 : 0;
+        int j0 = b + 1;
+        for (int j = b + 1; j >= last; --j)
+            before(j, [&]() {
+                if (j0 > j) launch_ring<T, true>(run, ring, g, j0, j + 1);
+                j0 = j;
+            });
+        launch_ring<T, true>(run, ring, g, j0, last);
+    }
+}
+
+// The groups (one_group: at most one), tables and ring of a resident receiver pass; false: the launched one.
+template <typename T>
+bool receiver_pass_build(Run<T>& run, int nshot, const eio_shot* shots, ResPlan& rp, ResRing<T>& ring, bool one_group) {
+    Ctx* c = run.c;
+    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::BADJ, std::min(RES_RING, run.sd[0].nts - 1) * run.sd[0].sub);
+    if (rp.groups.empty() || (one_group && rp.groups.size() > 1) || !ring_build(run, rp, ring)) return false;
+    res_build(run, shots, rp, "resa_");
+    return true;
+}
+
 template <typename T>
 void born_forward(Ctx* c, int nshot, const eio_shot* shots, const void* const dm[5], int flags) {
     if (!dm) fail("dm is NULL");
@@ -2112,6 +2215,13 @@ void born_adjoint(Ctx* c, int nshot, const eio_shot* shots, void* const dm[5], i
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
     run_loop(c, [&]() {
         if (!born_source_resident(run, nshot, shots)) born_source_pass(run, ntile, kmax);
+        ResPlan rp;
+        ResRing<T> ring;
+        if (receiver_pass_build(run, nshot, shots, rp, ring, false)) {
+            for (const ResGroup& g : rp.groups) receiver_pass_resident(run, rp, ring, g, [](int, auto&&) {});
+            if (!res_aborted(c, rp)) return;
+            for (int oi = 0; oi < nshot; ++oi) fill0<T>(c, run.sd[oi].dm, 5 * m.n);
+        }
         for (int oi = 0; oi < nshot; ++oi) {
             fill0<T>(c, run.sd[oi].A, 5 * m.n);
             fill0<T>(c, run.sd[oi].B, 5 * m.n);
@@ -2426,6 +2536,11 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
         else copy_dev<T>(c, fstate, static_cast<const T*>(f.ck) + size_t(j - 1) * f.state_elems, f.state_elems);
         for (int k = k0; k < k1; ++k) launch_fwd<T, eio::M_RECOMP>(run, ntile, k, 0, seg_begin(f, j), dhi, d_sdf);
     };
+    // the receiver pass resident, group by group; with several groups only where no segment is
+    // recomputed in between (a recompute serves every shot)
+    ResPlan rpa;
+    ResRing<T> ring;
+    const bool ares = receiver_pass_build(run, nshot, shots, rpa, ring, f.nseg > 1);
     const bool fresh = f.ring_fresh;
     f.ring_fresh = false;
     if (!fresh) nrecomp += (long long)(seg_end(f, f.nseg - 1) - seg_begin(f, f.nseg - 1)) * sub;
@@ -2433,6 +2548,17 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
         if (rtwo) fill0<T>(c, fstate, long(fstate_elems));
         // a store used before no longer holds the last segment in its ring
         if (!fresh) recompute(f.nseg - 1);
+        if (ares) {
+            int jn = f.nseg - 1;
+            for (const ResGroup& g : rpa.groups)
+                receiver_pass_resident(run, rpa, ring, g, [&](int j, auto&& flush) {
+                    if (jn >= 1 && j == seg_begin(f, jn) + 1) {
+                        flush();
+                        recompute(--jn);
+                    }
+                });
+            return;
+        }
         int p = 0;
         int jn = f.nseg - 1;  // next segment start to cross going backwards
         for (int its = nts - 2; its >= 0; --its) {
@@ -2449,7 +2575,7 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
     });
     EIO_CHECK_HIP(hipEventRecord(c->ev[3], c->stream));
     timing_end<T>(c, (long long)(nts - 1) * sub + nrecomp);
-    if (rres && res_aborted(c, rp)) {  // a wait was given up: the whole sweep again, launched
+    if ((rres && res_aborted(c, rp)) || (ares && res_aborted(c, rpa))) {  // a wait was given up: the whole sweep again, launched
         ResidentOff off(c);
         fwi_gradient<T>(c, handle, nshot, shots, dm, flags);
         return;

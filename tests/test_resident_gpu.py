@@ -244,3 +244,41 @@ def test_adjoint_batch(dtype):
         for k in range(5):
             assert np.any(p[k]) and rel_l2(p[k], src[k]) < TOL[dtype], k
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype,nz,nx,nts,sub", [
+    (np.float32, 73, 25, 70, 3),      # R = 1, one row and one column over, three launches of 32 coarse intervals
+    (np.float32, 76, 28, 34, 4),      # one interval over a launch
+    (np.float32, 139, 90, 33, 4),     # exactly one launch
+    (np.float32, 281, 967, 40, 2),    # R = 2
+    (np.float32, 563, 1103, 40, 2),   # R = 3
+    (np.float32, 601, 1593, 40, 2),   # R = 4
+    (np.float64, 73, 25, 70, 3),
+    (np.float64, 281, 967, 40, 2),    # R = 2
+])
+def test_born_adjoint_tiles(dtype, nz, nx, nts, sub):
+    """Both Born passes resident for a batch of two shots, twice in the same buffers, and with every wait given
+    up; the gradient against the oracle's, summed over the shots."""
+    ctx = _ctx(dtype)
+    mid, g, med = _model(ctx, nz, nx, nts, sub, nz + nx)
+    rng = np.random.default_rng(nz * nx + 2)
+    shots, keeps, ref = [], [], 0.0
+    for i in range(2 if nz * nx < 400000 else 1):
+        spos, rpos = _positions(rng, g, 10), _positions(rng, g, 80)
+        src = [O.time_interp(s, g.dts, sub) for s in random_traces(rng, spos, nts, np.float64)]
+        dat = random_traces(rng, rpos, nts, np.float64)
+        ref = ref + O.born_adj_reg(g, med, spos, src, rpos, dat, np.float64)
+        shot, keep = ctx.make_shot(mid, spos, rpos, [np.ascontiguousarray(s, dtype) for s in src],
+                                   [np.ascontiguousarray(s, dtype) for s in dat])
+        shots.append(shot)
+        keeps.append(keep)
+    grads = []
+    for limit in (0, 0, 1):
+        if limit:
+            ctx.set_persistent(0, limit)
+        dm = np.zeros((5, nx, nz), dtype)
+        ctx.born_adjoint(shots, dm)
+        assert rel_l2(dm, ref) < (2e-5 if dtype == np.float32 else 1e-10), rel_l2(dm, ref)
+        grads.append(dm)
+    assert np.array_equal(grads[0], grads[1])
+    ctx.close()
