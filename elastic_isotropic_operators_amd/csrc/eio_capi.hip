@@ -1438,19 +1438,22 @@ inline int res_tiles(const ModelBase& m, int R) {
 }
 
 // The passes that run resident and the widest tiles (columns per wave) their registers allow.
-enum class ResKind { NL, DEC, ADJ, BADJ };
+enum class ResKind { NL, DEC, SCAT, ADJ, BADJ };
 template <typename T>
 constexpr int res_max_r(ResKind k) {
-    return sizeof(T) == 8 ? 2 : k == ResKind::NL ? 6 : k == ResKind::BADJ ? 4 : 5;
+    return sizeof(T) == 8 ? 2 : k == ResKind::NL ? 6 : k == ResKind::BADJ || k == ResKind::SCAT ? 4 : 5;
 }
 // Measured time of one fine step of a launch with R columns per wave [us] (every CU busy; the
 // halo exchange and the barriers are about 2.5 us of it, so wide tiles do the most work per
-// time, and narrow ones finish a call that cannot fill the device soonest).
+// time, and narrow ones finish a call that cannot fill the device soonest); the Born passes that trade
+// coarse samples with the imaging include its time.
 template <typename T>
 double res_step_us(ResKind k, int R) {
     constexpr double nl[] = {3.4, 3.85, 5.05, 5.65, 7.0, 8.7}, dec[] = {3.5, 4.0, 5.2, 5.8, 8.2}, f64[] = {5.1, 6.15};
     constexpr double adj[] = {3.35, 4.1, 5.35, 6.0, 8.4}, adj64[] = {5.15, 7.65};
-    constexpr double badj[] = {3.6, 4.5, 6.0, 7.2}, badj64[] = {5.5, 9.0};
+    constexpr double badj[] = {3.9, 5.0, 7.0, 13.3}, badj64[] = {6.9, 15.5};
+    constexpr double scat[] = {3.9, 4.9, 7.2, 11.8}, scat64[] = {7.1, 19.0};
+    if (k == ResKind::SCAT) return sizeof(T) == 8 ? scat64[R - 1] : scat[R - 1];
     if (k == ResKind::ADJ) return sizeof(T) == 8 ? adj64[R - 1] : adj[R - 1];
     if (k == ResKind::BADJ) return sizeof(T) == 8 ? badj64[R - 1] : badj[R - 1];
     return sizeof(T) == 8 ? f64[R - 1] : k == ResKind::NL ? nl[R - 1] : dec[R - 1];
@@ -1594,7 +1597,7 @@ void res_launch(Run<T>& run, const ResPlan& rp, const ResGroup& g, const eio::Sh
 template <typename T, int MODE, bool FSURF = false>
 void res_launch_fwd(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, int k1, bool from_rest, bool save,
                     int dlo = 0, int dhi = -1, const eio::ShotDev<T>* dsh = nullptr) {
-    res_launch<T, res_max_r<T>((MODE & eio::F_DEC) ? ResKind::DEC : ResKind::NL)>(
+    res_launch<T, res_max_r<T>((MODE & eio::F_SS) ? ResKind::SCAT : (MODE & eio::F_DEC) ? ResKind::DEC : ResKind::NL)>(
         run, rp, g, dsh ? dsh : run.d_shots,
         [](auto r) { return reinterpret_cast<const void*>(eio::k_res_fwd<T, decltype(r)::value, MODE, FSURF>); }, k0, k1,
         int(from_rest), int(save), dlo, dhi, run.c->spin_limit);
@@ -1637,15 +1640,18 @@ bool res_allowed(Ctx* c, ResKind kind) {
 }
 
 // The groups of a pass of `per_launch` fine steps a launch (0: each group's own steps), or none
-// where the launched kernels are the faster form.  Launched, a step takes (FP32, two per launch) 2.6
-// us and its cells at 100 GCell/s, 4.2 us at least; (FP64, one per launch) its cells at 22 GCell/s, 6
-// us at least; an adjoint step 3 us and its cells at 75 GCell/s, FP64 5 us and 38 GCell/s.  (Adjoint, us
-// a step, launched and resident: 280 x 472, 4.7 and 3.35; 600 x 1592, 15.2 and 5.9; two of 520 x
-// 1000, 17.2 and 5.9; FP64, two of 280 x 472, 12.0 and 7.65.)  A resident launch takes its steps and a set-up: cleared inboxes, a cooperative launch
-// and the state's first load, some 60 us, and 160 where the state comes from and goes back to memory
-// between segments.  Whole calls, resident against launched: 280 x 472, 396 against 373 us at 64 fine
-// steps, 622 against 635 at 128; 600 x 1592, 262 against 249 us at 10, 310 against 352 at 18; a
+// where the launched kernels are the faster form: their time is a part per step and one per cell (the
+// table below, measured), a resident launch takes its steps and a set-up: cleared inboxes, a cooperative
+// launch and the state's first load, some 60 us, and 160 where the state comes from and goes back to
+// memory between segments.  Whole calls, resident against launched: 280 x 472, 396 against 373 us at 64
+// fine steps, 622 against 635 at 128; 600 x 1592, 262 against 249 us at 10, 310 against 352 at 18; a
 // checkpointed gradient of four shots of 280 x 472 in segments of 46 steps, 43.7 against 37.4 ms.
+// Per step, launched and resident (both Born passes together, with imaging), in us:
+//                       forward      adjoint      Born forward  Born adjoint
+//   280 x 472         4.2   3.4     4.7   3.35   10.4   7.4     12.1   7.5
+//   four of them      7.9   5.05    10.0  5.35   21.8   12.7    24.3   12.3
+//   600 x 1592        12.0  5.65    15.2  5.9    32.6   17.8    35.4   19.4
+//   FP64, 280 x 472   6.0   5.1     8.6   5.15   19.8   12.2    26.2   12.0
 constexpr double RES_SEGMENT_US = 160.0;
 template <typename T>
 std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
@@ -1660,10 +1666,14 @@ std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots
         for (int i = g.s0; i < g.s1; ++i)
             work += double(get_model(c, shots[plan.order[i]].model).n) * (per_launch ? per_launch : plan.nsteps[i]);
     }
-    const bool adj = kind == ResKind::ADJ || kind == ResKind::BADJ;
-    const double launched =
-        sizeof(T) == 4 ? std::max(4.2 * longest, adj ? 3.0 * longest + work / 75e3 : 2.6 * longest + work / 100e3)
-                       : std::max(6.0 * longest, adj ? 5.0 * longest + work / 38e3 : work / 22e3);
+    // launched: us a step and cells a us (FP32 two steps per launch, FP64 one); Born passes with their imaging
+    struct Cost {
+        double step, rate, least;
+    };
+    constexpr Cost f32[] = {{2.6, 100e3, 4.2}, {2.6, 100e3, 4.2}, {4.5, 57e3, 4.5}, {3.0, 75e3, 4.2}, {5.5, 48e3, 5.5}};
+    constexpr Cost f64[] = {{0.0, 22e3, 6.0}, {0.0, 22e3, 6.0}, {7.0, 21e3, 7.0}, {5.0, 38e3, 6.0}, {9.5, 13.5e3, 9.5}};
+    const Cost& l = (sizeof(T) == 4 ? f32 : f64)[int(kind)];
+    const double launched = std::max(l.least * longest, l.step * longest + work / l.rate);
     if (res >= launched) groups.clear();
     return groups;
 }
@@ -2118,8 +2128,35 @@ bool ring_build(Run<T>& run, const ResPlan& rp, ResRing<T>& ring) {
 template <typename T, bool ADJ>
 void launch_ring(Run<T>& run, const ResRing<T>& ring, const ResGroup& g, int j0, int j1) {
     const int t0 = ring.tile0[g.s0], nt = ring.tile0[g.s1] - t0;
-    klaunch(run.c, eio::k_imaging_many<T, ResRing<T>::R, ResRing<T>::WX, ADJ>, dim3(nt), dim3(64 * ResRing<T>::WX),
+    // forward: up to eight blocks share the samples of a tile where the tiles do not fill the device
+    const int ny = ADJ ? 1 : std::max(1, std::min({8, std::abs(j1 - j0) + 1, 4 * run.c->ncu / std::max(1, nt)}));
+    klaunch(run.c, eio::k_imaging_many<T, ResRing<T>::R, ResRing<T>::WX, ADJ>, dim3(nt, ny), dim3(64 * ResRing<T>::WX),
             ring.d_shots, ring.d_tiles + t0, nt, j0, j1);
+}
+
+// The Born scattered pass with every shot resident: the secondary sources of RES_RING coarse intervals
+// into the ring, then these intervals in one launch; false when a shot does not fit, there is no memory for
+// the ring or a wait was given up (the receiver traces are then cleared again).
+template <typename T>
+bool scattered_pass_resident(Run<T>& run, int nshot, const eio_shot* shots) {
+    Ctx* c = run.c;
+    const int nts = run.sd[0].nts, sub = run.sd[0].sub;
+    ResPlan rp;
+    ResRing<T> ring;
+    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::SCAT, std::min(RES_RING, nts - 1) * sub);
+    if (rp.groups.empty() || !ring_build(run, rp, ring)) return false;
+    res_build(run, shots, rp, "resa_");
+    for (const ResGroup& g : rp.groups)
+        for (int a = 0; a < nts - 1; a += ring.K) {   // intervals a .. b-1 use the samples a .. b
+            const int b = std::min(a + ring.K, nts - 1);
+            launch_ring<T, false>(run, ring, g, a > 0 ? a + 1 : 0, b);
+            res_launch_fwd<T, eio::M_BSCAT>(run, rp, g, a * sub, b * sub, a == 0, b < nts - 1, 0, -1, ring.d_shots);
+        }
+    if (!res_aborted(c, rp)) return true;
+    for (int oi = 0; oi < nshot; ++oi)
+        for (int k = 0; k < 5; ++k)
+            fill0<T>(c, run.sd[oi].rec_tr[k], long(shots[run.plan.order[oi]].n_rec[GRID_OF_COMP[k]]) * nts);
+    return false;
 }
 
 // The Born receiver pass of a group: RES_RING coarse intervals a launch, then their imaging.
@@ -2175,6 +2212,7 @@ void born_forward(Ctx* c, int nshot, const eio_shot* shots, const void* const dm
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
     run_loop(c, [&]() {
         if (!born_source_resident(run, nshot, shots)) born_source_pass(run, ntile, kmax);
+        if (scattered_pass_resident(run, nshot, shots)) return;
         // scattered pass restarts from a zero state (BornElasticGpuFunctions.cu:773-774)
         for (int oi = 0; oi < nshot; ++oi) {
             fill0<T>(c, run.sd[oi].A, 5 * m.n);

@@ -322,7 +322,8 @@ struct ResComm {
 };
 
 // Fine steps [k0, k1) of the forward loop (a shot stops at its own last step).  MODE: the flags
-// of k_step_fwd (F_INJ_COARSE, F_INJ_FINE, F_REC, F_DEC); FSURF: shots with a free surface.
+// of k_step_fwd (F_INJ_COARSE, F_INJ_FINE, F_REC, F_DEC, F_SS: secondary sources from the ring of
+// S.sscap coarse samples at S.ss[0], sample j at j % sscap); FSURF: shots with a free surface.
 // k0 is a multiple of the shots' sub-sampling.  The state starts from the levels A (older) and
 // B (current), or from rest with from_rest, and goes back there with save.
 template <typename T, int R, int MODE, bool FSURF>
@@ -339,13 +340,19 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
     constexpr bool INJ = (MODE & (F_INJ_COARSE | F_INJ_FINE)) != 0;
     constexpr bool REC = (MODE & F_REC) != 0;
     constexpr bool DEC = (MODE & F_DEC) != 0;
+    constexpr bool SS = (MODE & F_SS) != 0;
     constexpr bool PAIR = sizeof(T) == 4 && !FSURF;
     constexpr bool PIN = sizeof(T) == 8 || FSURF || R >= 4;
     // the widest tiles read the media again each step (20 B a cell, from L2) where registers end
     // (R = 5: 7.0 us a step with the media in registers and 10 spilled ones, 7.8 without them)
-    constexpr bool MEML2 = sizeof(T) == 4 && (R >= 6 || (R >= 5 && DEC));
+    constexpr bool NOW = SS && R >= (sizeof(T) == 4 ? 4 : 2);  // nor for a coarse sample on its way
+    constexpr bool MEML2 = sizeof(T) == 4 && (R >= 6 || (R >= 5 && DEC) || NOW);
     constexpr int RM = MEML2 ? 1 : R;
+    // secondary sources: the coarse sample its in registers, SL fields of its+1 in the LDS that the stage leaves
+    constexpr int RS = SS ? R : 1;
+    constexpr int SL = !SS ? 0 : sizeof(T) == 4 ? (R <= 3 ? 5 : 3) : (R <= 1 ? 5 : 2);
     __shared__ __attribute__((aligned(16))) T L[5][TXH][ZH];
+    __shared__ T LS[SL ? SL : 1][SL ? TX : 1][64];
     __shared__ int s_stop;
 
     const int tile = xcd_remap(blockIdx.x, ntiles);
@@ -474,6 +481,35 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
             }
         }
     };
+    // secondary sources of the own cells: samples its (gl) and its+1 (gr, fields 0 .. SL-1 in LS), and
+    // the next one on its way
+    T gl[5][RS], gr[5][RS], gn[5][RS];
+    const unsigned las = unsigned(reinterpret_cast<uintptr_t>((LdsT<T>*)&LS[0][SL ? w * R : 0][lane]));
+    auto ls = [&](int f, int r) { return const_cast<LdsT<T>*>(lds_at<T>(las, (f * TX + r) * 64)); };
+    auto load_ss = [&](int j, T (&u)[5][RS]) {
+        const rsrc_t rs = make_rsrc(S.ss[0] + size_t(j % S.sscap) * 5 * n, 5 * fbytes);
+#pragma unroll
+        for (int r = 0; r < RS; ++r)
+#pragma unroll
+            for (int f = 0; f < 5; ++f)
+                u[f][r] = zok && r < ncol ? bld<T>(rs, voff, unsigned(r) * colb + unsigned(f) * fbytes) : T(0);
+    };
+    auto take_ss = [&]() {  // gn becomes sample its+1
+#pragma unroll
+        for (int r = 0; r < RS; ++r)
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+                gl[f][r] = f < SL ? T(*ls(f, r)) : gr[f][r];
+                if (f < SL) *ls(f, r) = gn[f][r];
+                else gr[f][r] = gn[f][r];
+            }
+    };
+    if constexpr (SS) {
+        load_ss(its0, gn);
+        take_ss();
+        load_ss(its0 + 1, gn);
+        take_ss();
+    }
     constexpr int XG = sizeof(T) == 4 ? 4 : 2;  // columns within reach of one address
     // x derivative D+ / D- of staged field f at the own columns (a register window of R+8);
     // mid: the own values
@@ -512,7 +548,7 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
 #pragma unroll
         for (int f = 0; f < 5; ++f) mnext[f] = zok && r < ncol ? bld<T>(rmed, voff, unsigned(r) * colb + unsigned(f) * fbytes) : T(0);
     };
-    auto update = [&](bool odd) {
+    auto update = [&](bool odd, T fl, T fr) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             T mm[5];
@@ -539,6 +575,11 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
                 a3 = d[r] * o[3][r] + (below ? (mm[3] * vxx[r] + mm[2] * vzz) : T(0));
                 a4 = d[r] * o[4][r] + (below ? mm[4] * sh : T(0));
             }
+            if constexpr (SS) {  // secondary source sampled at it2-1 (kernelsGpuElastic.cu:1363-1368)
+                T* const a[5] = {&a0, &a1, &a2, &a3, &a4};
+#pragma unroll
+                for (int f = 0; f < 5; ++f) *a[f] += gl[f][r] * fl + (f < SL ? T(*ls(f, r)) : gr[f][r]) * fr;
+            }
             o[0][r] = d[r] * a0;
             o[1][r] = d[r] * a1;
             o[2][r] = d[r] * a2;
@@ -561,6 +602,8 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
         const unsigned pr = (unsigned(k) & 1u) * PARITY;
         Quad<T> q[ResComm<T, R>::NQ];
         if (k > k0) cm.send_x(Lf, k, pr);
+        if constexpr (SS)
+            if (!NOW && k > k0 && it2 == 0) take_ss();
         if (!edge) dx_all(js, j2);
         if (k > k0) {
             cm.request(q, pr);
@@ -570,7 +613,7 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
         if (s_stop) return;
         if (MEML2) load_media(0);
         if (edge) dx_all(js, j2);
-        update(k & 1);
+        update(k & 1, SS ? filt[it2] : T(0), SS ? filt[h + it2] : T(0));
         __syncthreads();  // every read of level k is done
         // the next level is staged, this one becomes the older one; what follows touches the
         // wave's own columns only, and the LDS accesses of one wave are in order
@@ -644,6 +687,11 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
                 }
             __builtin_amdgcn_wave_barrier();
         }
+        if constexpr (SS)
+            if (it2 + 1 == sub && k + 1 < kend) {
+                load_ss(its + 2, gn);
+                if (NOW) take_ss();
+            }
         if (k + 1 < kend) cm.send_z(Lf, k + 1, PARITY - pr);
         if (++it2 == sub) {
             it2 = 0;
@@ -1029,6 +1077,12 @@ void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
 template <typename T, int R, int WX, bool ADJ>
 __global__ __launch_bounds__(64 * WX) void k_imaging_many(const ShotDev<T>* __restrict__ shots,
                                                           const TileDev* __restrict__ tiles, int ntiles, int j0, int j1) {
+    if (!ADJ) {  // the samples are independent: the grid's y direction shares them out
+        const int per = (j1 - j0 + int(gridDim.y)) / int(gridDim.y);
+        j0 += int(blockIdx.y) * per;
+        j1 = min(j1, j0 + per - 1);
+        if (j0 > j1) return;
+    }
     constexpr int NT = 64 * WX;
     constexpr int TX = WX * R;
     constexpr int TXH = TX + 2 * FAT;

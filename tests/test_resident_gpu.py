@@ -282,3 +282,46 @@ def test_born_adjoint_tiles(dtype, nz, nx, nts, sub):
         grads.append(dm)
     assert np.array_equal(grads[0], grads[1])
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype,nz,nx,nts,sub", [
+    (np.float32, 73, 25, 70, 3),      # R = 1, one row and one column over, three launches of 32 coarse intervals
+    (np.float32, 76, 28, 34, 4),      # one interval over a launch
+    (np.float32, 139, 90, 33, 4),     # exactly one launch
+    (np.float32, 281, 967, 40, 2),    # R = 2
+    (np.float32, 563, 1103, 40, 2),   # R = 3
+    (np.float32, 601, 1593, 40, 2),   # R = 4
+    (np.float64, 73, 25, 70, 3),
+    (np.float64, 281, 967, 40, 2),    # R = 2
+])
+def test_born_forward_tiles(dtype, nz, nx, nts, sub):
+    """Both passes of the Born forward resident for a batch of two shots, twice in the same buffers, and with
+    every wait given up; the data against the oracle's."""
+    ctx = _ctx(dtype)
+    mid, g, med = _model(ctx, nz, nx, nts, sub, nz + nx)
+    rng = np.random.default_rng(nz * nx + 3)
+    dm = np.zeros((5, nx, nz))
+    dm[:, 4:-4, 4:-4] = rng.standard_normal((5, nx - 8, nz - 8)) * np.abs(med).reshape(5, -1).max(1)[:, None, None]
+    shots, keeps, recs, refs = [], [], [], []
+    for i in range(2 if nz * nx < 400000 else 1):
+        spos, rpos = _positions(rng, g, 10), _positions(rng, g, 300)
+        src = [O.time_interp(s, g.dts, sub) for s in random_traces(rng, spos, nts, np.float64)]
+        refs.append(O.born_fwd_reg(g, med, spos, src, dm, rpos, np.float64))
+        rec = [np.zeros((rpos[GRID_OF_COMP[k]].size, nts), dtype) for k in range(5)]
+        shot, keep = ctx.make_shot(mid, spos, rpos, [np.ascontiguousarray(s, dtype) for s in src], rec)
+        shots.append(shot)
+        keeps.append(keep)
+        recs.append(rec)
+    dmd = np.ascontiguousarray(dm, dtype)
+    first = None
+    for limit in (0, 0, 1):
+        if limit:
+            ctx.set_persistent(0, limit)
+        ctx.born_forward(shots, dmd)
+        for rec, ref in zip(recs, refs):
+            _check(rec, ref, dtype)
+        if first is None:
+            first = [[r.copy() for r in rec] for rec in recs]
+        elif not limit:
+            assert all(np.array_equal(a, b) for x, y in zip(first, recs) for a, b in zip(x, y))
+    ctx.close()
