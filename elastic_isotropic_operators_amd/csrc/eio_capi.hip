@@ -1642,17 +1642,17 @@ bool res_allowed(Ctx* c, ResKind kind) {
 // The groups of a pass of `per_launch` fine steps a launch (0: each group's own steps), or none
 // where the launched kernels are the faster form: their time is a part per step and one per cell (the
 // table below, measured), a resident launch takes its steps and a set-up: cleared inboxes, a cooperative
-// launch and the state's first load, some 60 us, and 160 where the state comes from and goes back to
+// launch and the state's first load, some 60 us, and 100 where the state comes from and goes back to
 // memory between segments.  Whole calls, resident against launched: 280 x 472, 396 against 373 us at 64
 // fine steps, 622 against 635 at 128; 600 x 1592, 262 against 249 us at 10, 310 against 352 at 18; a
-// checkpointed gradient of four shots of 280 x 472 in segments of 46 steps, 43.7 against 37.4 ms.
+// checkpointed forward and gradient of four shots of 280 x 472 in segments of 46 steps, 24.4 against 28.2 ms.
 // Per step, launched and resident (both Born passes together, with imaging), in us:
 //                       forward      adjoint      Born forward  Born adjoint
 //   280 x 472         4.2   3.4     4.7   3.35   10.4   7.4     12.1   7.5
 //   four of them      7.9   5.05    10.0  5.35   21.8   12.7    24.3   12.3
 //   600 x 1592        12.0  5.65    15.2  5.9    32.6   17.8    35.4   19.4
 //   FP64, 280 x 472   6.0   5.1     8.6   5.15   19.8   12.2    26.2   12.0
-constexpr double RES_SEGMENT_US = 160.0;
+constexpr double RES_SEGMENT_US = 100.0;
 template <typename T>
 std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
     if (!res_allowed<T>(c, kind)) return {};
