@@ -40,6 +40,8 @@ from elastic_isotropic_operators_amd import _capi, autotune, geometry as G, work
 
 BYTES_PER_CELL = {"nl_fwd": 80}
 HBM_PEAK_GBS = 8000.0
+FLOPS_PER_CELL = 117        # eight 8-point derivatives (11 each) and the five updates, a fused one as two
+FP32_PEAK_TFLOPS = 78.6     # 256 CUs x 128 FP32 lanes x 2 x 2.4 GHz / 2 (no packed FP32)
 METRIC = "GCell-updates/s + FWI-gradient s/shot at \u22641e-4 rel-L2 vs FP64, 1 MI355X"
 # measured bytes per cell-update of the dominant kernel per (time block, variant, grouping)
 TRAFFIC_FILES = [os.path.join(ROOT, "profiles", f) for f in
@@ -140,8 +142,8 @@ def _oracle_grid(O, w, nts=None):
 
 
 def c0_leg(args):
-    """Unbatched leg (workload C0: one 280x472 shot, nts 1000, sub_fd 2): the two-step NL
-    forward with one launch per pair of fine steps, the same loop replayed from the context's
+    """Unbatched leg (workload C0: one 280x472 shot, nts 1000, sub_fd 2): the NL forward as
+    the library runs it (one resident launch), with one launch per pair of fine steps, the same loop replayed from the context's
     cached hipGraph, the whole loop in one persistent launch, and the three-step forward (one
     launch per three fine steps); device time per call (HIP events) after warm-up calls, best
     of `args.c0_reps`; plus the FP32 oracle on the host cores (the whole shot)."""
@@ -151,10 +153,10 @@ def c0_leg(args):
     ctx.set_time_block(2, _capi.VARIANT_AUTO)
     shots, keep, _, _ = prepare_shots(ctx, [w])
     out = {"workload": w["name"], "cell_updates": cells, "dtype": "f32"}
-    for mode in ("launched", "graph", "persistent", "three_step"):
+    for mode in ("resident", "launched", "graph", "persistent", "three_step"):
         ctx.set_graph(mode == "graph")
         ctx.set_persistent(1 if mode == "persistent" else 0)
-        ctx.set_time_block(3 if mode == "three_step" else 2, _capi.VARIANT_AUTO)
+        ctx.set_time_block(3 if mode == "three_step" else 2, 12 if mode == "launched" else _capi.VARIANT_AUTO)
         for _ in range(2):
             ctx.nl_forward(shots, device_ptrs=True)
         ms = []
@@ -564,7 +566,12 @@ def main():
     value = cells * args.steps / elapsed / 1e9
     loop_s = float(np.mean([s * n for s, n in zip(step_ms, nlaunch)])) / 1e3
     achieved = BYTES_PER_CELL["nl_fwd"] * cells / loop_s / 1e9
-    if (args.time_block == 3 and args.variant3 < 0) or (args.time_block == 2 and args.variant2 < 0):
+    groups = ctx.last_shot_groups()
+    # the library's choice, one launch per group: the state of the shots stays on the chip
+    resident = args.time_block == 2 and args.variant2 < 0 and nlaunch[-1] == groups
+    if resident:
+        kname = "k_res_fwd<float,R,M_NL> (a group's whole loop per launch, R = 1..6 columns per wave)"
+    elif (args.time_block == 3 and args.variant3 < 0) or (args.time_block == 2 and args.variant2 < 0):
         kname = "k_step%d_fwd (the library's automatic variant per call, %d fine steps per launch)" % (
             args.time_block, args.time_block)
     elif args.time_block == 3:
@@ -581,7 +588,6 @@ def main():
     else:
         R, WX, OCC = _capi.Context.variants()[args.variant if args.variant >= 0 else 1]
         kname = "k_step_fwd<float,%d,%d,%d,M_NL>" % (R, WX, OCC)
-    groups = ctx.last_shot_groups()
     if groups > 1:
         kname += " in %d shot groups" % groups
     res = {
@@ -617,6 +623,14 @@ def main():
                               "time per launch) is half a kernel's own duration")
                      if groups > 1 else "achieved counts the reference algorithm's 80 B per cell-update"},
     }
+    if resident:  # no state crosses HBM: priced in arithmetic
+        tflops = FLOPS_PER_CELL * cells / loop_s / 1e12
+        res["roofline"].update({
+            "bound": "fp32 vector", "achieved": round(tflops, 2), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+            "frac": round(tflops / FP32_PEAK_TFLOPS, 4), "bytes_per_cell_update": None, "concurrent_streams": 1,
+            "flops_per_cell_update": FLOPS_PER_CELL, "equivalent_GBs": round(achieved, 1),
+            "note": "the time loop keeps levels and media in LDS and registers; equivalent_GBs is the reference "
+                    "algorithm's 80 B per cell-update over the loop"})
     if args.copy_probe:
         nb = 2 << 30
         cms = ctx.copy_probe(nb, 10, kind=1)

@@ -1430,6 +1430,7 @@ struct ResPlan {
     size_t inbox_bytes = 0;
     int* abort_flag = nullptr;
     int* xcd = nullptr;     // the XCD each workgroup of a launch runs on
+    mutable bool refused = false;   // the device took no cooperative launch
 };
 
 inline int res_tiles(const ModelBase& m, int R) {
@@ -1568,6 +1569,7 @@ void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp, const std::strin
 template <typename T, int RMAX, typename Pick, typename... A>
 void res_launch(Run<T>& run, const ResPlan& rp, const ResGroup& g, const eio::ShotDev<T>* sh, Pick&& kernel, A... extra) {
     Ctx* c = run.c;
+    if (rp.refused) return;
     // packets of another group, call or segment may carry the levels of this one
     fill0<T>(c, static_cast<T*>(rp.inbox), long(rp.inbox_bytes / sizeof(T)));
     fill0<int>(c, rp.xcd, c->ncu);
@@ -1590,7 +1592,14 @@ void res_launch(Run<T>& run, const ResPlan& rp, const ResGroup& g, const eio::Sh
     pick(std::integral_constant<int, 4>{});
     pick(std::integral_constant<int, 5>{});
     pick(std::integral_constant<int, 6>{});
-    EIO_CHECK_HIP(hipLaunchCooperativeKernel(fn, dim3(nt), dim3(64 * RES_WX), args, 0, c->stream));
+    const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(nt), dim3(64 * RES_WX), args, 0, c->stream);
+    if (e != hipSuccess) {
+        // refused (one process at a time holds a device's cooperative queue): the context keeps to the
+        // launched kernels from here on, this call included
+        (void)hipGetLastError();
+        c->resident = false;
+        rp.refused = true;
+    }
 }
 
 // Fine steps [k0, k1) of a group's forward loop.  `dsh` replaces the run's shot table.
@@ -1613,8 +1622,10 @@ void res_launch_adj(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, i
         int(from_rest), int(save), run.c->spin_limit);
 }
 
-// Whether the resident launches of this call gave up a wait (the call then repeats launched).
+// Whether the resident launches of this call were refused or gave up a wait (the call then repeats
+// launched).
 inline bool res_aborted(Ctx* c, const ResPlan& rp) {
+    if (rp.refused) return true;
     int aborted = 0;
     EIO_CHECK_HIP(hipMemcpyAsync(&aborted, rp.abort_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     EIO_CHECK_HIP(hipStreamSynchronize(c->stream));

@@ -3,6 +3,10 @@ the FP64 oracle, at the sizes where their tiles can go wrong: 64 rows by 16 R co
 with remainders of one to four rows and columns, tiles that end on the grid's edge, more devices than
 a wave keeps in registers, uneven batches, and the repeat with launched kernels after a wait is given up.
 Bars: those of the launched kernels, FP32 1e-5 and FP64 1e-11 relative L2."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -325,3 +329,57 @@ def test_born_forward_tiles(dtype, nz, nx, nts, sub):
         elif not limit:
             assert all(np.array_equal(a, b) for x, y in zip(first, recs) for a, b in zip(x, y))
     ctx.close()
+
+
+_CHILD = """
+import sys
+import numpy as np
+from elastic_isotropic_operators_amd import _capi
+import test_resident_gpu as t
+out = t._second_process_case()
+np.save(sys.argv[1], out)
+"""
+
+
+def _second_process_case():
+    """Data of an NL forward, an NL adjoint and both Born passes of one shot, in one row."""
+    ctx = _ctx(np.float32)
+    mid, g, med = _model(ctx, 139, 90, 90, 2, 21)
+    rng = np.random.default_rng(22)
+    spos, rpos = _positions(rng, g, 10), _positions(rng, g, 20)
+    src = [np.ascontiguousarray(s, np.float32) for s in random_traces(rng, spos, g.nts, np.float64)]
+    fine = [np.ascontiguousarray(O.time_interp(s.astype(np.float64), g.dts, 2), np.float32) for s in src]
+    dat = [np.ascontiguousarray(s, np.float32) for s in random_traces(rng, rpos, g.nts, np.float64)]
+    rec = [np.zeros_like(d) for d in dat]
+    back = [np.zeros_like(s) for s in src]
+    dm = np.zeros((5, g.nx, g.nz), np.float32)
+    lin = [np.zeros_like(d) for d in dat]
+    keep = []
+
+    def shot(s, r):
+        sh, k = ctx.make_shot(mid, spos, rpos, s, r)
+        keep.append(k)
+        return [sh]
+
+    ctx.nl_forward(shot(src, rec))
+    ctx.nl_adjoint(shot(back, dat))
+    ctx.born_adjoint(shot(fine, dat), dm)
+    ctx.born_forward(shot(fine, lin), np.ascontiguousarray(dm / np.abs(dm).max()))
+    h = ctx.fwi_forward(shot(src, rec), 44)
+    ctx.fwi_gradient(h, shot(src, dat), dm)
+    ctx.fwi_release(h)
+    ctx.close()
+    parts = rec + back + [dm] + lin
+    return np.concatenate([p.ravel() / np.linalg.norm(p) for p in parts])
+
+
+def test_second_process(tmp_path):
+    """Another process that uses the device while this one holds its cooperative queue: the same results, with
+    launched kernels where it gets no cooperative launch."""
+    mine = _second_process_case()
+    here = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([here, os.path.dirname(here)] + sys.path))
+    out = str(tmp_path / "out.npy")
+    subprocess.run([sys.executable, "-c", _CHILD, out], check=True, env=env, timeout=90)
+    theirs = np.load(out)
+    assert theirs.shape == mine.shape and rel_l2(theirs, mine) < 1e-5, rel_l2(theirs, mine)
