@@ -452,6 +452,17 @@ def run_abc_leg(args):
     raise RuntimeError("learned-boundary leg failed (exit %d)" % r.returncode)
 
 
+def run_leg(args, res, key, name, run):
+    """One secondary leg; one that fails is reported in its own field and does not cost the
+    headline line."""
+    t0 = time.perf_counter()
+    try:
+        res[key] = run(args)
+    except Exception as e:  # noqa: BLE001 (reported in the JSON line)
+        res[key] = {"error": "%s: %s" % (type(e).__name__, e)}
+    log("%s leg %.1f s" % (name, time.perf_counter() - t0))
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -506,6 +517,16 @@ def main():
               "shots would be partitioned (one batch per GPU) with one all-reduce of the FWI "
               "gradient and misfit.", file=sys.stderr)
         sys.exit(2)
+
+    # the secondary legs run in child processes, before this one launches anything: one process at a
+    # time holds the device's cooperative queue, which the resident loops need
+    side = {}
+    if args.fwi:
+        run_leg(args, side, "fwi_gradient", "fwi", run_fwi_leg)
+    if args.born:
+        run_leg(args, side, "born", "born", run_born_leg)
+    if args.abc and os.path.exists(ABC_WEIGHTS):
+        run_leg(args, side, "learned_boundary", "learned-boundary", run_abc_leg)
 
     t_build = time.perf_counter()
     if args.workload == "c2":
@@ -659,24 +680,9 @@ def main():
             res["roofline"]["traffic_source"] = os.path.relpath(tf, ROOT)
             if "traffic_level" in tr:
                 res["roofline"]["traffic_level"] = tr["traffic_level"]
-    # the secondary legs run in child processes; one that fails is reported in its own field
-    # and does not cost the headline line
-    legs = []
     if args.c0:
-        legs.append(("unbatched_c0", "unbatched C0", c0_leg))
-    if args.fwi:
-        legs.append(("fwi_gradient", "fwi", run_fwi_leg))
-    if args.born:
-        legs.append(("born", "born", run_born_leg))
-    if args.abc and os.path.exists(ABC_WEIGHTS):
-        legs.append(("learned_boundary", "learned-boundary", run_abc_leg))
-    for key, name, run in legs:
-        t0 = time.perf_counter()
-        try:
-            res[key] = run(args)
-        except Exception as e:  # noqa: BLE001 (reported in the JSON line)
-            res[key] = {"error": "%s: %s" % (type(e).__name__, e)}
-        log("%s leg %.1f s" % (name, time.perf_counter() - t0))
+        run_leg(args, res, "unbatched_c0", "unbatched C0", c0_leg)
+    res.update(side)
     if not args.no_cpu:
         t0 = time.perf_counter()
         res["cpu_baseline"] = cpu_baseline(shots_w)

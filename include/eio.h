@@ -109,7 +109,13 @@ int eio_ctx_set_variant(eio_ctx* ctx, int variant);
  * (owned tile 56 x WX*R2), or EIO_VARIANT_AUTO: per call, 56 x 8 tiles with the streamed
  * stage at 8 waves per SIMD (variant 12) for a batch of fewer than 1024 tiles of 56 x 32 and
  * for an NL forward that runs in several shot groups (eio_ctx_set_shot_group_bytes), else
- * 56 x 32 (variant 4).
+ * 56 x 32 (variant 4).  With EIO_VARIANT_AUTO, time block 2 and EIO_GROUP_AUTO (and in every FP64
+ * context), a pass whose shots fit the chip runs as RESIDENT loops instead where that is faster: one
+ * cooperative launch for the whole loop of a group of shots (32 coarse intervals at a time in the Born
+ * scattered and receiver passes), the state in LDS and registers.  eio_ctx_last_timing then counts these
+ * launches for the NL forward, eio_ctx_last_shot_groups the groups.  Graphs, the persistent mode, explicit
+ * variants, saved wavefields, snapshots, learned boundaries and the no-allocation call keep to launched
+ * steps, and so does a context whose device refuses a cooperative launch (another process holds it).
  * It applies to the NL forward (without
  * saved wavefield, free surface or learned boundary), the whole-record FWI forward and the
  * Born source and scattered passes.  No counterpart in the reference. */
@@ -139,7 +145,9 @@ int eio_ctx_time_block_layout(int variant);
  * shot; the Born adjoint fields of the pair are extracted with at most one read-modify-write
  * of each coarse slot), and the variant of the two-step adjoint kernel (owned tile
  * 56 x WX*R2), or EIO_VARIANT_AUTO: per call, 56 x 8 tiles (variant 10) for a batch of fewer
- * than 1024 tiles of 56 x 32, else 56 x 32 (variant 7).  FP64 contexts ignore it.  No counterpart in the reference (its receiver pass,
+ * than 1024 tiles of 56 x 32, else 56 x 32 (variant 7), or resident loops (see
+ * eio_ctx_set_time_block) for shots that fit the chip.  FP64 contexts ignore it and run resident where
+ * that is faster.  No counterpart in the reference (its receiver pass,
  * BornElasticGpuFunctions.cu:262-370, and its NL adjoint take one step per launch). */
 int eio_ctx_num_adjoint_time_block_variants(void);
 int eio_ctx_adjoint_time_block_info(int variant, int* R2, int* WX, int* occ);
@@ -149,7 +157,8 @@ int eio_ctx_set_adjoint_time_block(eio_ctx* ctx, int steps, int variant);
  * tile of the batch gets its own co-resident workgroup.  The grid is launched cooperatively;
  * tiles wait for their neighbours' previous pair through per-tile flags (no grid barrier).
  * spin_limit > 0 replaces the number of polls a wait may take before the launch is abandoned
- * with EIO_ERR_RUNTIME (default 2^20).  No counterpart in the reference, which launches every
+ * with EIO_ERR_RUNTIME (default 2^20); a resident loop that gives up a wait is repeated with launched
+ * kernels instead.  No counterpart in the reference, which launches every
  * kernel of every fine step (nonlinearPropElasticGpuFunctions.cu:588-617). */
 int eio_ctx_set_persistent(eio_ctx* ctx, int mode, int spin_limit);
 /* Tuning runs: NL forward and adjoint loops stop after `max_steps` fine steps (0: no limit).
