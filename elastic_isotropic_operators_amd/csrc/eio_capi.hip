@@ -1452,7 +1452,7 @@ template <typename T>
 double res_step_us(ResKind k, int R) {
     constexpr double nl[] = {3.4, 3.85, 5.05, 5.65, 7.0, 8.7}, dec[] = {3.5, 4.0, 5.2, 5.8, 8.2}, f64[] = {5.1, 6.15};
     constexpr double adj[] = {3.35, 4.1, 5.35, 6.0, 8.4}, adj64[] = {5.15, 7.65};
-    constexpr double badj[] = {3.9, 5.0, 7.0, 13.3}, badj64[] = {6.9, 15.5};
+    constexpr double badj[] = {3.9, 5.0, 7.0, 10.7}, badj64[] = {6.9, 14.0};
     constexpr double scat[] = {3.9, 4.9, 7.2, 11.8}, scat64[] = {7.1, 19.0};
     if (k == ResKind::SCAT) return sizeof(T) == 8 ? scat64[R - 1] : scat[R - 1];
     if (k == ResKind::ADJ) return sizeof(T) == 8 ? adj64[R - 1] : adj[R - 1];
@@ -1661,7 +1661,7 @@ bool res_allowed(Ctx* c, ResKind kind) {
 //                       forward      adjoint      Born forward  Born adjoint
 //   280 x 472         4.2   3.4     4.7   3.35   10.4   7.4     12.1   7.5
 //   four of them      7.9   5.05    10.0  5.35   21.8   12.7    24.3   12.3
-//   600 x 1592        12.0  5.65    15.2  5.9    32.6   17.8    35.4   19.4
+//   600 x 1592        12.0  5.65    15.2  5.9    32.6   17.8    35.4   16.5
 //   FP64, 280 x 472   6.0   5.1     8.6   5.15   19.8   12.2    26.2   12.0
 constexpr double RES_SEGMENT_US = 100.0;
 template <typename T>

@@ -741,7 +741,10 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
 // k_step_adj), so the current level itself stays in registers with the older one.  Bound as the
 // forward loop is (a step of R = 4 with the media from L2 where registers end); two shots of 520 x
 // 1000, R = 4, 5.9 us a reverse step against 17.2 with two steps per launch, 280 x 472, R = 1, 3.35
-// against 4.7, and FP64, two of 280 x 472, R = 2, 7.65 against 12.0.
+// against 4.7, and FP64, two of 280 x 472, R = 2, 7.65 against 12.0.  The receiver pass (with the source
+// pass and the imaging): 600 x 1592, R = 4, 16.5 against 35.4 (19.4 with the media from L2 and every x
+// derivative held over the exchange, 34 registers spilled; 17.6 with the derivatives one field at a time);
+// four of 280 x 472, R = 3, 12.3 against 24.3.
 template <typename T, int R, int MODE>
 __global__ __launch_bounds__(64 * RES_WX) __attribute__((amdgpu_waves_per_eu(RES_WX / 4, RES_WX / 4)))
 void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__ tiles,
@@ -754,11 +757,17 @@ void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
     constexpr int FS = TXH * ZH;
     constexpr unsigned SZ = sizeof(T);
     constexpr bool BORN = MODE == M_BADJ;
-    constexpr bool MEML2 = sizeof(T) == 4 && R >= (BORN ? 4 : 5);
+    // where registers end: the receiver pass takes its x derivatives one field at a time behind the halos
+    // and keeps ML media fields in the LDS that the stage leaves; the NL adjoint reads the media again each
+    // step (from L2)
+    constexpr bool WIDE = BORN && R >= (sizeof(T) == 4 ? 4 : 2);
+    constexpr int ML = !WIDE ? 0 : sizeof(T) == 4 ? 3 : 2;
+    constexpr bool MEML2 = !BORN && sizeof(T) == 4 && R >= 5;
     constexpr int RM = MEML2 ? 1 : R;
     constexpr int RB = BORN ? R : 1;
     constexpr bool PIN = sizeof(T) == 8 || R >= 3;
     __shared__ __attribute__((aligned(16))) T L[5][TXH][ZH];
+    __shared__ T LM[ML ? ML : 1][ML ? TX : 1][64];
     __shared__ int s_stop;
 
     const int tile = xcd_remap(blockIdx.x, ntiles);
@@ -794,7 +803,9 @@ void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
             for (int f = 0; f < 5; ++f) {
                 const unsigned so = unsigned(r) * colb + unsigned(f) * fbytes;
                 const bool ok = zok && r < ncol;
-                if (!MEML2) m[f][MEML2 ? 0 : r] = ok ? bld<T>(rmed, voff, so) : T(0);
+                const T mf = !MEML2 && ok ? bld<T>(rmed, voff, so) : T(0);
+                if (f < ML) LM[f < ML ? f : 0][ML ? w * R + r : 0][lane] = mf;
+                else if (!MEML2) m[f][MEML2 ? 0 : r] = mf;
                 o[f][r] = !from_rest && ok ? bld<T>(rold, voff, so) : T(0);
                 c[f][r] = !from_rest && ok ? bld<T>(rcur, voff, so) : T(0);
             }
@@ -820,6 +831,7 @@ void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
     cm.init(t, tile, w, lane, nz, nx, inbox, inbox_bytes, abort_flag, xcd, spin_limit);
     const bool edge = (w * R < FAT && t.left >= 0) || (w * R + R > TX - FAT && t.right >= 0);
     const unsigned lax = unsigned(reinterpret_cast<uintptr_t>((LdsT<T>*)&L[0][c0 - FAT][zz]));
+    const unsigned lam = unsigned(reinterpret_cast<uintptr_t>((LdsT<T>*)&LM[0][ML ? w * R : 0][lane]));
     const unsigned laz = unsigned(reinterpret_cast<uintptr_t>((LdsT<T>*)&L[0][c0][zz - FAT]));
 
     // the wave's entries (data to inject, source cells to read), the first 64 of each in registers
@@ -909,15 +921,38 @@ void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
         const unsigned pr = (unsigned(k) & 1u) * PARITY;
         Quad<T> q[ResComm<T, R>::NQ];
         if (k > k0) cm.send_x(Lf, k, pr);
-        if (!edge) dx_all();
+        if (!WIDE && !edge) dx_all();
         if (k > k0) {
             cm.request(q, pr);
             if (!cm.receive(q, Lf, k, pr)) s_stop = 1;
         }
         __syncthreads();  // the halos are staged
         if (s_stop) return;
-        if (edge) dx_all();
+        if (!WIDE && edge) dx_all();
         // the next level into o, which trades places with the current one
+        if constexpr (WIDE) {
+            T x[R];
+            auto next = [&](int f, int r, T sum) {
+                const T v = d[r] * (d[r] * o[f][r] - sum);
+                o[f][r] = c[f][r];
+                c[f][r] = v;
+                asm volatile("" : "+v"(c[f][r]), "+v"(o[f][r]));
+            };
+            dx(2, false, x);
+#pragma unroll
+            for (int r = 0; r < R; ++r) next(0, r, x[r] + dp_l(lds_at<T>(laz, 4 * FS + r * ZH), cz));
+            dx(4, true, x);
+#pragma unroll
+            for (int r = 0; r < R; ++r) next(1, r, dm_l(lds_at<T>(laz, 3 * FS + r * ZH), cz) + x[r]);
+            dx(0, true, x);
+#pragma unroll
+            for (int r = 0; r < R; ++r) next(2, r, x[r]);
+#pragma unroll
+            for (int r = 0; r < R; ++r) next(3, r, dp_l(lds_at<T>(laz, FS + r * ZH), cz));
+            dx(1, false, x);
+#pragma unroll
+            for (int r = 0; r < R; ++r) next(4, r, dm_l(lds_at<T>(laz, r * ZH), cz) + x[r]);
+        } else {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const T d6 = dp_l(lds_at<T>(laz, 4 * FS + r * ZH), cz);
@@ -940,6 +975,7 @@ void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
                 for (int f = 0; f < 5; ++f) asm volatile("" : "+v"(c[f][r]), "+v"(o[f][r]));
                 __builtin_amdgcn_sched_barrier(0);
             }
+        }
         }
         if (MEML2) load_media(0);
         __syncthreads();  // every read of level k is done
@@ -1007,7 +1043,8 @@ void k_res_adj(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
         for (int r = 0; r < R; ++r) {
             T g[5];
 #pragma unroll
-            for (int f = 0; f < 5; ++f) g[f] = MEML2 ? mnext[f] : m[f][MEML2 ? 0 : r];
+            for (int f = 0; f < 5; ++f)
+                g[f] = f < ML ? T(*lds_at<T>(lam, (f * TX + r) * 64)) : MEML2 ? mnext[f] : m[f][MEML2 ? 0 : r];
             if (MEML2 && r + 1 < R) load_media(r + 1);
             if (zok && r < ncol) {
                 LdsT<T>* p = const_cast<LdsT<T>*>(lds_at<T>(laz, r * ZH + FAT));
