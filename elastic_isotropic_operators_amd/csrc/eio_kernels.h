@@ -202,16 +202,33 @@ __device__ __forceinline__ void fs_map_col_transpose(T* vx, T* vz, T* szz, T* sx
     for (int r = SURF - 4; r <= SURF; ++r) vz[r] = T(0);
 }
 
+// Sums of products.  FP64 spells its fused operations out, because which product the compiler fuses
+// changes with the code around it and a call has to give the same bits launched and resident (k_res_fwd);
+// FP32 calls get theirs from k_step2_fwd and its resident counterpart.
+template <typename T>
+__device__ __forceinline__ T mac(T acc, T a, T b) {  // acc + a*b
+    if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, acc);
+    else return acc + a * b;
+}
+template <typename T>
+__device__ __forceinline__ T mul2(T a, T b, T c, T d) {  // a*b + c*d
+    if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, c * d);
+    else return a * b + c * d;
+}
+template <typename T>
+__device__ __forceinline__ T taps(const T* c, T d0, T d1, T d2, T d3) {  // sum_k C_k d_k
+    if constexpr (sizeof(T) == 8) return __builtin_fma(c[3], d3, __builtin_fma(c[2], d2, __builtin_fma(c[1], d1, c[0] * d0)));
+    else return c[0] * d0 + c[1] * d1 + c[2] * d2 + c[3] * d3;
+}
+
 // D-: sum_k C_k (q[m+k] - q[m-1-k]) ; D+: sum_k C_k (q[m+1+k] - q[m-k])
 template <typename T>
 __device__ __forceinline__ T dm_q(const T* q, int m, const T* c) {
-    return c[0] * (q[m] - q[m - 1]) + c[1] * (q[m + 1] - q[m - 2]) + c[2] * (q[m + 2] - q[m - 3]) +
-           c[3] * (q[m + 3] - q[m - 4]);
+    return taps(c, q[m] - q[m - 1], q[m + 1] - q[m - 2], q[m + 2] - q[m - 3], q[m + 3] - q[m - 4]);
 }
 template <typename T>
 __device__ __forceinline__ T dp_q(const T* q, int m, const T* c) {
-    return c[0] * (q[m + 1] - q[m]) + c[1] * (q[m + 2] - q[m - 1]) + c[2] * (q[m + 3] - q[m - 2]) +
-           c[3] * (q[m + 4] - q[m - 3]);
+    return taps(c, q[m + 1] - q[m], q[m + 2] - q[m - 1], q[m + 3] - q[m - 2], q[m + 4] - q[m - 3]);
 }
 
 // Time bookkeeping of fine step k (0-based launch index) for a direction.
@@ -375,11 +392,11 @@ void k_step_fwd(const ShotDev<T>* __restrict__ shots, const TileDev* __restrict_
         const T d = ok ? damp_at(S, iz, ix) : T(1);
         T a0, a1, a2, a3, a4;
         if (!fs_top) {
-            a0 = d * o[0][r] + m[0][r] * (dx_sxx[r] + dz_sxz);
-            a1 = d * o[1][r] + m[1][r] * (dz_szz + dx_sxz[r]);
-            a2 = d * o[2][r] + (m[2][r] * dx_vx[r] + m[3][r] * dz_vz);
-            a3 = d * o[3][r] + (m[3][r] * dx_vx[r] + m[2][r] * dz_vz);
-            a4 = d * o[4][r] + m[4][r] * (dz_vx + dx_vz[r]);
+            a0 = mul2(d, o[0][r], m[0][r], dx_sxx[r] + dz_sxz);
+            a1 = mul2(d, o[1][r], m[1][r], dz_szz + dx_sxz[r]);
+            a2 = mac(mul2(m[2][r], dx_vx[r], m[3][r], dz_vz), d, o[2][r]);
+            a3 = mac(mul2(m[3][r], dx_vx[r], m[2][r], dz_vz), d, o[3][r]);
+            a4 = mul2(d, o[4][r], m[4][r], dz_vx + dx_vz[r]);
         } else {  // kernelsGpuElastic.cu:589-776: updated rows per component, surface modulus
             const bool on = iz == SURF, below = iz > SURF;
             a0 = d * o[0][r] + ((on || below) ? m[0][r] * (dx_sxx[r] + dz_sxz) : T(0));
@@ -425,11 +442,12 @@ void k_step_fwd(const ShotDev<T>* __restrict__ shots, const TileDev* __restrict_
                 T s;
                 if (MODE & F_INJ_COARSE) {  // kernelsGpuElastic.cu:172-189 with it2-1
                     const long b = long(row) * S.nts + st.its;
-                    s = tr[b] * S.filt[st.it2 - 1] + tr[b + 1] * S.filt[S.h + st.it2 - 1];
+                    s = mul2(tr[b], S.filt[st.it2 - 1], tr[b + 1], S.filt[S.h + st.it2 - 1]);
                 } else {             // pre-fine-sampled source at itw-1 = k (kernelsGpuElastic.cu:121-168)
                     s = tr[long(row) * S.ntw + k];
                 }
-                lds[comp][FAT + lx][FAT + lz] += damp_at(S, t.z0 + lz, t.x0 + lx) * s;
+                T& v = lds[comp][FAT + lx][FAT + lz];
+                v = mac(v, damp_at(S, t.z0 + lz, t.x0 + lx), s);
             }
             __syncthreads();
 #pragma unroll
@@ -445,8 +463,8 @@ void k_step_fwd(const ShotDev<T>* __restrict__ shots, const TileDev* __restrict_
                 const int comp = en.crow >> 24, row = en.crow & 0xffffff;
                 const T v = lds[comp][FAT + lx][FAT + lz];
                 T* tr = S.rec_tr[comp] + long(row) * S.nts + st.its;
-                tr[0] += v * fa;
-                tr[1] += v * fb;
+                tr[0] = mac(tr[0], v, fa);
+                tr[1] = mac(tr[1], v, fb);
             }
         }
     }

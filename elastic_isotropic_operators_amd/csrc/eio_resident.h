@@ -1,4 +1,5 @@
-// eio_resident.h -- time loops that keep a shot's whole state on the chip (k_res_fwd).
+// eio_resident.h -- time loops that keep a shot's whole state on the chip (k_res_fwd, k_res_adj), and the
+// imaging of many coarse samples that the Born passes trade with them through a ring (k_imaging_many).
 //
 // The launched kernels (eio_kernels.h, eio_step2.h) read two state levels and the media and
 // write one or two levels per launch: 50-80 B per cell-update through the caches, and one
@@ -146,30 +147,33 @@ __device__ __forceinline__ const LdsT<T>* lds_at(unsigned la, int elem) {
 // D- and D+ along z at row 4 of a window of 9
 template <typename T>
 __device__ __forceinline__ T dm_l(const LdsT<T>* q, const T* c) {
-    return c[0] * (q[4] - q[3]) + c[1] * (q[5] - q[2]) + c[2] * (q[6] - q[1]) + c[3] * (q[7] - q[0]);
+    return taps<T>(c, q[4] - q[3], q[5] - q[2], q[6] - q[1], q[7] - q[0]);
 }
 template <typename T>
 __device__ __forceinline__ T dp_l(const LdsT<T>* q, const T* c) {
-    return c[0] * (q[5] - q[4]) + c[1] * (q[6] - q[3]) + c[2] * (q[7] - q[2]) + c[3] * (q[8] - q[1]);
+    return taps<T>(c, q[5] - q[4], q[6] - q[3], q[7] - q[2], q[8] - q[1]);
 }
 
-// The updates' sums.  PAIR: rounded as the launched loop of the same calls rounds them
-// (k_step2_fwd's streamed stage, variant 12: d*o first for the velocities and, in the second step of
-// a pair, for sxz), so that an FP32 call gives the same bits in either form; else as k_step_fwd.
-template <typename T, bool PAIR>
-__device__ __forceinline__ T upd_velocity(T d, T o, T m, T s) {
-    if constexpr (PAIR) return __builtin_fmaf(m, s, d * o);
-    else return d * o + m * s;
+// The updates' sums, rounded as the launched loop of the same calls rounds them, so that a call gives
+// the same bits in either form: with fused operations spelled out, since which product the compiler fuses
+// changes with the code around it.  PAIR (FP32): as k_step2_fwd's streamed stage, variant 12 (d*o first for
+// the velocities and, in the second step of a pair, for sxz); else as k_step_fwd.
+template <typename T>
+__device__ __forceinline__ T fma_t(T a, T b, T c) {
+    if constexpr (sizeof(T) == 4) return __builtin_fmaf(a, b, c);
+    else return __builtin_fma(a, b, c);
 }
 template <typename T, bool PAIR>
+__device__ __forceinline__ T upd_velocity(T d, T o, T m, T s) {
+    return PAIR ? fma_t(m, s, d * o) : fma_t(d, o, m * s);
+}
+template <typename T>
 __device__ __forceinline__ T upd_normal(T d, T o, T mx, T vx, T mz, T vz) {
-    if constexpr (PAIR) return __builtin_fmaf(d, o, __builtin_fmaf(mx, vx, mz * vz));
-    else return d * o + (mx * vx + mz * vz);
+    return fma_t(d, o, fma_t(mx, vx, mz * vz));
 }
 template <typename T, bool PAIR>
 __device__ __forceinline__ T upd_shear(bool odd, T d, T o, T m, T s) {
-    if constexpr (PAIR) return odd ? __builtin_fmaf(m, s, d * o) : __builtin_fmaf(d, o, m * s);
-    else return d * o + m * s;
+    return PAIR && odd ? fma_t(m, s, d * o) : fma_t(d, o, m * s);
 }
 
 // The communication of one wave of a tile.
@@ -563,8 +567,8 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
             if (!FSURF || !fs_top) {
                 a0 = upd_velocity<T, PAIR>(d[r], o[0][r], mm[0], s0);
                 a1 = upd_velocity<T, PAIR>(d[r], o[1][r], mm[1], s1);
-                a2 = upd_normal<T, PAIR>(d[r], o[2][r], mm[2], vxx[r], mm[3], vzz);
-                a3 = upd_normal<T, PAIR>(d[r], o[3][r], mm[3], vxx[r], mm[2], vzz);
+                a2 = upd_normal<T>(d[r], o[2][r], mm[2], vxx[r], mm[3], vzz);
+                a3 = upd_normal<T>(d[r], o[3][r], mm[3], vxx[r], mm[2], vzz);
                 a4 = upd_shear<T, PAIR>(odd, d[r], o[4][r], mm[4], sh);
             } else {  // kernelsGpuElastic.cu:589-776, as in k_step_fwd
                 const bool on = iz == SURF, below = iz > SURF;
@@ -635,7 +639,7 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
         if (INJ && sb0 < se0) {
             const T fa = filt[it2], fb = filt[h + it2];
             if (srow >= 0) {
-                Lf[scell] += sd * ((MODE & F_INJ_FINE) ? sa : sa * fa + sb * fb);
+                Lf[scell] = mac(T(Lf[scell]), sd, (MODE & F_INJ_FINE) ? sa : mul2(sa, fa, sb, fb));
                 if (MODE & F_INJ_FINE) {
                     sa = source(srow, k + 1, 0);
                 } else if (it2 + 1 == sub) {
@@ -646,8 +650,9 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
             for (int e = sb0 + 64 + lane; e < se0; e += 64) {
                 const Entry en = ents[e];
                 const int lz = en.lcell & 255, lx = en.lcell >> 8;
-                const T s = (MODE & F_INJ_FINE) ? source(en.crow, k, 0) : source(en.crow, 0, its) * fa + source(en.crow, 0, its + 1) * fb;
-                L[en.crow >> 24][FAT + lx][FAT + lz] += damp_at(S, z0 + lz, x0 + lx) * s;
+                const T s = (MODE & F_INJ_FINE) ? source(en.crow, k, 0) : mul2(source(en.crow, 0, its), fa, source(en.crow, 0, its + 1), fb);
+                T& v = L[en.crow >> 24][FAT + lx][FAT + lz];
+                v = mac(v, damp_at(S, z0 + lz, x0 + lx), s);
             }
             __builtin_amdgcn_wave_barrier();
         }
@@ -657,8 +662,8 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
             const T fa = filt[j2], fb = filt[h + j2];
             if (rrow >= 0) {
                 const T v = Lf[rcell];
-                ra += v * fa;
-                rb += v * fb;
+                ra = mac(ra, v, fa);
+                rb = mac(rb, v, fb);
                 if (j2 == sub) {
                     S.rec_tr[rrow >> 24][long(rrow & 0xffffff) * nts + js] = ra;
                     ra = rb;
@@ -669,8 +674,8 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
                 const Entry en = ents[e];
                 const T v = L[en.crow >> 24][FAT + (en.lcell >> 8)][FAT + (en.lcell & 255)];
                 T* tr = S.rec_tr[en.crow >> 24] + long(en.crow & 0xffffff) * nts + js;
-                tr[0] += v * fa;
-                tr[1] += v * fb;
+                tr[0] = mac(tr[0], v, fa);
+                tr[1] = mac(tr[1], v, fb);
             }
             __builtin_amdgcn_wave_barrier();
         }
