@@ -3,7 +3,7 @@
 Candidates are every single-step variant (tile 64 x WX*R, R x-cells per lane, requested
 waves per SIMD), every two-step variant (owned tile 56 x WX*R2, two fine steps per
 launch), every three-step variant and the library's own choice, which runs a batch that fits the
-chip as resident loops (64 shots of 305-687 x 597-1887 cells: 127 GCell/s against 89 of the
+chip as resident loops (64 shots of 305-687 x 597-1887 cells: 153 GCell/s against 89 of the
 fastest launched variant).  Each candidate runs the caller's own batch for a bounded number of fine steps
 (``eio_ctx_set_step_limit``) and is timed with the HIP events of the context
 (``eio_ctx_last_timing``); the fastest per fine step wins and is set on the context.
