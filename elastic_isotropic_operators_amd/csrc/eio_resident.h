@@ -328,8 +328,10 @@ struct ResComm {
 // Fine steps [k0, k1) of the forward loop (a shot stops at its own last step).  MODE: the flags
 // of k_step_fwd (F_INJ_COARSE, F_INJ_FINE, F_REC, F_DEC, F_SS: secondary sources from the ring of
 // S.sscap coarse samples at S.ss[0], sample j at j % sscap); FSURF: shots with a free surface.
-// k0 is a multiple of the shots' sub-sampling.  The state starts from the levels A (older) and
-// B (current), or from rest with from_rest, and goes back there with save.
+// k0 is a multiple of the shots' sub-sampling.  The state starts from the levels A and B, or from rest
+// with from_rest, and goes back there with save, as k_step_fwd finds and leaves it: at an even step A is the
+// older level and B the current one, at an odd step (odd sub-samplings) the other way round, so that a
+// checkpoint of either form serves both.
 template <typename T, int R, int MODE, bool FSURF>
 __global__ __launch_bounds__(64 * RES_WX) __attribute__((amdgpu_waves_per_eu(RES_WX / 4, RES_WX / 4)))
 void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__ tiles,
@@ -385,7 +387,7 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
 #pragma unroll
     for (int r = 0; r < R; ++r) d[r] = zok && r < ncol ? damp_at(S, iz, ix0 + r) : T(1);
     {
-        const rsrc_t rold = make_rsrc(S.A, 5 * fbytes), rcur = make_rsrc(S.B, 5 * fbytes);
+        const rsrc_t rold = make_rsrc((k0 & 1) ? S.B : S.A, 5 * fbytes), rcur = make_rsrc((k0 & 1) ? S.A : S.B, 5 * fbytes);
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -724,7 +726,7 @@ void k_res_fwd(const ShotDev<T>* __restrict__ shots, const ResTile* __restrict__
             }
     }
     if (save) {
-        const rsrc_t rold = make_rsrc(S.A, 5 * fbytes), rcur = make_rsrc(S.B, 5 * fbytes);
+        const rsrc_t rold = make_rsrc((kend & 1) ? S.B : S.A, 5 * fbytes), rcur = make_rsrc((kend & 1) ? S.A : S.B, 5 * fbytes);
 #pragma unroll
         for (int r = 0; r < R; ++r)
             if (zok && r < ncol) {
