@@ -103,6 +103,7 @@ def lib():
             ("eio_ctx_set_shot_group_bytes", [vp, ctypes.c_longlong]),
             ("eio_ctx_set_shot_group_streams", [vp, ctypes.c_int]),
             ("eio_ctx_last_shot_groups", [vp, ctypes.POINTER(ctypes.c_int)]),
+            ("eio_ctx_resident_info", [vp] + [ctypes.POINTER(ctypes.c_longlong)] * 3 + [ctypes.POINTER(ctypes.c_int)]),
             ("eio_host_alloc", [ctypes.c_ulonglong, ctypes.POINTER(vp)]),
             ("eio_host_free", [vp]),
             ("eio_ctx_set_persistent", [vp, ctypes.c_int, ctypes.c_int]),
@@ -129,7 +130,7 @@ EXPORTED = ("eio_last_error", "eio_ctx_create", "eio_ctx_destroy", "eio_ctx_set_
             "eio_nl_step_states", "eio_ctx_release_workspace", "eio_ctx_num_adjoint_time_block_variants",
             "eio_ctx_adjoint_time_block_info", "eio_ctx_set_adjoint_time_block",
             "eio_ctx_set_shot_group_bytes", "eio_ctx_set_shot_group_streams", "eio_ctx_last_shot_groups",
-            "eio_host_alloc", "eio_host_free")
+            "eio_ctx_resident_info", "eio_host_alloc", "eio_host_free")
 
 
 def check(rc):
@@ -268,6 +269,13 @@ class Context:
         n = ctypes.c_int()
         check(lib().eio_ctx_last_shot_groups(self.h, ctypes.byref(n)))
         return n.value
+
+    def resident_info(self):
+        """Resident loops so far: (cooperative launches, passes that gave up a wait, launches refused, HIP
+        error of the last refusal)."""
+        a, b, r, e = ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_longlong(), ctypes.c_int()
+        check(lib().eio_ctx_resident_info(self.h, ctypes.byref(a), ctypes.byref(b), ctypes.byref(r), ctypes.byref(e)))
+        return a.value, b.value, r.value, e.value
 
     @staticmethod
     def time_block_variants():

@@ -219,7 +219,11 @@ struct Ctx {
     hipEvent_t fork = nullptr, join = nullptr;
     int persistent = 0;  // two-step NL forward in one persistent launch: 0 off, 1 on, 2 when it fits
     int spin_limit = 1 << 20;  // polls per neighbour wait of the persistent launch before it aborts
-    bool resident = true;      // false while a call is repeated with the launched kernels
+    bool resident = true;      // this call may run resident loops (ResCall; false while it is repeated launched)
+    long long res_launches = 0, res_given_up = 0, res_refused = 0;   // launches; passes that gave up; refusals
+    int res_error = 0;         // HIP error of the last refusal
+    bool res_failed = false;   // a resident pass of this call gave up or was refused
+    int res_skip = 0, res_backoff = 0;   // calls left that do not try resident loops, and how many after the last failure
     int ncu = 0;               // compute units of the device
     std::map<int, FwiStore> fwi;
     int next_fwi = 1;
@@ -1564,6 +1568,14 @@ void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp, const std::strin
     fill0<int>(c, rp.abort_flag, 1);
 }
 
+// The errors of a cooperative launch that a device which cannot take it now returns: one process at a time
+// holds its cooperative queue (hipErrorIllegalState to the others), a full device has no memory for the
+// queue, a device may have none.  Every other error is raised: a launch that does not fit the device, or
+// what earlier work left, is a fault to be seen and the launched kernels would not mend it.
+inline bool res_refusal(hipError_t e) {
+    return e == hipErrorIllegalState || e == hipErrorOutOfMemory || e == hipErrorNotSupported;
+}
+
 // One cooperative launch of a group, over kernels k_res_*<T, R, ..> by the group's R (at most
 // RMAX): `pick(integral_constant R)` names the kernel, `extra` its arguments after the tile count.
 template <typename T, int RMAX, typename Pick, typename... A>
@@ -1593,13 +1605,17 @@ void res_launch(Run<T>& run, const ResPlan& rp, const ResGroup& g, const eio::Sh
     pick(std::integral_constant<int, 5>{});
     pick(std::integral_constant<int, 6>{});
     const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(nt), dim3(64 * RES_WX), args, 0, c->stream);
-    if (e != hipSuccess) {
-        // refused (one process at a time holds a device's cooperative queue): the context keeps to the
-        // launched kernels from here on, this call included
-        (void)hipGetLastError();
-        c->resident = false;
-        rp.refused = true;
+    if (e == hipSuccess) {
+        ++c->res_launches;
+        return;
     }
+    if (!res_refusal(e)) throw EioError{EIO_ERR_RUNTIME, std::string("hipLaunchCooperativeKernel: ") + hipGetErrorString(e)};
+    (void)hipGetLastError();
+    ++c->res_refused;
+    c->res_error = int(e);
+    c->res_failed = true;
+    c->resident = false;   // the rest of this call runs launched
+    rp.refused = true;
 }
 
 // Fine steps [k0, k1) of a group's forward loop.  `dsh` replaces the run's shot table.
@@ -1625,12 +1641,35 @@ void res_launch_adj(Run<T>& run, const ResPlan& rp, const ResGroup& g, int k0, i
 // Whether the resident launches of this call were refused or gave up a wait (the call then repeats
 // launched).
 inline bool res_aborted(Ctx* c, const ResPlan& rp) {
-    if (rp.refused) return true;
     int aborted = 0;
     EIO_CHECK_HIP(hipMemcpyAsync(&aborted, rp.abort_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     EIO_CHECK_HIP(hipStreamSynchronize(c->stream));
-    return aborted != 0;
+    if (aborted) {
+        ++c->res_given_up;
+        c->res_failed = true;
+    }
+    return rp.refused || aborted;
 }
+
+// One call of an entry point that may run resident loops.  After a call that gave up a wait or was refused
+// a launch, the next 1, 3, 7, .. RES_BACKOFF calls do not try (a wait of the default limit is 2^20 polls
+// of memory before it is given up; a queue that another process holds may stay held); a call that runs
+// resident to its end resets the count.
+constexpr int RES_BACKOFF = 63;
+struct ResCall {
+    Ctx* c;
+    long long before;
+    explicit ResCall(Ctx* c_) : c(c_), before(c_->res_launches) {
+        c->res_failed = false;
+        c->resident = c->res_skip == 0;
+        if (c->res_skip > 0) --c->res_skip;
+    }
+    ~ResCall() {
+        if (c->res_failed) c->res_skip = c->res_backoff = std::min(2 * c->res_backoff + 1, RES_BACKOFF);
+        else if (c->res_launches > before) c->res_backoff = 0;
+        c->resident = true;
+    }
+};
 
 // While a call is repeated with the launched kernels.
 struct ResidentOff {
@@ -2784,6 +2823,16 @@ int eio_ctx_last_shot_groups(eio_ctx* ctx, int* groups) {
     });
 }
 
+int eio_ctx_resident_info(eio_ctx* ctx, long long* launches, long long* given_up, long long* refused, int* last_error) {
+    return guarded([&]() {
+        Ctx* c = as_ctx(ctx);
+        if (launches) *launches = c->res_launches;
+        if (given_up) *given_up = c->res_given_up;
+        if (refused) *refused = c->res_refused;
+        if (last_error) *last_error = c->res_error;
+    });
+}
+
 int eio_ctx_time_block_info(int variant, int* R2, int* WX, int* occ) {
     return guarded([&]() {
         if (variant < 0 || variant >= N_F32_VARIANTS2) fail("two-step variant out of range");
@@ -2920,6 +2969,7 @@ int eio_nl_forward(eio_ctx* ctx, int nshot, const eio_shot* shots, int flags) {
     return guarded([&]() {
         Ctx* c = as_ctx(ctx);
         DeviceGuard dg(c->device);
+        ResCall rc(c);
         if (c->prec == 4) nl_forward<float>(c, nshot, shots, flags);
         else nl_forward<double>(c, nshot, shots, flags);
     });
@@ -2987,6 +3037,7 @@ int eio_nl_adjoint(eio_ctx* ctx, int nshot, const eio_shot* shots, int flags) {
     return guarded([&]() {
         Ctx* c = as_ctx(ctx);
         DeviceGuard dg(c->device);
+        ResCall rc(c);
         if (c->prec == 4) nl_adjoint<float>(c, nshot, shots, flags);
         else nl_adjoint<double>(c, nshot, shots, flags);
     });
@@ -2997,6 +3048,7 @@ int eio_born_forward(eio_ctx* ctx, int nshot, const eio_shot* shots, const void*
     return guarded([&]() {
         Ctx* c = as_ctx(ctx);
         DeviceGuard dg(c->device);
+        ResCall rc(c);
         if (nshot <= 0 || !shots) fail("no shots");
         if (c->prec == 4) born_forward<float>(c, nshot, shots, dm, flags);
         else born_forward<double>(c, nshot, shots, dm, flags);
@@ -3007,6 +3059,7 @@ int eio_born_adjoint(eio_ctx* ctx, int nshot, const eio_shot* shots, void* const
     return guarded([&]() {
         Ctx* c = as_ctx(ctx);
         DeviceGuard dg(c->device);
+        ResCall rc(c);
         if (nshot <= 0 || !shots) fail("no shots");
         if (c->prec == 4) born_adjoint<float>(c, nshot, shots, dm, flags);
         else born_adjoint<double>(c, nshot, shots, dm, flags);
@@ -3019,6 +3072,7 @@ int eio_fwi_forward(eio_ctx* ctx, int nshot, const eio_shot* shots, int flags, i
         if (!handle) fail("handle is NULL");
         if (segment < 0) fail("segment must be >= 0");
         DeviceGuard dg(c->device);
+        ResCall rc(c);
         *handle = (c->prec == 4) ? fwi_forward<float>(c, nshot, shots, flags, segment)
                                  : fwi_forward<double>(c, nshot, shots, flags, segment);
     });
@@ -3028,6 +3082,7 @@ int eio_fwi_gradient(eio_ctx* ctx, int handle, int nshot, const eio_shot* shots,
     return guarded([&]() {
         Ctx* c = as_ctx(ctx);
         DeviceGuard dg(c->device);
+        ResCall rc(c);
         if (c->prec == 4) fwi_gradient<float>(c, handle, nshot, shots, dm, flags);
         else fwi_gradient<double>(c, handle, nshot, shots, dm, flags);
     });

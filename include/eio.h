@@ -115,7 +115,9 @@ int eio_ctx_set_variant(eio_ctx* ctx, int variant);
  * scattered and receiver passes), the state in LDS and registers.  eio_ctx_last_timing then counts these
  * launches for the NL forward, eio_ctx_last_shot_groups the groups.  Graphs, the persistent mode, explicit
  * variants, saved wavefields, snapshots, learned boundaries and the no-allocation call keep to launched
- * steps, and so does a context whose device refuses a cooperative launch (another process holds it).
+ * steps.  A call whose device refuses a cooperative launch (one process at a time holds a device's
+ * cooperative queue) or that gives up a wait runs launched instead, and the context's next 1, 3, 7, .. 63
+ * calls, one count per failure in a row, do not try (eio_ctx_resident_info).
  * It applies to the NL forward (without
  * saved wavefield, free surface or learned boundary), the whole-record FWI forward and the
  * Born source and scattered passes.  No counterpart in the reference. */
@@ -184,6 +186,12 @@ int eio_ctx_set_shot_group_bytes(eio_ctx* ctx, long long bytes);
 int eio_ctx_set_shot_group_streams(eio_ctx* ctx, int streams);
 /* Number of shot groups of the context's last NL forward call.  No counterpart in the reference. */
 int eio_ctx_last_shot_groups(eio_ctx* ctx, int* groups);
+
+/* Resident loops (eio_ctx_set_time_block) of the context since its creation: cooperative launches made,
+ * passes that gave up a wait, launches that were refused, and the HIP error of the last refusal (0: none).
+ * A call that left `launches` where it was ran launched.  Pointers may be NULL.  No counterpart in the
+ * reference. */
+int eio_ctx_resident_info(eio_ctx* ctx, long long* launches, long long* given_up, long long* refused, int* last_error);
 
 /* The grid checks of eio_model_add, on the host only (no device, no context): sizes, sampling,
  * sponge width (the reference's messages, fdParamElastic.cpp:29-32,

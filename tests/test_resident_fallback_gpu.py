@@ -2,17 +2,58 @@
 that ask for launched steps: the launched kernels take over with the same answers.
 Bars: those of the launched kernels, FP32 1e-5 and FP64 1e-11 relative L2 (gradients twice that and ten
 times that, as sums over many products)."""
+import ctypes
+import importlib.util
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
 import oracle as O
+from elastic_isotropic_operators_amd import _capi
 
 from helpers import GRID_OF_COMP, random_traces, rel_l2
-from test_resident_gpu import _check, _ctx, _model, _positions
+from test_resident_gpu import _check, _ctx, _forward_case, _model, _positions
 
 pytestmark = pytest.mark.gpu
 
 GRAD_TOL = {np.float32: 2e-5, np.float64: 1e-10}
+ILLEGAL_STATE, LAUNCH_FAILURE = 401, 719   # hipErrorIllegalState (a held queue), hipErrorLaunchFailure
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    """(shim, the C ABI's binding on a copy of the library that calls the HIP runtime through it)."""
+    d = tmp_path_factory.mktemp("shim")
+    so, lib = str(d / "hip_shim.so"), str(d / "libeio_copy.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", so, os.path.join(os.path.dirname(__file__), "hip_shim.c"),
+                    "-L/opt/rocm/lib", "-Wl,--no-as-needed", "-lamdhip64"], check=True)
+    shutil.copy(_capi.LIB_PATH, lib)
+    s = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)
+    s.shim_memory.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+    spec = importlib.util.spec_from_file_location("eio_capi_shimmed", _capi.__file__)
+    capi = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(capi)
+    capi.LIB_PATH = lib
+    capi.lib()
+    return s, capi
+
+
+@pytest.fixture
+def shimmed(shim):
+    yield shim
+    shim[0].shim_launches(0, 0, 0)
+    shim[0].shim_memory(~0 & (2 ** 64 - 1), 0)
+
+
+def _shim_ctx(capi, dtype):
+    ctx = capi.Context(0, dtype)
+    if dtype == np.float32:
+        ctx.set_time_block(2, capi.VARIANT_AUTO)
+        ctx.set_adjoint_time_block(2, capi.VARIANT_AUTO)
+    return ctx
 
 
 @pytest.mark.parametrize("change", ["given_up", "graph"])
@@ -46,4 +87,73 @@ def test_launched_recompute_from_resident_checkpoints(dtype, sub, change):
         ctx.fwi_gradient(h, [shot], dm)
         assert rel_l2(dm, ref_dm) < GRAD_TOL[dtype], rel_l2(dm, ref_dm)
     ctx.fwi_release(h)
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_refused_launch_is_tried_again(shimmed, dtype):
+    """A refused cooperative launch costs its call, and a growing count of the calls after it, the resident
+    form, not the context's life; each call's data are right."""
+    shim, capi = shimmed
+    ctx = _shim_ctx(capi, dtype)
+    mid, g, med = _model(ctx, 139, 90, 101, 2, 41)
+    rng = np.random.default_rng(42)
+    shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, dtype, 10, 20)
+
+    def forms(n):
+        out = ""
+        for _ in range(n):
+            for r in rec:
+                r[...] = 7
+            before = ctx.resident_info()[0]
+            ctx.nl_forward([shot])
+            resident = ctx.resident_info()[0] > before
+            assert (ctx.last_timing()[1] == 1) == resident
+            _check(rec, ref, dtype)
+            out += "RL"[not resident]
+        return out
+
+    assert forms(2) == "RR"
+    shim.shim_launches(ILLEGAL_STATE, 1, 0)
+    assert forms(4) == "LLRR"
+    assert ctx.resident_info()[1:] == (0, 1, ILLEGAL_STATE)
+    shim.shim_launches(ILLEGAL_STATE, 2, 0)          # and the next try again: 1, then 3 calls without one
+    assert forms(8) == "LLLLLLRR"
+    assert ctx.resident_info()[1:] == (0, 3, ILLEGAL_STATE)
+    shim.shim_launches(ILLEGAL_STATE, 1, 0)          # a call that ran resident has reset the count
+    assert forms(3) == "LLR"
+    ctx.close()
+
+
+def test_other_launch_errors_are_raised(shimmed):
+    """An error that is no refusal reaches the caller; the context runs resident afterwards."""
+    shim, capi = shimmed
+    ctx = _shim_ctx(capi, np.float32)
+    mid, g, med = _model(ctx, 139, 90, 101, 2, 43)
+    rng = np.random.default_rng(44)
+    shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, np.float32, 10, 20)
+    shim.shim_launches(LAUNCH_FAILURE, 1, 0)
+    with pytest.raises(capi.EioError, match="hipLaunchCooperativeKernel"):
+        ctx.nl_forward([shot])
+    assert ctx.resident_info()[:3] == (0, 0, 0)
+    ctx.nl_forward([shot])
+    assert ctx.resident_info()[0] == 1
+    _check(rec, ref, np.float32)
+    ctx.close()
+
+
+def test_given_up_wait_is_not_paid_on_every_call():
+    """After a call that gave up a wait, the next one does not try; then one in four, and so on."""
+    ctx = _ctx(np.float32)
+    ctx.set_persistent(0, 1)
+    mid, g, med = _model(ctx, 281, 301, 51, 2, 45)
+    rng = np.random.default_rng(46)
+    shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, np.float32, 10, 20)
+    tries = []
+    for _ in range(8):
+        before = ctx.resident_info()[1]
+        ctx.nl_forward([shot])
+        tries.append(ctx.resident_info()[1] - before)
+        _check(rec, ref, np.float32)
+    assert tries == [1, 0, 1, 0, 0, 0, 1, 0]
     ctx.close()
