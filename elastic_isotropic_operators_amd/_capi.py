@@ -213,6 +213,8 @@ class Context:
         check(lib().eio_ctx_set_stream(self.h, ctypes.c_void_p(stream_handle)))
 
     def set_variant(self, v):
+        """One-step kernel variant, or VARIANT_AUTO (the default): passes launched one step at a time
+        keep to a variant that is set, and run resident where that is faster without one."""
         check(lib().eio_ctx_set_variant(self.h, int(v)))
 
     @staticmethod

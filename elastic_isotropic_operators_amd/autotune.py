@@ -64,6 +64,7 @@ def _apply(ctx, cand):
         ctx.set_time_block(1, 0)
         ctx.set_variant(v)
     else:
+        ctx.set_variant(_capi.VARIANT_AUTO)
         ctx.set_time_block(tb, v)
 
 

@@ -92,6 +92,7 @@ struct Variant {
 };
 constexpr Variant F32_VARIANTS[] = {{4, 4, 2}, {2, 8, 4}, {2, 4, 4}, {4, 8, 2}, {8, 4, 1}, {2, 8, 2}};
 constexpr int N_F32_VARIANTS = int(sizeof(F32_VARIANTS) / sizeof(F32_VARIANTS[0]));
+constexpr int F32_VARIANT_AUTO = 1;   // the fastest on the 64-shot layered batch
 constexpr Variant F64_VARIANT = {2, 4, 1};
 
 // Two-step (temporally blocked) NL forward variants: owned tile = 56 x WX*R2, WX waves, OCC
@@ -205,7 +206,8 @@ struct Ctx {
     std::map<unsigned long long, GraphEntry> graphs;
     unsigned long long graph_clock = 0;
     long long graph_builds = 0, graph_launches = 0, graph_node_updates = 0;
-    int variant = 1;  // best measured FP32 variant on the 64-shot layered batch
+    int variant = F32_VARIANT_AUTO;
+    bool variant_set = false;  // chosen by eio_ctx_set_variant
     int time_block = 1;  // fine steps per launch of the FP32 NL forward (1, 2 or 3)
     int variant3 = 0;    // three-step kernel variant, or EIO_VARIANT_AUTO
     int variant2 = 0;    // two-step kernel variant, or EIO_VARIANT_AUTO (chosen per call)
@@ -1679,11 +1681,25 @@ struct ResidentOff {
     ~ResidentOff() { c->resident = was; }
 };
 
-// A context that leaves the launch form to the library, outside graphs, the persistent launch
-// and the no-allocation call.
+// Whether the launched form of a pass takes one step per launch, with the context's one-step tile: every
+// FP64 pass, and in FP32 the free surface, an NL adjoint of an odd step count, and Born and FWI passes with an
+// odd sub-sampling.
 template <typename T>
-bool res_allowed(Ctx* c, ResKind kind) {
+bool one_step_pass(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) {
+    if (sizeof(T) == 8) return true;
+    if (kind == ResKind::ADJ) return (c->step_limit > 0 ? std::min(plan.nsteps[0], c->step_limit) : plan.nsteps[0]) % 2 != 0;
+    if (kind != ResKind::NL) return get_model(c, shots[0].model).g.sub_fd % 2 != 0;
+    for (int i : plan.order)
+        if (get_model(c, shots[i].model).g.surface) return true;
+    return false;
+}
+
+// A context that leaves the launch form to the library, outside graphs, the persistent launch
+// and the no-allocation call: no explicit variant of the launched form that the pass would take.
+template <typename T>
+bool res_allowed(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) {
     if (!c->resident || c->use_graph || c->persistent || c->bump) return false;
+    if (c->variant_set && one_step_pass<T>(c, plan, shots, kind)) return false;
     if (sizeof(T) == 8) return true;
     if (kind == ResKind::ADJ || kind == ResKind::BADJ) return c->adj_time_block == 2 && c->variant2a == EIO_VARIANT_AUTO;
     return c->time_block == 2 && c->variant2 == EIO_VARIANT_AUTO && c->group_bytes == EIO_GROUP_AUTO;
@@ -1705,7 +1721,7 @@ bool res_allowed(Ctx* c, ResKind kind) {
 constexpr double RES_SEGMENT_US = 100.0;
 template <typename T>
 std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
-    if (!res_allowed<T>(c, kind)) return {};
+    if (!res_allowed<T>(c, plan, shots, kind)) return {};
     std::vector<ResGroup> groups = res_groups<T>(c, plan, shots, kind);
     double res = 0.0, work = 0.0;
     int longest = 0;
@@ -2770,8 +2786,10 @@ int eio_ctx_graph_info(eio_ctx* ctx, long long* builds, long long* launches, lon
 
 int eio_ctx_set_variant(eio_ctx* ctx, int variant) {
     return guarded([&]() {
-        if (variant < 0 || variant >= N_F32_VARIANTS) fail("variant out of range");
-        as_ctx(ctx)->variant = variant;
+        if (variant != EIO_VARIANT_AUTO && (variant < 0 || variant >= N_F32_VARIANTS)) fail("variant out of range");
+        Ctx* c = as_ctx(ctx);
+        c->variant_set = variant != EIO_VARIANT_AUTO;
+        c->variant = c->variant_set ? variant : F32_VARIANT_AUTO;
     });
 }
 

@@ -98,8 +98,12 @@ int eio_ctx_set_graph(eio_ctx* ctx, int use_graph);
 int eio_ctx_graph_info(eio_ctx* ctx, long long* builds, long long* launches, long long* node_updates);
 
 /* FP32 step-kernel variant (tile of 64 x WX*R cells, WX waves per workgroup, R x-cells per
- * lane, requested occupancy) used by the next calls.  FP64 contexts ignore it.  No counterpart
- * in the reference (fixed 16x16 blocks, varDeclare.h:5). */
+ * lane, requested occupancy) used by the next calls, or EIO_VARIANT_AUTO (the default): variant 1, and
+ * resident loops (eio_ctx_set_time_block) where they are faster.  With a variant, the passes whose launched
+ * form takes one step per launch (a free surface; an NL adjoint of an odd step count, Born and FWI passes
+ * with an odd sub_fd) keep to it; FP64 contexts have one tile, and a variant keeps all their passes launched.
+ * No counterpart in the reference (fixed 16x16 blocks, varDeclare.h:5). */
+#define EIO_VARIANT_AUTO (-1)
 int eio_ctx_num_variants(void);
 int eio_ctx_variant_info(int variant, int* R, int* WX, int* occ);
 int eio_ctx_set_variant(eio_ctx* ctx, int variant);
@@ -114,14 +118,13 @@ int eio_ctx_set_variant(eio_ctx* ctx, int variant);
  * cooperative launch for the whole loop of a group of shots (32 coarse intervals at a time in the Born
  * scattered and receiver passes), the state in LDS and registers.  eio_ctx_last_timing then counts these
  * launches for the NL forward, eio_ctx_last_shot_groups the groups.  Graphs, the persistent mode, explicit
- * variants, saved wavefields, snapshots, learned boundaries and the no-allocation call keep to launched
+ * variants of the launched form a pass would take, saved wavefields, snapshots, learned boundaries and the no-allocation call keep to launched
  * steps.  A call whose device refuses a cooperative launch (one process at a time holds a device's
  * cooperative queue) or that gives up a wait runs launched instead, and the context's next 1, 3, 7, .. 63
  * calls, one count per failure in a row, do not try (eio_ctx_resident_info).
  * It applies to the NL forward (without
  * saved wavefield, free surface or learned boundary), the whole-record FWI forward and the
  * Born source and scattered passes.  No counterpart in the reference. */
-#define EIO_VARIANT_AUTO (-1)
 int eio_ctx_num_time_block_variants(void);
 int eio_ctx_time_block_info(int variant, int* R2, int* WX, int* occ);
 int eio_ctx_set_time_block(eio_ctx* ctx, int steps, int variant);

@@ -157,3 +157,61 @@ def test_given_up_wait_is_not_paid_on_every_call():
         _check(rec, ref, np.float32)
     assert tries == [1, 0, 1, 0, 0, 0, 1, 0]
     ctx.close()
+
+
+def _passes(ctx, mid, g, dtype):
+    """One call of each entry point on one shot: which of them ran resident."""
+    rng = np.random.default_rng(52)
+    spos, rpos = _positions(rng, g, 5), _positions(rng, g, 5)
+    nt = {"src": np.ones((1, g.nts), dtype), "fine": np.ones((1, (g.nts - 1) * g.sub + 1), dtype)}
+
+    def traces(pos, key):
+        return [np.repeat(nt[key], pos[GRID_OF_COMP[k]].size, 0) for k in range(5)]
+
+    src, fine, dat = traces(spos, "src"), traces(spos, "fine"), traces(rpos, "src")
+    dm = np.ones((5, g.nx, g.nz), dtype)
+
+    def gradient(s):
+        h = ctx.fwi_forward(s(src), g.nts - 1)
+        ctx.fwi_gradient(h, s(src), dm)
+        ctx.fwi_release(h)
+
+    calls = {"nl_forward": lambda s: ctx.nl_forward(s(src)), "nl_adjoint": lambda s: ctx.nl_adjoint(s(src))}
+    if not g.surface:
+        calls.update(born_forward=lambda s: ctx.born_forward(s(fine), dm), born_adjoint=lambda s: ctx.born_adjoint(s(fine), dm),
+                     fwi=gradient)
+    out, keep = {}, []
+
+    def shot(tr):
+        sh, k = ctx.make_shot(mid, spos, rpos, tr, dat)
+        keep.append(k)
+        return [sh]
+
+    for name, call in calls.items():
+        before = ctx.resident_info()[0]
+        call(shot)
+        out[name] = ctx.resident_info()[0] > before
+    return out
+
+
+@pytest.mark.parametrize("dtype,sub,surface", [(np.float32, 2, 1), (np.float32, 3, 0), (np.float64, 2, 0), (np.float64, 2, 1),
+                                               (np.float32, 2, 0)])
+def test_explicit_variant_keeps_launched_steps(dtype, sub, surface):
+    """A one-step variant that the caller sets is run where a pass would be launched one step at a time;
+    FP32 passes that take two steps a launch have variants of their own, which stay automatic here."""
+    ctx = _ctx(dtype)
+    nts = 102 if sub == 3 else 201           # 303 fine steps are an odd count for the NL adjoint
+    mid, g, med = _model(ctx, 139, 90, nts, sub, 51, surface=surface)
+    auto = _passes(ctx, mid, g, dtype)
+    assert auto["nl_forward"] and (surface or all(auto.values())), auto
+    ctx.set_variant(3)
+    fixed = _passes(ctx, mid, g, dtype)
+    if dtype == np.float32 and sub == 2 and not surface:
+        assert fixed == auto
+    elif dtype == np.float32 and sub == 3:
+        assert fixed == {k: k == "nl_forward" for k in fixed}, fixed
+    else:
+        assert not any(fixed.values()), fixed
+    ctx.set_variant(_capi.VARIANT_AUTO)
+    assert _passes(ctx, mid, g, dtype) == auto
+    ctx.close()
