@@ -230,7 +230,30 @@ struct Ctx {
     std::map<int, FwiStore> fwi;
     int next_fwi = 1;
     bool fwi_ws_busy = false;  // a store holds the workspace's "fwi_ring" / "fwi_ck" buffers
+    bool ring_busy = false;    // a call uses the workspace's "res_ring" buffer (ResRing)
 };
+
+// Gives the ring of the resident Born passes back (the streams are idle); the next call that wants it
+// allocates it again.
+void ring_free(Ctx* c) {
+    auto it = c->ws.find("res_ring");
+    if (it == c->ws.end() || c->ring_busy) return;
+    if (it->second.p) (void)hipFree(it->second.p);
+    c->ws.erase(it);
+}
+
+// Device memory for the context; where there is none left, the ring is given back first: no call fails for a
+// buffer that only makes another one faster.
+hipError_t device_malloc(Ctx* c, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && !c->ring_busy && c->ws.count("res_ring")) {
+        (void)hipGetLastError();
+        EIO_CHECK_HIP(hipStreamSynchronize(c->stream));
+        ring_free(c);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
 
 void* ws_get(Ctx* c, const std::string& name, size_t bytes) {
     if (c->bump) {  // no-allocation call: 256-byte aligned pieces of the scratch array
@@ -250,10 +273,34 @@ void* ws_get(Ctx* c, const std::string& name, size_t bytes) {
             b.p = nullptr;
             b.bytes = 0;
         }
-        EIO_CHECK_HIP(hipMalloc(&b.p, bytes));
+        void* p = nullptr;
+        EIO_CHECK_HIP(device_malloc(c, &p, bytes));
+        b.p = p;
         b.bytes = bytes;
     }
     return b.p;
+}
+
+// As ws_get, but nullptr where there is no memory, for buffers that a call can do without.
+void* ws_try(Ctx* c, const std::string& name, size_t bytes) {
+    DevBuf& b = c->ws[name];
+    if (b.bytes >= bytes) return b.p;
+    if (b.p) {
+        EIO_CHECK_HIP(hipStreamSynchronize(c->stream));
+        EIO_CHECK_HIP(hipFree(b.p));
+        b = DevBuf{};
+    }
+    void* p = nullptr;
+    const hipError_t e = device_malloc(c, &p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    EIO_CHECK_HIP(e);
+    DevBuf& made = c->ws[name];   // device_malloc may have given "res_ring" back
+    made.p = p;
+    made.bytes = bytes;
+    return p;
 }
 
 struct DeviceGuard {
@@ -371,9 +418,9 @@ int model_add(Ctx* c, const eio_grid* g, const void* const media[5], int flags) 
         const double arg = M_PI / double(g->minPad) * double(g->minPad - j);
         damp[j] = T(g->alphaCos + (1.0 - g->alphaCos) * std::cos(arg));
     }
-    EIO_CHECK_HIP(hipMalloc(&m.med, size_t(5) * m.n * sizeof(T)));
-    EIO_CHECK_HIP(hipMalloc(&m.damp, damp.size() * sizeof(T)));
-    EIO_CHECK_HIP(hipMalloc(&m.filt, filt.size() * sizeof(T)));
+    EIO_CHECK_HIP(device_malloc(c, &m.med, size_t(5) * m.n * sizeof(T)));
+    EIO_CHECK_HIP(device_malloc(c, &m.damp, damp.size() * sizeof(T)));
+    EIO_CHECK_HIP(device_malloc(c, &m.filt, filt.size() * sizeof(T)));
     EIO_CHECK_HIP(hipMemcpy(m.damp, damp.data(), damp.size() * sizeof(T), hipMemcpyHostToDevice));
     EIO_CHECK_HIP(hipMemcpy(m.filt, filt.data(), filt.size() * sizeof(T), hipMemcpyHostToDevice));
     upload_model<T>(c, m, media, flags);
@@ -1507,10 +1554,10 @@ std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots
     return out;
 }
 
-// Tiles and entries of the groups, their device tables and the exchange buffers.  `tag` keeps the
-// buffers of two plans of one call apart.
+// Tiles and entries of the groups, their device tables and the exchange buffers (at most 21 MB); false: no
+// memory for them.  `tag` keeps the buffers of two plans of one call apart.
 template <typename T>
-void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp, const std::string& tag = "res_") {
+bool res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp, const std::string& tag = "res_") {
     Ctx* c = run.c;
     int maxR = 1;
     for (const ResGroup& g : rp.groups) {
@@ -1555,19 +1602,21 @@ void res_build(Run<T>& run, const eio_shot* shots, ResPlan& rp, const std::strin
         }
     }
     const hipMemcpyKind h2d = hipMemcpyHostToDevice;
-    rp.d_tiles = static_cast<eio::ResTile*>(ws_get(c, tag + "tiles", sizeof(eio::ResTile) * rp.tiles.size()));
-    rp.d_ents = static_cast<eio::Entry*>(ws_get(c, tag + "ents", sizeof(eio::Entry) * std::max<size_t>(1, rp.ents.size())));
-    EIO_CHECK_HIP(hipMemcpyAsync(rp.d_tiles, rp.tiles.data(), sizeof(eio::ResTile) * rp.tiles.size(), h2d, c->stream));
-    if (!rp.ents.empty())
-        EIO_CHECK_HIP(hipMemcpyAsync(rp.d_ents, rp.ents.data(), sizeof(eio::Entry) * rp.ents.size(), h2d, c->stream));
     const size_t per_tile = 2 * (32 * size_t(RES_WX * maxR) + 2048);  // Inbox<TX>::TILE
     int ntile = 0;
     for (const ResGroup& g : rp.groups) ntile = std::max(ntile, g.ntile);
     rp.inbox_bytes = size_t(ntile) * per_tile * eio::Packet<T>::BYTES;
-    rp.inbox = ws_get(c, tag + "inbox", rp.inbox_bytes);
-    rp.abort_flag = static_cast<int*>(ws_get(c, tag + "abort", 256));
-    rp.xcd = static_cast<int*>(ws_get(c, tag + "xcd", size_t(c->ncu) * sizeof(int)));
+    rp.d_tiles = static_cast<eio::ResTile*>(ws_try(c, tag + "tiles", sizeof(eio::ResTile) * rp.tiles.size()));
+    rp.d_ents = static_cast<eio::Entry*>(ws_try(c, tag + "ents", sizeof(eio::Entry) * std::max<size_t>(1, rp.ents.size())));
+    rp.inbox = ws_try(c, tag + "inbox", rp.inbox_bytes);
+    rp.abort_flag = static_cast<int*>(ws_try(c, tag + "abort", 256));
+    rp.xcd = static_cast<int*>(ws_try(c, tag + "xcd", size_t(c->ncu) * sizeof(int)));
+    if (!rp.d_tiles || !rp.d_ents || !rp.inbox || !rp.abort_flag || !rp.xcd) return false;
+    EIO_CHECK_HIP(hipMemcpyAsync(rp.d_tiles, rp.tiles.data(), sizeof(eio::ResTile) * rp.tiles.size(), h2d, c->stream));
+    if (!rp.ents.empty())
+        EIO_CHECK_HIP(hipMemcpyAsync(rp.d_ents, rp.ents.data(), sizeof(eio::Entry) * rp.ents.size(), h2d, c->stream));
     fill0<int>(c, rp.abort_flag, 1);
+    return true;
 }
 
 // The errors of a cooperative launch that a device which cannot take it now returns: one process at a time
@@ -1760,7 +1809,7 @@ bool nl_forward_resident(Ctx* c, int nshot, const eio_shot* shots, int flags, bo
     rp.groups = res_choose<T>(c, make_plan<T>(c, nshot, shots, Op::NL_FWD, PlanKind::NONE), shots, ResKind::NL);
     if (rp.groups.empty()) return false;
     Run<T> run = prepare<T>(c, nshot, shots, Op::NL_FWD, flags, nullptr, nullptr, 0, false, false, false, false, false, 1);
-    res_build(run, shots, rp);
+    if (!res_build(run, shots, rp)) return false;
     c->last_groups = int(rp.groups.size());
     timing_begin<T>(c);
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
@@ -2039,7 +2088,7 @@ bool nl_adjoint_resident(Ctx* c, int nshot, const eio_shot* shots, int flags) {
     rp.groups = res_choose<T>(c, make_plan<T>(c, nshot, shots, Op::NL_ADJ, PlanKind::NONE), shots, ResKind::ADJ);
     if (rp.groups.empty()) return false;
     Run<T> run = prepare<T>(c, nshot, shots, Op::NL_ADJ, flags, nullptr, nullptr, 0, false, false, false, false, false, 1);
-    res_build(run, shots, rp);
+    if (!res_build(run, shots, rp)) return false;
     int kmax = run.plan.nsteps[0];
     if (c->step_limit > 0) kmax = std::min(kmax, c->step_limit);
     timing_begin<T>(c);
@@ -2129,8 +2178,7 @@ bool born_source_resident(Run<T>& run, int nshot, const eio_shot* shots) {
     Ctx* c = run.c;
     ResPlan rp;
     rp.groups = res_choose<T>(c, run.plan, shots, ResKind::DEC);
-    if (rp.groups.empty()) return false;
-    res_build(run, shots, rp);
+    if (rp.groups.empty() || !res_build(run, shots, rp)) return false;
     for (const ResGroup& g : rp.groups)
         res_launch_fwd<T, eio::M_BSRC>(run, rp, g, 0, run.plan.nsteps[g.s0], true, false, 0, -1);
     return !res_aborted(c, rp);
@@ -2148,9 +2196,29 @@ struct ResRing {
     eio::TileDev* d_tiles = nullptr;
     std::vector<eio::ShotDev<T>> sd;
     eio::ShotDev<T>* d_shots = nullptr;
+    Ctx* c = nullptr;     // while the context's ring buffer is in use
+    bool keep = true;     // the buffer stays with the context
+    // after the stream's work on the ring is done (res_aborted waits for it)
+    void done() {
+        if (!c) return;
+        Ctx* const ctx = c;
+        c = nullptr;
+        ctx->ring_busy = false;
+        if (keep) return;
+        (void)hipStreamSynchronize(ctx->stream);
+        ring_free(ctx);
+    }
+    ResRing() = default;
+    ResRing(const ResRing&) = delete;
+    ResRing& operator=(const ResRing&) = delete;
+    ~ResRing() { done(); }
 };
 
-// The ring of a plan's groups (one after the other in the same memory); false: no memory for it.
+// The ring of a plan's groups (one after the other in the same memory); false: no memory for it.  0.7 GB
+// at most (33 samples of five fields of the cells that fit the chip; half as much again for the smallest
+// grids, whose pads count).  Whether it fits is the allocation's to say, not
+// what happens to be free, so that a call gives the same bits on a full card as on an empty one; where less
+// than three times its size is left beside it, it is given back at the end of the call.
 template <typename T>
 bool ring_build(Run<T>& run, const ResPlan& rp, ResRing<T>& ring) {
     Ctx* c = run.c;
@@ -2159,11 +2227,15 @@ bool ring_build(Run<T>& run, const ResPlan& rp, ResRing<T>& ring) {
     ring.K = std::min(RES_RING, run.sd[0].nts - 1);
     int most = 0;
     for (const ResGroup& g : rp.groups) most = std::max(most, g.s1 - g.s0);
-    // a ring is extra memory: only where it leaves plenty of what is free to the rest of the call
     const size_t bytes = size_t(most) * (ring.K + 1) * n5 * sizeof(T);
+    auto held = c->ws.find("res_ring");
+    const bool grows = held == c->ws.end() || held->second.bytes < bytes;
+    T* buf = static_cast<T*>(ws_try(c, "res_ring", bytes));
+    if (!buf) return false;
+    c->ring_busy = true;
+    ring.c = c;
     size_t avail = 0, total = 0;
-    if (c->ws["res_ring"].bytes < bytes && (hipMemGetInfo(&avail, &total) != hipSuccess || bytes > avail / 4)) return false;
-    T* buf = static_cast<T*>(ws_get(c, "res_ring", bytes));
+    ring.keep = !grows || (hipMemGetInfo(&avail, &total) == hipSuccess && avail / 3 >= bytes);
     ring.sd = run.sd;
     for (const ResGroup& g : rp.groups)
         for (int oi = g.s0; oi < g.s1; ++oi) {
@@ -2210,8 +2282,7 @@ bool scattered_pass_resident(Run<T>& run, int nshot, const eio_shot* shots) {
     ResPlan rp;
     ResRing<T> ring;
     rp.groups = res_choose<T>(c, run.plan, shots, ResKind::SCAT, std::min(RES_RING, nts - 1) * sub);
-    if (rp.groups.empty() || !ring_build(run, rp, ring)) return false;
-    res_build(run, shots, rp, "resa_");
+    if (rp.groups.empty() || !ring_build(run, rp, ring) || !res_build(run, shots, rp, "resa_")) return false;
     for (const ResGroup& g : rp.groups)
         for (int a = 0; a < nts - 1; a += ring.K) {   // intervals a .. b-1 use the samples a .. b
             const int b = std::min(a + ring.K, nts - 1);
@@ -2251,8 +2322,7 @@ bool receiver_pass_build(Run<T>& run, int nshot, const eio_shot* shots, ResPlan&
     Ctx* c = run.c;
     rp.groups = res_choose<T>(c, run.plan, shots, ResKind::BADJ, std::min(RES_RING, run.sd[0].nts - 1) * run.sd[0].sub);
     if (rp.groups.empty() || (one_group && rp.groups.size() > 1) || !ring_build(run, rp, ring)) return false;
-    res_build(run, shots, rp, "resa_");
-    return true;
+    return res_build(run, shots, rp, "resa_");
 }
 
 template <typename T>
@@ -2435,7 +2505,7 @@ bool fwi_forward_resident(Ctx* c, int nshot, const eio_shot* shots, int flags, F
     if (rp.groups.empty()) return false;
     Run<T> run = prepare<T>(c, nshot, shots, Op::FWI_FWD, flags, nullptr, static_cast<T*>(f.ring), f.wcap, false, false,
                             false, false, false, f.nseg > 1 ? 2 : 1);
-    res_build(run, shots, rp);
+    if (!res_build(run, shots, rp)) return false;
     const size_t n10 = 10 * size_t(run.sd[0].nz) * run.sd[0].nx;
     timing_begin<T>(c);
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
@@ -2491,8 +2561,8 @@ int fwi_forward(Ctx* c, int nshot, const eio_shot* shots, int flags, int segment
             throw EioError{EIO_ERR_RUNTIME, oom};
         }
     } else {
-        if (hipMalloc(&f.ring, ring_elems * sizeof(T)) != hipSuccess ||
-            (ck_elems && hipMalloc(&f.ck, ck_elems * sizeof(T)) != hipSuccess)) {
+        if (device_malloc(c, &f.ring, ring_elems * sizeof(T)) != hipSuccess ||
+            (ck_elems && device_malloc(c, &f.ck, ck_elems * sizeof(T)) != hipSuccess)) {
             (void)hipGetLastError();
             fwi_free(c, f);
             throw EioError{EIO_ERR_RUNTIME, oom};
@@ -2600,7 +2670,11 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
     if (rres) {
         rp.groups = res_groups<T>(c, make_plan<T>(c, nshot, shots, Op::FWI_GRAD, PlanKind::NONE), shots, ResKind::DEC);
         if (rp.groups.empty()) throw EioError{EIO_ERR_STATE, "the device no longer takes the resident loop of this store"};
-        res_build(run, shots, rp);
+        if (!res_build(run, shots, rp)) {
+            ResidentOff off(c);
+            fwi_gradient<T>(c, handle, nshot, shots, dm, flags);
+            return;
+        }
     }
     long long nrecomp = 0;
     for (int j = 0; j + 1 < f.nseg; ++j) nrecomp += (long long)(seg_end(f, j) - seg_begin(f, j)) * sub;
@@ -2680,10 +2754,12 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
     EIO_CHECK_HIP(hipEventRecord(c->ev[3], c->stream));
     timing_end<T>(c, (long long)(nts - 1) * sub + nrecomp);
     if ((rres && res_aborted(c, rp)) || (ares && res_aborted(c, rpa))) {  // a wait was given up: the whole sweep again, launched
+        ring.done();
         ResidentOff off(c);
         fwi_gradient<T>(c, handle, nshot, shots, dm, flags);
         return;
     }
+    ring.done();
     stack_into(run, m, nshot, dm, flags);
     finish(run);
 }
@@ -3151,7 +3227,7 @@ int eio_device_alloc(eio_ctx* ctx, unsigned long long bytes, void** ptr) {
         Ctx* c = as_ctx(ctx);
         if (!ptr) fail("ptr is NULL");
         DeviceGuard dg(c->device);
-        EIO_CHECK_HIP(hipMalloc(ptr, bytes));
+        EIO_CHECK_HIP(device_malloc(c, ptr, bytes));
     });
 }
 

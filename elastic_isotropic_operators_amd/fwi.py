@@ -157,6 +157,19 @@ def cache_group(nz, nx, itemsize, budget=CACHE_GROUP_BYTES):
     return max(1, int(budget // (GRADIENT_VALUES_PER_CELL * int(nz) * int(nx) * int(itemsize))))
 
 
+# The widest tiles of a resident receiver pass of the library, 64 rows by 256 bytes of columns, and how many
+# of them the chip holds.
+RESIDENT_TILES = 256
+
+
+def resident_ring_bytes(nshot, nz, nx, nts, itemsize):
+    """Most that the ring of the library's resident receiver pass takes: 33 coarse samples of five fields
+    of as many of the shots as the chip holds at once (0 where not even one fits)."""
+    tiles = -(-(int(nz) - 8) // 64) * -(-(int(nx) - 8) // (256 // int(itemsize)))
+    fit = RESIDENT_TILES // max(1, tiles)
+    return 5 * min(33, int(nts)) * int(nz) * int(nx) * int(itemsize) * min(int(nshot), fit)
+
+
 def group_and_segment(group, fit, nshot, nts, segment, checkpoint=None):
     """Shots per group and the store's segment length (coarse intervals) of one
     misfit_and_gradient call.  fit: shots whose whole coarse Vx/Vz record fits in memory;
@@ -375,10 +388,11 @@ class ElasticFwi:
         """Shots per group whose full coarse Vx/Vz storage (2 nz nx nts values per shot) fits in
         `margin` of the free device memory (0 when not even one shot fits)."""
         free, _ = torch.cuda.mem_get_info(self.device)
+        size = torch.tensor([], dtype=self.dtype).element_size()
         # the record (2 nts fields) + state levels (4 x 5), recompute state (4 x 5), adjoint-field
         # slots (2 x 5), accumulators (5) and traces, rounded up
-        per_shot = (2 * self.nts + 60) * self.nz * self.nx * torch.tensor([], dtype=self.dtype).element_size()
-        return int(margin * free // per_shot)
+        per_shot = (2 * self.nts + 60) * self.nz * self.nx * size
+        return int(margin * max(0, free - resident_ring_bytes(self.nshot, self.nz, self.nx, self.nts, size)) // per_shot)
 
     def default_group(self):
         """Shots per group of misfit_and_gradient when the caller gives none: as many as keep

@@ -116,7 +116,8 @@ int eio_ctx_set_variant(eio_ctx* ctx, int variant);
  * 56 x 32 (variant 4).  With EIO_VARIANT_AUTO, time block 2 and EIO_GROUP_AUTO (and in every FP64
  * context), a pass whose shots fit the chip runs as RESIDENT loops instead where that is faster: one
  * cooperative launch for the whole loop of a group of shots (32 coarse intervals at a time in the Born
- * scattered and receiver passes), the state in LDS and registers.  eio_ctx_last_timing then counts these
+ * scattered and receiver passes, through a ring of at most about 1 GB that the context keeps, and gives back
+ * where little memory is left beside it), the state in LDS and registers.  eio_ctx_last_timing then counts these
  * launches for the NL forward, eio_ctx_last_shot_groups the groups.  Graphs, the persistent mode, explicit
  * variants of the launched form a pass would take, saved wavefields, snapshots, learned boundaries and the no-allocation call keep to launched
  * steps.  A call whose device refuses a cooperative launch (one process at a time holds a device's

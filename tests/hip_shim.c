@@ -9,18 +9,15 @@
 typedef struct { unsigned x, y, z; } dim3_t;
 
 static int launch_code, launch_left, launch_after;   /* after `after` more launches, `left` of them return `code` */
-static size_t malloc_limit = ~(size_t)0;             /* larger allocations: hipErrorOutOfMemory */
-static size_t free_shown;                            /* free memory to report (0: the device's) */
+static size_t capacity = ~(size_t)0, live;           /* the device's memory, and what is allocated of it here */
 
 void shim_launches(int code, int count, int after) {
     launch_code = code;
     launch_left = count;
     launch_after = after;
 }
-void shim_memory(size_t limit, size_t shown) {
-    malloc_limit = limit;
-    free_shown = shown;
-}
+void shim_capacity(size_t bytes) { capacity = bytes; }
+size_t shim_live(void) { return live; }
 
 int hipLaunchCooperativeKernel(const void* f, dim3_t g, dim3_t b, void** args, unsigned lds, void* stream) {
     static int (*real)(const void*, dim3_t, dim3_t, void**, unsigned, void*);
@@ -32,16 +29,40 @@ int hipLaunchCooperativeKernel(const void* f, dim3_t g, dim3_t b, void** args, u
     return real(f, g, b, args, lds, stream);
 }
 
+static struct { void* p; size_t n; } table[4096];
+
 int hipMalloc(void** p, size_t n) {
     static int (*real)(void**, size_t);
     if (!real) *(void**)&real = dlsym(RTLD_NEXT, "hipMalloc");
-    return n > malloc_limit ? 2 : real(p, n);
+    if (n > capacity || live > capacity - n) return 2; /* hipErrorOutOfMemory */
+    const int e = real(p, n);
+    for (int i = 0; !e && i < 4096; ++i)
+        if (!table[i].p) {
+            table[i].p = *p;
+            table[i].n = n;
+            live += n;
+            break;
+        }
+    return e;
+}
+
+int hipFree(void* p) {
+    static int (*real)(void*);
+    if (!real) *(void**)&real = dlsym(RTLD_NEXT, "hipFree");
+    for (int i = 0; p && i < 4096; ++i)
+        if (table[i].p == p) {
+            live -= table[i].n;
+            table[i].p = NULL;
+            break;
+        }
+    return real(p);
 }
 
 int hipMemGetInfo(size_t* avail, size_t* total) {
     static int (*real)(size_t*, size_t*);
     if (!real) *(void**)&real = dlsym(RTLD_NEXT, "hipMemGetInfo");
     const int e = real(avail, total);
-    if (!e && free_shown) *avail = free_shown;
+    const size_t left = capacity > live ? capacity - live : 0;
+    if (!e && left < *avail) *avail = left;
     return e;
 }

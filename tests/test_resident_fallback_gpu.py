@@ -32,7 +32,8 @@ def shim(tmp_path_factory):
                     "-L/opt/rocm/lib", "-Wl,--no-as-needed", "-lamdhip64"], check=True)
     shutil.copy(_capi.LIB_PATH, lib)
     s = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)
-    s.shim_memory.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+    s.shim_capacity.argtypes = [ctypes.c_size_t]
+    s.shim_live.restype = ctypes.c_size_t
     spec = importlib.util.spec_from_file_location("eio_capi_shimmed", _capi.__file__)
     capi = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(capi)
@@ -45,7 +46,7 @@ def shim(tmp_path_factory):
 def shimmed(shim):
     yield shim
     shim[0].shim_launches(0, 0, 0)
-    shim[0].shim_memory(~0 & (2 ** 64 - 1), 0)
+    shim[0].shim_capacity(2 ** 64 - 1)
 
 
 def _shim_ctx(capi, dtype):
@@ -215,3 +216,69 @@ def test_explicit_variant_keeps_launched_steps(dtype, sub, surface):
     ctx.set_variant(_capi.VARIANT_AUTO)
     assert _passes(ctx, mid, g, dtype) == auto
     ctx.close()
+
+
+@pytest.mark.parametrize("dtype,nz,nx", [(np.float32, 139, 90), (np.float64, 300, 500)])
+def test_born_ring_on_a_full_card(shimmed, dtype, nz, nx):
+    """The ring of the Born passes: the same bits whatever memory is free, kept where there is plenty, given back
+    at the call's end where there is little and when another allocation needs it, and done without (launched
+    passes) where there is none."""
+    shim, capi = shimmed
+    nts, sub = 70, 4
+    size = np.dtype(dtype).itemsize
+    ring = 33 * 5 * nz * nx * size
+    rng = np.random.default_rng(61)
+    grads, data, fit, ref = [], [], [], None
+    # what is left when the call has all but the ring: plenty, half a ring more than it, half a ring
+    for spare in (100.0, 1.5, 0.5):
+        shim.shim_capacity(2 ** 64 - 1)
+        ctx = _shim_ctx(capi, dtype)
+        mid, g, med = _model(ctx, nz, nx, nts, sub, 62)
+        if ref is None:
+            spos, rpos = _positions(rng, g, 10), _positions(rng, g, 80)
+            src = [O.time_interp(s, g.dts, sub) for s in random_traces(rng, spos, nts, np.float64)]
+            dat = random_traces(rng, rpos, nts, np.float64)
+            dmod = np.zeros((5, nx, nz))
+            dmod[:, 4:-4, 4:-4] = rng.standard_normal((5, nx - 8, nz - 8)) * np.abs(med).reshape(5, -1).max(1)[:, None, None]
+            ref = (O.born_adj_reg(g, med, spos, src, rpos, dat, np.float64), O.born_fwd_reg(g, med, spos, src, dmod, rpos, np.float64))
+        srcd, datd, dmd = ([np.ascontiguousarray(t, dtype) for t in src], [np.ascontiguousarray(t, dtype) for t in dat],
+                           np.ascontiguousarray(dmod, dtype))
+
+        def call():
+            dm = np.zeros((5, nx, nz), dtype)
+            sh, keep = ctx.make_shot(mid, spos, rpos, srcd, datd)
+            ctx.born_adjoint([sh], dm)
+            rec = [np.zeros_like(t) for t in datd]
+            sh, keep = ctx.make_shot(mid, spos, rpos, srcd, rec)
+            ctx.born_forward([sh], dmd)
+            assert rel_l2(dm, ref[0]) < GRAD_TOL[dtype]
+            _check(rec, ref[1], dtype)
+            return dm, rec
+
+        call()
+        fit.append(shim.shim_live() - ring)      # every buffer of the two calls but the ring
+        if spare < 100:
+            ctx.release_workspace()
+            shim.shim_capacity(int(fit[-1] + spare * ring))
+        before = ctx.resident_info()[0]
+        for _ in range(2):
+            dm, rec = call()
+            grads.append(dm)
+            data.append(rec)
+        launches = ctx.resident_info()[0] - before
+        if spare > 1:
+            # source pass and three launches of 32 intervals each, twice the pair of calls
+            assert launches == 2 * 2 * 4, launches
+            assert np.array_equal(grads[0], dm) and all(np.array_equal(a, b) for a, b in zip(data[0], rec))
+        else:
+            assert launches == 2 * 2, launches    # the source passes only
+            assert shim.shim_live() <= fit[-1]
+        if spare > 1:
+            assert shim.shim_live() == fit[-1] + (ring if spare > 3 else 0)
+        if spare == 100.0:     # memory for something else that only the ring's would give
+            shim.shim_capacity(fit[-1] + ring + ring // 4)
+            p = ctx.alloc(ring)
+            assert shim.shim_live() == fit[-1] + ring
+            ctx.free(p)
+        ctx.close()
+        assert shim.shim_live() == 0
