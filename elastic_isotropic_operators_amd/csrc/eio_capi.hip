@@ -3227,7 +3227,7 @@ int eio_device_alloc(eio_ctx* ctx, unsigned long long bytes, void** ptr) {
         Ctx* c = as_ctx(ctx);
         if (!ptr) fail("ptr is NULL");
         DeviceGuard dg(c->device);
-        EIO_CHECK_HIP(device_malloc(c, ptr, bytes));
+        EIO_CHECK_HIP(hipMalloc(ptr, bytes));
     });
 }
 

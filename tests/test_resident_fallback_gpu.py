@@ -275,10 +275,9 @@ def test_born_ring_on_a_full_card(shimmed, dtype, nz, nx):
             assert shim.shim_live() <= fit[-1]
         if spare > 1:
             assert shim.shim_live() == fit[-1] + (ring if spare > 3 else 0)
-        if spare == 100.0:     # memory for something else that only the ring's would give
+        if spare == 100.0:     # a model whose media (33 x 5 fields of the grid) only the ring's memory can hold
             shim.shim_capacity(fit[-1] + ring + ring // 4)
-            p = ctx.alloc(ring)
-            assert shim.shim_live() == fit[-1] + ring
-            ctx.free(p)
+            _model(ctx, nz, 33 * nx, nts, sub, 63)
+            assert fit[-1] + ring <= shim.shim_live() < fit[-1] + ring + 4096
         ctx.close()
         assert shim.shim_live() == 0
