@@ -281,3 +281,63 @@ def test_born_ring_on_a_full_card(shimmed, dtype, nz, nx):
             assert fit[-1] + ring <= shim.shim_live() < fit[-1] + ring + 4096
         ctx.close()
         assert shim.shim_live() == 0
+
+
+@pytest.mark.parametrize("dtype,nz,nx", [(np.float32, 300, 700), (np.float64, 300, 500)])
+def test_refused_in_the_middle_of_a_pass(shimmed, dtype, nz, nx):
+    """A refusal after some launches of a scattered or receiver pass or of a checkpointed gradient: what they left
+    in the outputs, the ring and the record is made again, launched."""
+    shim, capi = shimmed
+    nts, sub, segment = 70, 3, 23
+    ctx = _shim_ctx(capi, dtype)
+    mid, g, med = _model(ctx, nz, nx, nts, sub, 81)
+    rng = np.random.default_rng(82)
+    spos, rpos = _positions(rng, g, 10), _positions(rng, g, 80)
+    src = random_traces(rng, spos, nts, np.float64)
+    fine = [O.time_interp(s, g.dts, sub) for s in src]
+    dat = random_traces(rng, rpos, nts, np.float64)
+    dmod = np.zeros((5, nx, nz))
+    dmod[:, 4:-4, 4:-4] = rng.standard_normal((5, nx - 8, nz - 8)) * np.abs(med).reshape(5, -1).max(1)[:, None, None]
+    ref_dm = O.born_adj_reg(g, med, spos, fine, rpos, dat, np.float64)
+    ref_lin = O.born_fwd_reg(g, med, spos, fine, dmod, rpos, np.float64)
+    srcd, fined, datd = ([np.ascontiguousarray(t, dtype) for t in tr] for tr in (src, fine, dat))
+
+    def fresh_ctx_state():
+        while ctx.resident_info()[0] == forms[0]:      # the calls that do not try after a failure
+            shot, keep = ctx.make_shot(mid, spos, rpos, srcd, [np.zeros_like(t) for t in datd])
+            ctx.nl_forward([shot])
+        forms[0] = ctx.resident_info()[0]
+
+    forms = [-1]
+    refusals = 0
+    for after in (0, 1, 2, 3):
+        forms[0] = ctx.resident_info()[0]
+        fresh_ctx_state()
+        shim.shim_launches(ILLEGAL_STATE, 1, after)
+        dm = np.zeros((5, nx, nz), dtype)
+        shot, keep = ctx.make_shot(mid, spos, rpos, fined, datd)
+        ctx.born_adjoint([shot], dm)
+        assert rel_l2(dm, ref_dm) < GRAD_TOL[dtype], (after, rel_l2(dm, ref_dm))
+
+        forms[0] = ctx.resident_info()[0]
+        fresh_ctx_state()
+        shim.shim_launches(ILLEGAL_STATE, 1, after)
+        rec = [np.full_like(t, 7) for t in datd]
+        shot, keep = ctx.make_shot(mid, spos, rpos, fined, rec)
+        ctx.born_forward([shot], np.ascontiguousarray(dmod, dtype))
+        _check(rec, ref_lin, dtype)
+
+        forms[0] = ctx.resident_info()[0]
+        fresh_ctx_state()
+        shot, keep = ctx.make_shot(mid, spos, rpos, srcd, [np.zeros_like(t) for t in datd])
+        h = ctx.fwi_forward([shot], segment)
+        shim.shim_launches(ILLEGAL_STATE, 1, after)
+        for _ in range(2):
+            dm = np.zeros((5, nx, nz), dtype)
+            shot, keep = ctx.make_shot(mid, spos, rpos, srcd, datd)
+            ctx.fwi_gradient(h, [shot], dm)
+            assert rel_l2(dm, ref_dm) < GRAD_TOL[dtype], (after, rel_l2(dm, ref_dm))
+        ctx.fwi_release(h)
+        refusals += 3
+        assert ctx.resident_info()[2] == refusals
+    ctx.close()
