@@ -1472,6 +1472,7 @@ struct ResGroup {
     int s0, s1;       // shots, in plan order
     int R;            // columns per wave
     int tile0, ntile;
+    double us;        // of one fine step (res_step_us)
 };
 struct ResPlan {
     std::vector<ResGroup> groups;
@@ -1497,20 +1498,31 @@ template <typename T>
 constexpr int res_max_r(ResKind k) {
     return sizeof(T) == 8 ? 2 : k == ResKind::NL ? 6 : k == ResKind::BADJ || k == ResKind::SCAT ? 4 : 5;
 }
-// Measured time of one fine step of a launch with R columns per wave [us] (every CU busy; the
-// halo exchange and the barriers are about 2.5 us of it, so wide tiles do the most work per
-// time, and narrow ones finish a call that cannot fill the device soonest); the Born passes that trade
-// coarse samples with the imaging include its time.
+// Measured time of one fine step of a launch with R columns per wave [us] (the halo exchange and the
+// barriers are about 2.5 us of it, so wide tiles do the most work per time, and narrow ones finish a call that
+// cannot fill the device soonest); the Born passes that trade coarse samples with the imaging include its time.
+// At R = 1 the exchange is all there is, and a step follows what the tiles trade over: nothing (each shot one
+// tile), one row or column of tiles or shots that mostly lie on one XCD each, or both ways across XCDs.
+enum class ResShape { TILE, LINE, GRID };
 template <typename T>
-double res_step_us(ResKind k, int R) {
-    constexpr double nl[] = {3.4, 3.85, 5.05, 5.65, 7.0, 8.7}, dec[] = {3.5, 4.0, 5.2, 5.8, 8.2}, f64[] = {5.1, 6.15};
-    constexpr double adj[] = {3.35, 4.1, 5.35, 6.0, 8.4}, adj64[] = {5.15, 7.65};
-    constexpr double badj[] = {3.9, 5.0, 7.0, 10.7}, badj64[] = {6.9, 14.0};
-    constexpr double scat[] = {3.9, 4.9, 7.2, 11.8}, scat64[] = {7.1, 19.0};
-    if (k == ResKind::SCAT) return sizeof(T) == 8 ? scat64[R - 1] : scat[R - 1];
-    if (k == ResKind::ADJ) return sizeof(T) == 8 ? adj64[R - 1] : adj[R - 1];
-    if (k == ResKind::BADJ) return sizeof(T) == 8 ? badj64[R - 1] : badj[R - 1];
-    return sizeof(T) == 8 ? f64[R - 1] : k == ResKind::NL ? nl[R - 1] : dec[R - 1];
+double res_step_us(ResKind k, int R, ResShape shape) {
+    constexpr bool F32 = sizeof(T) == 4;
+    // R = 1: TILE, LINE, GRID
+    constexpr double one32[][3] = {{1.95, 2.85, 3.5}, {2.25, 3.3, 3.7}, {3.9, 3.9, 3.9}, {2.1, 2.9, 3.5}, {3.9, 3.9, 3.9}};
+    constexpr double one64[][3] = {{2.95, 4.8, 5.35}, {3.4, 5.1, 5.7}, {7.1, 7.1, 7.1}, {3.05, 4.7, 5.3}, {6.9, 6.9, 6.9}};
+    // R = 2 and wider
+    constexpr double wide32[][5] = {{3.85, 5.05, 5.65, 7.0, 8.7}, {4.4, 5.7, 6.3, 8.8}, {4.9, 7.2, 11.8}, {4.1, 5.35, 6.0, 8.4}, {5.0, 7.0, 10.7}};
+    constexpr double two64[] = {6.4, 8.0, 19.0, 8.0, 14.0};
+    if (R == 1) return (F32 ? one32 : one64)[int(k)][int(shape)];
+    return F32 ? wide32[int(k)][R - 2] : two64[int(k)];
+}
+// The shots of a launch of R = 1.  Tiles go to the eight XCDs in runs of consecutive ones, so that the shots of
+// a launch of four or more are cut once or not at all; up to two tiles an XCD (FP64: three) no tile trades
+// with more than a few others.
+template <typename T>
+ResShape res_shape(int nshot, int ntile, bool line) {
+    if (ntile == nshot) return ResShape::TILE;
+    return line || nshot >= 4 || ntile <= 8 * (sizeof(T) == 4 ? 2 : 3) ? ResShape::LINE : ResShape::GRID;
 }
 
 // The groups of a call that take the least time in all, or none when a shot does not fit the device.
@@ -1525,20 +1537,24 @@ std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots
     std::vector<ResGroup> best(n);
     std::vector<double> cost(n + 1, 0.0);
     for (int s0 = n - 1; s0 >= 0; --s0) {
-        best[s0] = ResGroup{s0, s0, 0, 0, 0};
+        best[s0] = ResGroup{s0, s0, 0, 0, 0, 0.0};
         cost[s0] = 1e30;
         for (int R = 1; R <= RM; ++R) {
             int nt = 0, s1 = s0;
+            bool line = true;
             while (s1 < n) {
-                const int k = res_tiles(get_model(c, shots[plan.order[s1]].model), R);
+                const ModelBase& m = get_model(c, shots[plan.order[s1]].model);
+                const int k = res_tiles(m, R);
                 if (nt + k > c->ncu) break;
                 nt += k;
+                line = line && (m.g.nz - 2 * eio::FAT <= eio::TZ || m.g.nx - 2 * eio::FAT <= RES_WX);
                 ++s1;
             }
             if (s1 == s0) continue;
-            const double t = RES_SETUP_US + res_step_us<T>(kind, R) * plan.nsteps[s0] + cost[s1];
+            const double us = res_step_us<T>(kind, R, res_shape<T>(s1 - s0, nt, line));
+            const double t = RES_SETUP_US + us * plan.nsteps[s0] + cost[s1];
             if (t < cost[s0]) {
-                best[s0] = {s0, s1, R, 0, nt};
+                best[s0] = {s0, s1, R, 0, nt, us};
                 cost[s0] = t;
             }
         }
@@ -1756,17 +1772,23 @@ bool res_allowed(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) 
 
 // The groups of a pass of `per_launch` fine steps a launch (0: each group's own steps), or none
 // where the launched kernels are the faster form: their time is a part per step and one per cell (the
-// table below, measured), a resident launch takes its steps and a set-up: cleared inboxes, a cooperative
+// tables below, measured), a resident launch takes its steps and a set-up: cleared inboxes, a cooperative
 // launch and the state's first load, some 60 us, and 100 where the state comes from and goes back to
-// memory between segments.  Whole calls, resident against launched: 280 x 472, 396 against 373 us at 64
-// fine steps, 622 against 635 at 128; 600 x 1592, 262 against 249 us at 10, 310 against 352 at 18; a
-// checkpointed forward and gradient of four shots of 280 x 472 in segments of 46 steps, 24.4 against 28.2 ms.
-// Per step, launched and resident (both Born passes together, with imaging), in us:
+// memory between segments.  Per step of whole calls, launched and resident (both Born passes together, with
+// imaging), in us:
 //                       forward      adjoint      Born forward  Born adjoint
-//   280 x 472         4.2   3.4     4.7   3.35   10.4   7.4     12.1   7.5
-//   four of them      7.9   5.05    10.0  5.35   21.8   12.7    24.3   12.3
-//   600 x 1592        12.0  5.65    15.2  5.9    32.6   17.8    35.4   16.5
-//   FP64, 280 x 472   6.0   5.1     8.6   5.15   19.8   12.2    26.2   12.0
+//   72 x 88           3.35  2.85    3.55  2.8    8.9   6.8     10.1  7.1
+//   200 x 200         3.3   3.5     3.45  3.6    9.0   8.0     10.7  8.7
+//   280 x 472         4.0   3.5     4.3   3.35   11.7  8.1     13.4  8.3
+//   four of them      7.9   5.05    10.0  5.35   21.8  12.7    24.3  12.3
+//   600 x 1592        12.0  5.65    15.2  5.9    36.3  21.8    40.4  20.0
+//   FP64, 200 x 200   5.4   5.4     6.2   5.25   14.7  12.7    17.4  12.8
+//   FP64, 280 x 472   6.9   5.3     8.2   5.15   21.6  13.3    26.5  13.0
+// Whole calls, resident against launched: 280 x 472, 0.60 ms both at 100 fine steps, 0.78 against 0.84 at 160;
+// 600 x 1592, 0.26 against 0.25 at 10, 0.31 against 0.35 at 18; a checkpointed forward and gradient of four shots of
+// 280 x 472 in segments of 46 steps, 24.4 against 28.2.  Where an FP32 forward has 17 tiles or more and up to 90,000 cells
+// the launched form is the faster one (200 x 200: 1.05 against 0.97 at 238 steps, 3.7 against 3.5 at 1000); on fewer tiles
+// the two are within 5 % of one another, and one launch a call leaves the host free.
 constexpr double RES_SEGMENT_US = 100.0;
 template <typename T>
 std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
@@ -1776,19 +1798,24 @@ std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots
     int longest = 0;
     for (const ResGroup& g : groups) {
         const int steps = per_launch ? per_launch : plan.nsteps[g.s0];
-        res += (per_launch ? RES_SEGMENT_US : RES_SETUP_US) + steps * res_step_us<T>(kind, g.R);
+        res += (per_launch ? RES_SEGMENT_US : RES_SETUP_US) + steps * g.us;
         longest = std::max(longest, steps);
         for (int i = g.s0; i < g.s1; ++i)
             work += double(get_model(c, shots[plan.order[i]].model).n) * (per_launch ? per_launch : plan.nsteps[i]);
     }
-    // launched: us a step and cells a us (FP32 two steps per launch, FP64 one); Born passes with their imaging
+    // launched: us a step and cells a us; Born passes with their imaging
     struct Cost {
         double step, rate, least;
     };
-    constexpr Cost f32[] = {{2.6, 100e3, 4.2}, {2.6, 100e3, 4.2}, {4.5, 57e3, 4.5}, {3.0, 75e3, 4.2}, {5.5, 48e3, 5.5}};
-    constexpr Cost f64[] = {{0.0, 22e3, 6.0}, {0.0, 22e3, 6.0}, {7.0, 21e3, 7.0}, {5.0, 38e3, 6.0}, {9.5, 13.5e3, 9.5}};
-    const Cost& l = (sizeof(T) == 4 ? f32 : f64)[int(kind)];
-    const double launched = std::max(l.least * longest, l.step * longest + work / l.rate);
+    // FP32, two steps per launch; `one_step` passes take at least this long (the free surface 5.2 to 5.4 us up to
+    // 240,000 cells, an odd sub-sampling's Born adjoint 14 to 20), FP64 with one
+    constexpr Cost f32[] = {{2.6, 100e3, 3.5}, {2.7, 90e3, 3.55}, {4.5, 57e3, 4.5}, {2.5, 75e3, 3.6}, {5.5, 48e3, 5.5}};
+    constexpr double one_step[] = {5.0, 5.5, 6.0, 5.4, 8.0};
+    constexpr Cost f64[] = {{4.45, 48e3, 5.5}, {5.0, 35e3, 6.2}, {7.0, 21e3, 7.0}, {5.0, 38e3, 6.2}, {9.5, 13.5e3, 9.5}};
+    const int i = int(kind);
+    const Cost& l = (sizeof(T) == 4 ? f32 : f64)[i];
+    const double least = sizeof(T) == 4 && one_step_pass<T>(c, plan, shots, kind) ? one_step[i] : l.least;
+    const double launched = std::max(least * longest, l.step * longest + work / l.rate);
     if (res >= launched) groups.clear();
     return groups;
 }

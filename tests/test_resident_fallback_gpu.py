@@ -76,7 +76,9 @@ def test_launched_recompute_from_resident_checkpoints(dtype, sub, change):
     datd = [np.ascontiguousarray(s, dtype) for s in dat]
     rec = [np.zeros((rpos[GRID_OF_COMP[k]].size, nts), dtype) for k in range(5)]
     shot, keep = ctx.make_shot(mid, spos, rpos, srcd, rec)
+    before = ctx.resident_info()[0]
     h = ctx.fwi_forward([shot], segment)
+    assert ctx.resident_info()[0] == before + 2
     _check(rec, ref, dtype)
     if change == "given_up":
         ctx.set_persistent(0, 1)
@@ -97,7 +99,7 @@ def test_refused_launch_is_tried_again(shimmed, dtype):
     form, not the context's life; each call's data are right."""
     shim, capi = shimmed
     ctx = _shim_ctx(capi, dtype)
-    mid, g, med = _model(ctx, 139, 90, 101, 2, 41)
+    mid, g, med = _model(ctx, 500, 480, 101, 2, 41)
     rng = np.random.default_rng(42)
     shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, dtype, 10, 20)
 
@@ -130,7 +132,7 @@ def test_other_launch_errors_are_raised(shimmed):
     """An error that is no refusal reaches the caller; the context runs resident afterwards."""
     shim, capi = shimmed
     ctx = _shim_ctx(capi, np.float32)
-    mid, g, med = _model(ctx, 139, 90, 101, 2, 43)
+    mid, g, med = _model(ctx, 500, 480, 101, 2, 43)
     rng = np.random.default_rng(44)
     shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, np.float32, 10, 20)
     shim.shim_launches(LAUNCH_FAILURE, 1, 0)
@@ -147,7 +149,7 @@ def test_given_up_wait_is_not_paid_on_every_call():
     """After a call that gave up a wait, the next one does not try; then one in four, and so on."""
     ctx = _ctx(np.float32)
     ctx.set_persistent(0, 1)
-    mid, g, med = _model(ctx, 281, 301, 51, 2, 45)
+    mid, g, med = _model(ctx, 500, 480, 51, 2, 45)
     rng = np.random.default_rng(46)
     shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, np.float32, 10, 20)
     tries = []
@@ -202,7 +204,7 @@ def test_explicit_variant_keeps_launched_steps(dtype, sub, surface):
     FP32 passes that take two steps a launch have variants of their own, which stay automatic here."""
     ctx = _ctx(dtype)
     nts = 102 if sub == 3 else 201           # 303 fine steps are an odd count for the NL adjoint
-    mid, g, med = _model(ctx, 139, 90, nts, sub, 51, surface=surface)
+    mid, g, med = _model(ctx, 300, 700, nts, sub, 51, surface=surface)
     auto = _passes(ctx, mid, g, dtype)
     assert auto["nl_forward"] and (surface or all(auto.values())), auto
     ctx.set_variant(3)
@@ -218,7 +220,7 @@ def test_explicit_variant_keeps_launched_steps(dtype, sub, surface):
     ctx.close()
 
 
-@pytest.mark.parametrize("dtype,nz,nx", [(np.float32, 139, 90), (np.float64, 300, 500)])
+@pytest.mark.parametrize("dtype,nz,nx", [(np.float32, 300, 500), (np.float64, 300, 500)])
 def test_born_ring_on_a_full_card(shimmed, dtype, nz, nx):
     """The ring of the Born passes: the same bits whatever memory is free, kept where there is plenty, given back
     at the call's end where there is little and when another allocation needs it, and done without (launched

@@ -93,7 +93,7 @@ def test_free_surface_tiles(dtype, nz, nx, r):
 
 
 @pytest.mark.parametrize("dtype,nz,nx,r", [
-    (np.float32, 139, 90, 1), (np.float32, 281, 967, 2), (np.float32, 563, 1103, 3), (np.float32, 601, 1593, 4),
+    (np.float32, 500, 480, 1), (np.float32, 281, 967, 2), (np.float32, 563, 1103, 3), (np.float32, 601, 1593, 4),
     (np.float32, 683, 1503, 5), (np.float64, 139, 90, 1), (np.float64, 391, 1200, 2)])
 def test_adjoint_runs_resident(dtype, nz, nx, r):
     assert _r(nz, nx) == r
@@ -204,4 +204,25 @@ def test_born_batch_runs_resident():
     # at least two groups, whose receiver passes take two launches each, and the source pass
     assert after[0] - before[0] >= 1 + 2 * 2 and after[1:] == before[1:], (before, after)
     assert rel_l2(dm, ref) < GRAD_TOL[np.float32], rel_l2(dm, ref)
+    ctx.close()
+
+
+@pytest.mark.parametrize("dtype,nz,nx,nshot,nts,resident", [
+    (np.float32, 72, 24, 1, 51, True),       # one tile: no exchange
+    (np.float32, 72, 1500, 1, 101, True),    # one row of tiles
+    (np.float32, 139, 61, 1, 51, True),      # 12 tiles, two an XCD
+    (np.float32, 200, 200, 1, 120, False),   # 36 tiles that all trade across XCDs: launched steps are faster
+    (np.float32, 200, 200, 4, 120, True),    # four of them: most of a shot on one XCD
+    (np.float32, 500, 480, 1, 120, True),    # enough cells for a step of its own length
+    (np.float64, 200, 200, 1, 120, False), (np.float64, 200, 200, 4, 120, True), (np.float64, 280, 472, 1, 120, True)])
+def test_forward_takes_the_faster_form(dtype, nz, nx, nshot, nts, resident):
+    """The rule between resident and launched steps on small grids, either form against the oracle."""
+    ctx = _ctx(dtype)
+    mid, g, med = _model(ctx, nz, nx, nts, 2, nz + nx)
+    rng = np.random.default_rng(nz * nx + 15)
+    cases = [_forward_case(ctx, mid, g, med, rng, dtype, 10, 20) for _ in range(nshot)]
+    with _Resident(ctx, int(resident)):
+        ctx.nl_forward([c[0] for c in cases])
+    for _, _, rec, ref in cases:
+        _check(rec, ref, dtype)
     ctx.close()
