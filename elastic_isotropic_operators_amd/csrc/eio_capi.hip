@@ -1525,14 +1525,16 @@ ResShape res_shape(int nshot, int ntile, bool line) {
     return line || nshot >= 4 || ntile <= 8 * (sizeof(T) == 4 ? 2 : 3) ? ResShape::LINE : ResShape::GRID;
 }
 
-// The groups of a call that take the least time in all, or none when a shot does not fit the device.
+// The groups of a call that take the least time in all, or none when a shot does not fit the device; `per_launch`
+// fine steps a launch, with the set-up of each (0: a group's steps in one).
 // A group of a given R holds as many shots as fit (steps decrease along the plan, so fewer would
 // leave the later groups no less); over R and over the groups' ends the best split is exact: eight shots
 // of 280 x 472 take one launch of R = 5 (8.4 us an adjoint step), not six shots of R = 4 and two of
 // R = 2 (6.0 + 4.1), which do the most work per time first.
-constexpr double RES_SETUP_US = 60.0;   // of one launch, see res_choose
+constexpr double RES_SETUP_US = 60.0;      // of one launch, see res_choose
+constexpr double RES_SEGMENT_US = 100.0;   // of a launch between others
 template <typename T>
-std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) {
+std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
     const int n = int(plan.order.size()), RM = res_max_r<T>(kind);
     std::vector<ResGroup> best(n);
     std::vector<double> cost(n + 1, 0.0);
@@ -1552,7 +1554,9 @@ std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots
             }
             if (s1 == s0) continue;
             const double us = res_step_us<T>(kind, R, res_shape<T>(s1 - s0, nt, line));
-            const double t = RES_SETUP_US + us * plan.nsteps[s0] + cost[s1];
+            const int steps = plan.nsteps[s0];
+            const double setup = per_launch ? RES_SEGMENT_US * ((steps + per_launch - 1) / per_launch) : RES_SETUP_US;
+            const double t = setup + us * steps + cost[s1];
             if (t < cost[s0]) {
                 best[s0] = {s0, s1, R, 0, nt, us};
                 cost[s0] = t;
@@ -1789,11 +1793,10 @@ bool res_allowed(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) 
 // 280 x 472 in segments of 46 steps, 24.4 against 28.2.  Where an FP32 forward has 17 tiles or more and up to 90,000 cells
 // the launched form is the faster one (200 x 200: 1.05 against 0.97 at 238 steps, 3.7 against 3.5 at 1000); on fewer tiles
 // the two are within 5 % of one another, and one launch a call leaves the host free.
-constexpr double RES_SEGMENT_US = 100.0;
 template <typename T>
 std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
     if (!res_allowed<T>(c, plan, shots, kind)) return {};
-    std::vector<ResGroup> groups = res_groups<T>(c, plan, shots, kind);
+    std::vector<ResGroup> groups = res_groups<T>(c, plan, shots, kind, per_launch);
     double res = 0.0, work = 0.0;
     int longest = 0;
     for (const ResGroup& g : groups) {
@@ -2695,7 +2698,8 @@ void fwi_gradient(Ctx* c, int handle, int nshot, const eio_shot* shots, void* co
                                  c->stream));
     ResPlan rp;
     if (rres) {
-        rp.groups = res_groups<T>(c, make_plan<T>(c, nshot, shots, Op::FWI_GRAD, PlanKind::NONE), shots, ResKind::DEC);
+        rp.groups = res_groups<T>(c, make_plan<T>(c, nshot, shots, Op::FWI_GRAD, PlanKind::NONE), shots, ResKind::DEC,
+                                  std::min(f.L, f.nts - 1) * f.sub);
         if (rp.groups.empty()) throw EioError{EIO_ERR_STATE, "the device no longer takes the resident loop of this store"};
         if (!res_build(run, shots, rp)) {
             ResidentOff off(c);

@@ -226,3 +226,27 @@ def test_forward_takes_the_faster_form(dtype, nz, nx, nshot, nts, resident):
     for _, _, rec, ref in cases:
         _check(rec, ref, dtype)
     ctx.close()
+
+
+def test_born_groups_pay_for_every_launch():
+    """Sixteen small shots: the receiver pass takes one group of R = 4, whose three launches of 32 intervals are set
+    up three times, not two groups of R = 2, which are six and slower for it."""
+    ctx = _ctx(np.float32)
+    nz, nx, nts, sub = 92, 434, 70, 4
+    mid, g, med = _model(ctx, nz, nx, nts, sub, 73)
+    rng = np.random.default_rng(74)
+    shots, keeps, ref = [], [], 0.0
+    for i in range(16):
+        spos, rpos = _positions(rng, g, 4), _positions(rng, g, 20)
+        src = [O.time_interp(s, g.dts, sub) for s in random_traces(rng, spos, nts, np.float64)]
+        dat = random_traces(rng, rpos, nts, np.float64)
+        ref = ref + O.born_adj_reg(g, med, spos, src, rpos, dat, np.float64)
+        shot, keep = ctx.make_shot(mid, spos, rpos, [np.ascontiguousarray(s, np.float32) for s in src],
+                                   [np.ascontiguousarray(s, np.float32) for s in dat])
+        shots.append(shot)
+        keeps.append(keep)
+    dm = np.zeros((5, nx, nz), np.float32)
+    with _Resident(ctx, 1 + 3):              # the source pass in one launch of R = 4
+        ctx.born_adjoint(shots, dm)
+    assert rel_l2(dm, ref) < GRAD_TOL[np.float32], rel_l2(dm, ref)
+    ctx.close()
