@@ -167,24 +167,16 @@ __device__ __forceinline__ T damp_at(const ShotDev<T>& S, int iz, int ix) {
 constexpr int SURF = 2 * FAT;
 
 template <typename T>
-__device__ __forceinline__ void fs_map_stress(T* szz, T* sxz) {
+__device__ __forceinline__ void fs_map_col(T* vx, T* vz, T* szz, T* sxz) {
     szz[SURF] = T(0);
 #pragma unroll
     for (int k = 0; k < 4; ++k) szz[SURF - 1 - k] = -szz[SURF + 1 + k];
 #pragma unroll
     for (int k = 0; k < 4; ++k) sxz[SURF - k] = -sxz[SURF + 1 + k];
-}
-template <typename T>
-__device__ __forceinline__ void fs_map_velocity(T* vx, T* vz) {
 #pragma unroll
     for (int r = SURF - 4; r < SURF; ++r) vx[r] = T(0);
 #pragma unroll
     for (int r = SURF - 4; r <= SURF; ++r) vz[r] = T(0);
-}
-template <typename T>
-__device__ __forceinline__ void fs_map_col(T* vx, T* vz, T* szz, T* sxz) {
-    fs_map_stress<T>(szz, sxz);
-    fs_map_velocity<T>(vx, vz);
 }
 template <typename T>
 __device__ __forceinline__ void fs_map_col_transpose(T* vx, T* vz, T* szz, T* sxz) {
