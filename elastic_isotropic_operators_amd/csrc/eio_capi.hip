@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -225,7 +226,8 @@ struct Ctx {
     long long res_launches = 0, res_given_up = 0, res_refused = 0;   // launches; passes that gave up; refusals
     int res_error = 0;         // HIP error of the last refusal
     bool res_failed = false;   // a resident pass of this call gave up or was refused
-    int res_skip = 0, res_backoff = 0;   // calls left that do not try resident loops, and how many after the last failure
+    int res_failures = 0;      // such calls in a row (at most 5)
+    std::chrono::steady_clock::time_point res_retry{};   // calls before it do not try resident loops
     int ncu = 0;               // compute units of the device
     std::map<int, FwiStore> fwi;
     int next_fwi = 1;
@@ -1723,21 +1725,28 @@ inline bool res_aborted(Ctx* c, const ResPlan& rp) {
 }
 
 // One call of an entry point that may run resident loops.  After a call that gave up a wait or was refused
-// a launch, the next 1, 3, 7, .. RES_BACKOFF calls do not try (a wait of the default limit is 2^20 polls
-// of memory before it is given up; a queue that another process holds may stay held); a call that runs
-// resident to its end resets the count.
-constexpr int RES_BACKOFF = 63;
+// a launch, the context does not try for 32 times what that call took, at least a quarter of a second, and
+// twice as long for each further failure in a row: trying costs at most 3 % of the time and soon 0.1 % (a refused
+// launch takes 37 ms before it returns, a wait of the default limit 2^20 polls of memory), and a queue that is free
+// again is used again.  A call that runs resident to its end ends the row.
 struct ResCall {
+    using clock = std::chrono::steady_clock;
     Ctx* c;
     long long before;
+    clock::time_point begin = clock::now();
     explicit ResCall(Ctx* c_) : c(c_), before(c_->res_launches) {
         c->res_failed = false;
-        c->resident = c->res_skip == 0;
-        if (c->res_skip > 0) --c->res_skip;
+        c->resident = begin >= c->res_retry;
     }
     ~ResCall() {
-        if (c->res_failed) c->res_skip = c->res_backoff = std::min(2 * c->res_backoff + 1, RES_BACKOFF);
-        else if (c->res_launches > before) c->res_backoff = 0;
+        if (c->res_failed) {
+            const clock::time_point end = clock::now();
+            const clock::duration pause = std::max<clock::duration>(32 * (end - begin), std::chrono::milliseconds(250));
+            c->res_retry = end + pause * (1 << c->res_failures);
+            c->res_failures = std::min(c->res_failures + 1, 5);
+        } else if (c->res_launches > before) {
+            c->res_failures = 0;
+        }
         c->resident = true;
     }
 };

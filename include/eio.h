@@ -121,8 +121,8 @@ int eio_ctx_set_variant(eio_ctx* ctx, int variant);
  * launches for the NL forward, eio_ctx_last_shot_groups the groups.  Graphs, the persistent mode, explicit
  * variants of the launched form a pass would take, saved wavefields, snapshots, learned boundaries and the no-allocation call keep to launched
  * steps.  A call whose device refuses a cooperative launch (one process at a time holds a device's
- * cooperative queue) or that gives up a wait runs launched instead, and the context's next 1, 3, 7, .. 63
- * calls, one count per failure in a row, do not try (eio_ctx_resident_info).
+ * cooperative queue) or that gives up a wait runs launched instead, and the context does not try again for 32
+ * times what that call took, at least 0.25 s, doubled for each failure in a row (eio_ctx_resident_info).
  * It applies to the NL forward (without
  * saved wavefield, free surface or learned boundary), the whole-record FWI forward and the
  * Born source and scattered passes.  No counterpart in the reference. */

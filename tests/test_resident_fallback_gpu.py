@@ -7,6 +7,8 @@ import importlib.util
 import os
 import shutil
 import subprocess
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -103,28 +105,36 @@ def test_refused_launch_is_tried_again(shimmed, dtype):
     rng = np.random.default_rng(42)
     shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, dtype, 10, 20)
 
-    def forms(n):
-        out = ""
-        for _ in range(n):
-            for r in rec:
-                r[...] = 7
-            before = ctx.resident_info()[0]
-            ctx.nl_forward([shot])
-            resident = ctx.resident_info()[0] > before
-            assert (ctx.last_timing()[1] == 1) == resident
-            _check(rec, ref, dtype)
-            out += "RL"[not resident]
-        return out
+    def form():
+        for r in rec:
+            r[...] = 7
+        before = ctx.resident_info()[0]
+        ctx.nl_forward([shot])
+        resident = ctx.resident_info()[0] > before
+        assert (ctx.last_timing()[1] == 1) == resident
+        _check(rec, ref, dtype)
+        return "RL"[not resident]
 
-    assert forms(2) == "RR"
-    shim.shim_launches(ILLEGAL_STATE, 1, 0)
-    assert forms(4) == "LLRR"
-    assert ctx.resident_info()[1:] == (0, 1, ILLEGAL_STATE)
-    shim.shim_launches(ILLEGAL_STATE, 2, 0)          # and the next try again: 1, then 3 calls without one
-    assert forms(8) == "LLLLLLRR"
-    assert ctx.resident_info()[1:] == (0, 3, ILLEGAL_STATE)
-    shim.shim_launches(ILLEGAL_STATE, 1, 0)          # a call that ran resident has reset the count
-    assert forms(3) == "LLR"
+    def refused(launches, pause):
+        """Refuses the next launches; the calls of the next `pause` seconds do not try, those after it do."""
+        shim.shim_launches(ILLEGAL_STATE, launches, 0)
+        for _ in range(launches):
+            n = ctx.resident_info()[2]
+            begin = time.monotonic()
+            assert form() == "L" and ctx.resident_info()[1:] == (0, n + 1, ILLEGAL_STATE)
+            again = form()
+            if time.monotonic() < begin + pause:
+                assert again == "L" and ctx.resident_info()[2] == n + 1
+            time.sleep(pause + 32 * (time.monotonic() - begin))
+            pause *= 2
+
+    assert form() + form() == "RR"
+    refused(1, 0.25)
+    assert form() + form() == "RR"
+    refused(2, 0.25)              # twice in a row: the second pause is twice as long
+    assert form() == "R"
+    refused(1, 0.25)              # a call that ran resident has ended the row
+    assert form() == "R"
     ctx.close()
 
 
@@ -146,19 +156,22 @@ def test_other_launch_errors_are_raised(shimmed):
 
 
 def test_given_up_wait_is_not_paid_on_every_call():
-    """After a call that gave up a wait, the next one does not try; then one in four, and so on."""
+    """After a call that gave up a wait, those of the next quarter of a second do not try."""
     ctx = _ctx(np.float32)
     ctx.set_persistent(0, 1)
     mid, g, med = _model(ctx, 500, 480, 51, 2, 45)
     rng = np.random.default_rng(46)
     shot, keep, rec, ref = _forward_case(ctx, mid, g, med, rng, np.float32, 10, 20)
-    tries = []
-    for _ in range(8):
-        before = ctx.resident_info()[1]
+    for given_up in (1, 2):
+        begin = time.monotonic()
         ctx.nl_forward([shot])
-        tries.append(ctx.resident_info()[1] - before)
+        assert ctx.resident_info()[1] == given_up
         _check(rec, ref, np.float32)
-    assert tries == [1, 0, 1, 0, 0, 0, 1, 0]
+        ctx.nl_forward([shot])
+        if time.monotonic() < begin + 0.25:
+            assert ctx.resident_info()[1] == given_up
+        _check(rec, ref, np.float32)
+        time.sleep(0.25 + 32 * (time.monotonic() - begin))
     ctx.close()
 
 
@@ -291,9 +304,15 @@ def test_refused_in_the_middle_of_a_pass(shimmed, dtype, nz, nx):
     in the outputs, the ring and the record is made again, launched."""
     shim, capi = shimmed
     nts, sub, segment = 70, 3, 23
-    ctx = _shim_ctx(capi, dtype)
-    mid, g, med = _model(ctx, nz, nx, nts, sub, 81)
     rng = np.random.default_rng(82)
+    g = None
+
+    def context():
+        ctx = _shim_ctx(capi, dtype)
+        return (ctx,) + _model(ctx, nz, nx, nts, sub, 81)
+
+    ctx, mid, g, med = context()
+    ctx.close()
     spos, rpos = _positions(rng, g, 10), _positions(rng, g, 80)
     src = random_traces(rng, spos, nts, np.float64)
     fine = [O.time_interp(s, g.dts, sub) for s in src]
@@ -304,35 +323,24 @@ def test_refused_in_the_middle_of_a_pass(shimmed, dtype, nz, nx):
     ref_lin = O.born_fwd_reg(g, med, spos, fine, dmod, rpos, np.float64)
     srcd, fined, datd = ([np.ascontiguousarray(t, dtype) for t in tr] for tr in (src, fine, dat))
 
-    def fresh_ctx_state():
-        while ctx.resident_info()[0] == forms[0]:      # the calls that do not try after a failure
-            shot, keep = ctx.make_shot(mid, spos, rpos, srcd, [np.zeros_like(t) for t in datd])
-            ctx.nl_forward([shot])
-        forms[0] = ctx.resident_info()[0]
-
-    forms = [-1]
-    refusals = 0
-    for after in (0, 1, 2, 3):
-        forms[0] = ctx.resident_info()[0]
-        fresh_ctx_state()
+    def born_adjoint(ctx, mid, after):
         shim.shim_launches(ILLEGAL_STATE, 1, after)
         dm = np.zeros((5, nx, nz), dtype)
         shot, keep = ctx.make_shot(mid, spos, rpos, fined, datd)
         ctx.born_adjoint([shot], dm)
         assert rel_l2(dm, ref_dm) < GRAD_TOL[dtype], (after, rel_l2(dm, ref_dm))
 
-        forms[0] = ctx.resident_info()[0]
-        fresh_ctx_state()
+    def born_forward(ctx, mid, after):
         shim.shim_launches(ILLEGAL_STATE, 1, after)
         rec = [np.full_like(t, 7) for t in datd]
         shot, keep = ctx.make_shot(mid, spos, rpos, fined, rec)
         ctx.born_forward([shot], np.ascontiguousarray(dmod, dtype))
         _check(rec, ref_lin, dtype)
 
-        forms[0] = ctx.resident_info()[0]
-        fresh_ctx_state()
+    def fwi_gradient(ctx, mid, after):
         shot, keep = ctx.make_shot(mid, spos, rpos, srcd, [np.zeros_like(t) for t in datd])
         h = ctx.fwi_forward([shot], segment)
+        assert ctx.resident_info()[0] == 3
         shim.shim_launches(ILLEGAL_STATE, 1, after)
         for _ in range(2):
             dm = np.zeros((5, nx, nz), dtype)
@@ -340,6 +348,44 @@ def test_refused_in_the_middle_of_a_pass(shimmed, dtype, nz, nx):
             ctx.fwi_gradient(h, [shot], dm)
             assert rel_l2(dm, ref_dm) < GRAD_TOL[dtype], (after, rel_l2(dm, ref_dm))
         ctx.fwi_release(h)
-        refusals += 3
-        assert ctx.resident_info()[2] == refusals
-    ctx.close()
+
+    for call in (born_adjoint, born_forward, fwi_gradient):
+        for after in (0, 1, 2, 3):
+            ctx, mid, _, _ = context()
+            call(ctx, mid, after)
+            assert ctx.resident_info()[1:] == (0, 1, ILLEGAL_STATE), (call, after)
+            ctx.close()
+
+
+def test_two_threads_run_resident():
+    """Two contexts on two threads of one process at once, each on its own stream: both resident, their launches one
+    after the other on the device, with the data of each alone."""
+    def case(seed):
+        ctx = _ctx(np.float32)
+        mid, g, med = _model(ctx, 500, 480, 101, 2, seed)
+        rng = np.random.default_rng(seed)
+        return (ctx,) + _forward_case(ctx, mid, g, med, rng, np.float32, 10, 20)
+
+    cases = [case(91), case(92)]
+    alone = []
+    for ctx, shot, keep, rec, ref in cases:
+        ctx.nl_forward([shot])
+        _check(rec, ref, np.float32)
+        alone.append([r.copy() for r in rec])
+    ready = threading.Barrier(2)
+
+    def run(case):
+        ctx, shot, keep, rec, ref = case
+        ready.wait()
+        for _ in range(20):
+            ctx.nl_forward([shot])
+
+    threads = [threading.Thread(target=run, args=(c,)) for c in cases]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for (ctx, shot, keep, rec, ref), first in zip(cases, alone):
+        assert ctx.resident_info() == (21, 0, 0, 0)
+        assert all(np.array_equal(a, b) for a, b in zip(rec, first))
+        ctx.close()
