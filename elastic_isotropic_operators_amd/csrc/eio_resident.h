@@ -3,7 +3,7 @@
 //
 // The launched kernels (eio_kernels.h, eio_step2.h) read two state levels and the media and
 // write one or two levels per launch: 50-80 B per cell-update through the caches, and one
-// launch per one or two fine steps.  A shot of up to about 1.3 M cells fits on the chip: the
+// launch per one or two fine steps.  A shot of up to 1.57 M cells (FP64: 0.5 M) fits on the chip: the
 // current level in LDS (20 B per FP32 cell of the 160 KB per CU), the older level and the
 // media in registers.  Here ONE cooperative launch runs a whole loop: workgroup b owns one
 // tile of 64 x TX cells for every fine step, and only the 4-cell halos move, through inboxes in
@@ -27,19 +27,20 @@
 // the waves (two each), the rows along z belong to the wave of their columns.
 //
 // Measured (one launch for the whole loop, FP32): 280 x 472 with R = 1, 3.4 us per fine step
-// against 4.2 with two steps per launch; two shots of 520 x 1000 with R = 4, 5.65 us (181
+// against 4.0 with two steps per launch; two shots of 520 x 1000 with R = 4, 5.65 us (181
 // GCell/s) against 11.2 (92 GCell/s); FP64, two shots of 280 x 472 with R = 2, 6.2 us against 12.2
 // with one step per launch.  At R = 4 a step is 14,000 cycles: 1400 the x derivatives, 4700 the z
 // derivatives and the update (VALU 383 instructions a wave, LDS 44 words a cell: both about 6500
 // cycles of the step when nothing waits), 2000 the staging of the new level, the rest barriers
 // and the part of the exchange that the x derivatives do not cover.  Stores that cross the
-// fabric cap the exchange at about 3 TB/s; neighbours on the same XCD trade through its L2
+// fabric cap the exchange at about 3 TB/s (counters of R = 4: 63 % of the wave cycles wait, on the exchange
+// and its barriers, 13 % for an issue slot, 24 % issue); neighbours on the same XCD trade through its L2
 // (plain stores), which took R = 1 from 4.6 to 3.5 us and R = 4 from 6.4 to 5.85.
 //
 // Waiting.  All workgroups are co-resident (cooperative launch, at most one workgroup per CU
 // by LDS); every wait is bounded by spin_limit polls, after which the workgroup sets *abort
 // and leaves, every other workgroup leaves at its next wait, and the host repeats the call with
-// the launched kernels.
+// the launched kernels (and does not try again for a while).
 #pragma once
 #include "eio_kernels.h"
 
@@ -154,9 +155,10 @@ __device__ __forceinline__ T dp_l(const LdsT<T>* q, const T* c) {
     return taps<T>(c, q[5] - q[4], q[6] - q[3], q[7] - q[2], q[8] - q[1]);
 }
 
-// The updates' sums, rounded as the launched loop of the same calls rounds them, so that a call gives
-// the same bits in either form: with fused operations spelled out, since which product the compiler fuses
-// changes with the code around it.  PAIR (FP32): as k_step2_fwd's streamed stage, variant 12 (d*o first for
+// The updates' sums of a forward loop, rounded as the launched loop of the same calls rounds them, so that an NL
+// forward gives the same bits in either form: with fused operations spelled out, since which product the compiler
+// fuses changes with the code around it.  The free surface's sums, the secondary sources and the adjoint loops are left
+// to the compiler: their two forms agree to rounding (an FP32 Born gradient to 5e-7 relative L2).  PAIR (FP32): as k_step2_fwd's streamed stage, variant 12 (d*o first for
 // the velocities and, in the second step of a pair, for sxz); else as k_step_fwd.
 template <typename T>
 __device__ __forceinline__ T fma_t(T a, T b, T c) {
