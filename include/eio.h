@@ -81,7 +81,8 @@ int eio_ctx_release_workspace(eio_ctx* ctx);
 int eio_ctx_set_stream(eio_ctx* ctx, void* hip_stream);
 /* Timing of the last propagation call, from HIP events on the context stream:
  * total device time [ms], number of fused stencil launches, and the mean time of one
- * stencil launch [ms] measured over a bracketed run of them. */
+ * stencil launch [ms] measured over a bracketed run of them.  An NL forward counts its launches (resident: the
+ * cooperative ones); an adjoint, Born or FWI call counts its fine steps, however many a launch takes. */
 int eio_ctx_last_timing(eio_ctx* ctx, double* total_ms, long long* n_step_launches,
                         double* step_ms);
 /* 0 = launch each fine step (default); 1 = run each call's time loop from an executable
