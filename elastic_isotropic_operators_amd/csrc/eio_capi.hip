@@ -1802,8 +1802,13 @@ bool res_allowed(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) 
 // 280 x 472 in segments of 46 steps, 24.4 against 28.2.  Where an FP32 forward has 17 tiles or more and up to 90,000 cells
 // the launched form is the faster one (200 x 200: 1.05 against 0.97 at 238 steps, 3.7 against 3.5 at 1000); on fewer tiles
 // the two are within 5 % of one another, and one launch a call leaves the host free.
+// `between`: the pass runs beside resident ones (a Born source pass before them, a recompute between the
+// segments of a receiver pass), where a launched one takes this much longer a step.  Born adjoint, FP32, 139 x 90: 2.00 ms a
+// call with the source pass resident against 1.99 launched at 192 fine steps, 6.62 against 6.93 at 768; FWI forward and
+// gradient of two 328 x 120 in segments of 200 steps, 6.8 against 7.4.  With every pass launched it is not so.
+constexpr double RES_BETWEEN_US = 0.7;
 template <typename T>
-std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0) {
+std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind, int per_launch = 0, bool between = false) {
     if (!res_allowed<T>(c, plan, shots, kind)) return {};
     std::vector<ResGroup> groups = res_groups<T>(c, plan, shots, kind, per_launch);
     double res = 0.0, work = 0.0;
@@ -1827,7 +1832,7 @@ std::vector<ResGroup> res_choose(Ctx* c, const Plan& plan, const eio_shot* shots
     const int i = int(kind);
     const Cost& l = (sizeof(T) == 4 ? f32 : f64)[i];
     const double least = sizeof(T) == 4 && one_step_pass<T>(c, plan, shots, kind) ? one_step[i] : l.least;
-    const double launched = std::max(least * longest, l.step * longest + work / l.rate);
+    const double launched = std::max(least * longest, l.step * longest + work / l.rate) + (between ? RES_BETWEEN_US * longest : 0.0);
     if (res >= launched) groups.clear();
     return groups;
 }
@@ -2210,22 +2215,29 @@ void born_source_pass(Run<T>& run, int ntile, int kmax) {
     for (int k = 0; k < kmax; ++k) launch_fwd<T, eio::M_BSRC>(run, ntile, k, 0, 0, -1);
 }
 
-// The Born source pass with every shot resident; false when a shot does not fit or a wait was
+// Coarse samples of one launch of a resident pass that trades them with k_imaging_many through a ring, and its fine
+// steps.
+constexpr int RES_RING = 32;
+template <typename T>
+int ring_steps(const Run<T>& run) {
+    return std::min(RES_RING, run.sd[0].nts - 1) * run.sd[0].sub;
+}
+
+// The Born source pass with every shot resident (`other`: the pass that follows it); false when a shot does not fit or a wait was
 // given up (the launched pass then overwrites the record).
 template <typename T>
-bool born_source_resident(Run<T>& run, int nshot, const eio_shot* shots) {
+bool born_source_resident(Run<T>& run, int nshot, const eio_shot* shots, ResKind other) {
     Ctx* c = run.c;
     ResPlan rp;
-    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::DEC);
+    const bool between = !res_choose<T>(c, run.plan, shots, other, ring_steps(run)).empty();
+    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::DEC, 0, between);
     if (rp.groups.empty() || !res_build(run, shots, rp)) return false;
     for (const ResGroup& g : rp.groups)
         res_launch_fwd<T, eio::M_BSRC>(run, rp, g, 0, run.plan.nsteps[g.s0], true, false, 0, -1);
     return !res_aborted(c, rp);
 }
 
-// Coarse samples of one launch of a resident pass that trades them with k_imaging_many through a ring,
-// that kernel's tiles, and the shot table with the ring.
-constexpr int RES_RING = 32;
+// The ring of such a pass, the tiles of k_imaging_many, and the shot table with the ring.
 template <typename T>
 struct ResRing {
     static constexpr int R = 2, WX = sizeof(T) == 8 ? 4 : 8, TX = R * WX;
@@ -2320,7 +2332,7 @@ bool scattered_pass_resident(Run<T>& run, int nshot, const eio_shot* shots) {
     const int nts = run.sd[0].nts, sub = run.sd[0].sub;
     ResPlan rp;
     ResRing<T> ring;
-    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::SCAT, std::min(RES_RING, nts - 1) * sub);
+    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::SCAT, ring_steps(run));
     if (rp.groups.empty() || !ring_build(run, rp, ring) || !res_build(run, shots, rp, "resa_")) return false;
     for (const ResGroup& g : rp.groups)
         for (int a = 0; a < nts - 1; a += ring.K) {   // intervals a .. b-1 use the samples a .. b
@@ -2359,7 +2371,7 @@ void receiver_pass_resident(Run<T>& run, const ResPlan& rp, const ResRing<T>& ri
 template <typename T>
 bool receiver_pass_build(Run<T>& run, int nshot, const eio_shot* shots, ResPlan& rp, ResRing<T>& ring, bool one_group) {
     Ctx* c = run.c;
-    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::BADJ, std::min(RES_RING, run.sd[0].nts - 1) * run.sd[0].sub);
+    rp.groups = res_choose<T>(c, run.plan, shots, ResKind::BADJ, ring_steps(run));
     if (rp.groups.empty() || (one_group && rp.groups.size() > 1) || !ring_build(run, rp, ring)) return false;
     return res_build(run, shots, rp, "resa_");
 }
@@ -2386,7 +2398,7 @@ void born_forward(Ctx* c, int nshot, const eio_shot* shots, const void* const dm
     timing_begin<T>(c);
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
     run_loop(c, [&]() {
-        if (!born_source_resident(run, nshot, shots)) born_source_pass(run, ntile, kmax);
+        if (!born_source_resident(run, nshot, shots, ResKind::SCAT)) born_source_pass(run, ntile, kmax);
         if (scattered_pass_resident(run, nshot, shots)) return;
         // scattered pass restarts from a zero state (BornElasticGpuFunctions.cu:773-774)
         for (int oi = 0; oi < nshot; ++oi) {
@@ -2427,7 +2439,7 @@ void born_adjoint(Ctx* c, int nshot, const eio_shot* shots, void* const dm[5], i
     timing_begin<T>(c);
     EIO_CHECK_HIP(hipEventRecord(c->ev[2], c->stream));
     run_loop(c, [&]() {
-        if (!born_source_resident(run, nshot, shots)) born_source_pass(run, ntile, kmax);
+        if (!born_source_resident(run, nshot, shots, ResKind::BADJ)) born_source_pass(run, ntile, kmax);
         ResPlan rp;
         ResRing<T> ring;
         if (receiver_pass_build(run, nshot, shots, rp, ring, false)) {
@@ -2539,8 +2551,11 @@ inline int seg_end(const FwiStore& f, int j) { return std::min((j + 1) * f.L, f.
 template <typename T>
 bool fwi_forward_resident(Ctx* c, int nshot, const eio_shot* shots, int flags, FwiStore& f) {
     ResPlan rp;
-    rp.groups = res_choose<T>(c, make_plan<T>(c, nshot, shots, Op::FWI_FWD, PlanKind::NONE), shots, ResKind::DEC,
-                              std::min(f.L, f.nts - 1) * f.sub);
+    // the store's form is that of its recompute, which runs beside the gradient's receiver pass
+    const Plan plan = make_plan<T>(c, nshot, shots, Op::FWI_FWD, PlanKind::NONE);
+    const std::vector<ResGroup> rec = res_choose<T>(c, plan, shots, ResKind::BADJ, std::min(RES_RING, f.nts - 1) * f.sub);
+    rp.groups = res_choose<T>(c, plan, shots, ResKind::DEC, std::min(f.L, f.nts - 1) * f.sub,
+                              rec.size() == 1 || (f.nseg == 1 && !rec.empty()));
     if (rp.groups.empty()) return false;
     Run<T> run = prepare<T>(c, nshot, shots, Op::FWI_FWD, flags, nullptr, static_cast<T*>(f.ring), f.wcap, false, false,
                             false, false, false, f.nseg > 1 ? 2 : 1);

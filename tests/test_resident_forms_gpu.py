@@ -250,3 +250,30 @@ def test_born_groups_pay_for_every_launch():
         ctx.born_adjoint(shots, dm)
     assert rel_l2(dm, ref) < GRAD_TOL[np.float32], rel_l2(dm, ref)
     ctx.close()
+
+
+def test_born_source_pass_takes_the_form_of_the_others():
+    """One shot of 200 x 200: the receiver pass of the Born adjoint is resident and so is the source pass beside it; the
+    scattered pass of the Born forward is launched (intervals of 64 steps) and so is its source pass."""
+    ctx = _ctx(np.float32)
+    nz, nx, nts, sub = 200, 200, 150, 2
+    mid, g, med = _model(ctx, nz, nx, nts, sub, 75)
+    rng = np.random.default_rng(76)
+    spos, rpos = _positions(rng, g, 10), _positions(rng, g, 60)
+    src = [O.time_interp(s, g.dts, sub) for s in random_traces(rng, spos, nts, np.float64)]
+    dat = random_traces(rng, rpos, nts, np.float64)
+    dmod = np.zeros((5, nx, nz))
+    dmod[:, 4:-4, 4:-4] = rng.standard_normal((5, nx - 8, nz - 8)) * np.abs(med).reshape(5, -1).max(1)[:, None, None]
+    srcd, datd = [np.ascontiguousarray(s, np.float32) for s in src], [np.ascontiguousarray(s, np.float32) for s in dat]
+    dm = np.zeros((5, nx, nz), np.float32)
+    shot, keep = ctx.make_shot(mid, spos, rpos, srcd, datd)
+    with _Resident(ctx, 1 + 5):
+        ctx.born_adjoint([shot], dm)
+    ref = O.born_adj_reg(g, med, spos, src, rpos, dat, np.float64)
+    assert rel_l2(dm, ref) < GRAD_TOL[np.float32], rel_l2(dm, ref)
+    rec = [np.zeros_like(d) for d in datd]
+    shot, keep = ctx.make_shot(mid, spos, rpos, srcd, rec)
+    with _Resident(ctx, 0):
+        ctx.born_forward([shot], np.ascontiguousarray(dmod, np.float32))
+    _check(rec, O.born_fwd_reg(g, med, spos, src, dmod, rpos, np.float64), np.float32)
+    ctx.close()
