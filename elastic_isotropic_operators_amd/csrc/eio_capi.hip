@@ -1503,28 +1503,33 @@ constexpr int res_max_r(ResKind k) {
 // Measured time of one fine step of a launch with R columns per wave [us] (the halo exchange and the
 // barriers are about 2.5 us of it, so wide tiles do the most work per time, and narrow ones finish a call that
 // cannot fill the device soonest); the Born passes that trade coarse samples with the imaging include its time.
-// At R = 1 the exchange is all there is, and a step follows what the tiles trade over: nothing (each shot one
-// tile), one row or column of tiles or shots that mostly lie on one XCD each, or both ways across XCDs.
-enum class ResShape { TILE, LINE, GRID };
+// At R = 1 the exchange is all there is, and a step follows what the tiles trade over: nothing (TILE: each shot one
+// tile), one row or column of tiles or few of them (LINE), runs of tiles that share an XCD (RUNS), or both ways across XCDs
+// (GRID).
+enum class ResShape { TILE, LINE, RUNS, GRID };
 template <typename T>
 double res_step_us(ResKind k, int R, ResShape shape) {
     constexpr bool F32 = sizeof(T) == 4;
-    // R = 1: TILE, LINE, GRID
-    constexpr double one32[][3] = {{1.95, 2.85, 3.5}, {2.25, 3.3, 3.7}, {3.9, 3.9, 3.9}, {2.1, 2.9, 3.5}, {3.9, 3.9, 3.9}};
-    constexpr double one64[][3] = {{2.95, 4.8, 5.35}, {3.4, 5.1, 5.7}, {7.1, 7.1, 7.1}, {3.05, 4.7, 5.3}, {6.9, 6.9, 6.9}};
+    // R = 1: TILE, LINE, RUNS, GRID
+    constexpr double one32[][4] = {
+        {1.95, 2.85, 3.05, 3.5}, {2.25, 3.3, 3.45, 3.7}, {3.9, 3.9, 3.9, 3.9}, {2.1, 2.9, 3.1, 3.5}, {3.9, 3.9, 3.9, 3.9}};
+    constexpr double one64[][4] = {
+        {2.95, 4.8, 5.05, 5.35}, {3.4, 5.1, 5.4, 5.7}, {7.1, 7.1, 7.1, 7.1}, {3.05, 4.7, 5.0, 5.3}, {6.9, 6.9, 6.9, 6.9}};
     // R = 2 and wider
     constexpr double wide32[][5] = {{3.85, 5.05, 5.65, 7.0, 8.7}, {4.4, 5.7, 6.3, 8.8}, {4.9, 7.2, 11.8}, {4.1, 5.35, 6.0, 8.4}, {5.0, 7.0, 10.7}};
     constexpr double two64[] = {6.4, 8.0, 19.0, 8.0, 14.0};
     if (R == 1) return (F32 ? one32 : one64)[int(k)][int(shape)];
     return F32 ? wide32[int(k)][R - 2] : two64[int(k)];
 }
-// The shots of a launch of R = 1.  Tiles go to the eight XCDs in runs of consecutive ones, so that the shots of
-// a launch of four or more are cut once or not at all; up to two tiles an XCD (FP64: three) no tile trades
-// with more than a few others.
+// The shots of a launch of R = 1.  Tiles go to the eight XCDs in runs of consecutive ones, column by column: the shots of
+// a launch of four or more are cut once or not at all, and runs of whole columns (`nbz` tiles each, 0: of several heights)
+// trade across XCDs along x only (an adjoint step of two 200 x 200, nine tiles an XCD, three columns: 2.9 us; one, four and a
+// half tiles: 3.6); up to three tiles an XCD trade with a few others only.
 template <typename T>
-ResShape res_shape(int nshot, int ntile, bool line) {
+ResShape res_shape(int nshot, int ntile, bool line, int nbz) {
     if (ntile == nshot) return ResShape::TILE;
-    return line || nshot >= 4 || ntile <= 8 * (sizeof(T) == 4 ? 2 : 3) ? ResShape::LINE : ResShape::GRID;
+    if (line || ntile <= 8 * (sizeof(T) == 4 ? 2 : 3)) return ResShape::LINE;
+    return nshot >= 4 || ntile <= 24 || (nbz > 0 && ntile % (8 * nbz) == 0) ? ResShape::RUNS : ResShape::GRID;
 }
 
 // The groups of a call that take the least time in all, or none when a shot does not fit the device; `per_launch`
@@ -1544,18 +1549,20 @@ std::vector<ResGroup> res_groups(Ctx* c, const Plan& plan, const eio_shot* shots
         best[s0] = ResGroup{s0, s0, 0, 0, 0, 0.0};
         cost[s0] = 1e30;
         for (int R = 1; R <= RM; ++R) {
-            int nt = 0, s1 = s0;
+            int nt = 0, s1 = s0, nbz = -1;
             bool line = true;
             while (s1 < n) {
                 const ModelBase& m = get_model(c, shots[plan.order[s1]].model);
                 const int k = res_tiles(m, R);
                 if (nt + k > c->ncu) break;
                 nt += k;
-                line = line && (m.g.nz - 2 * eio::FAT <= eio::TZ || m.g.nx - 2 * eio::FAT <= RES_WX);
+                const int h = (m.g.nz - 2 * eio::FAT + eio::TZ - 1) / eio::TZ;
+                nbz = nbz < 0 || nbz == h ? h : 0;
+                line = line && (h == 1 || m.g.nx - 2 * eio::FAT <= RES_WX);
                 ++s1;
             }
             if (s1 == s0) continue;
-            const double us = res_step_us<T>(kind, R, res_shape<T>(s1 - s0, nt, line));
+            const double us = res_step_us<T>(kind, R, res_shape<T>(s1 - s0, nt, line, nbz));
             const int steps = plan.nsteps[s0];
             const double setup = per_launch ? RES_SEGMENT_US * ((steps + per_launch - 1) / per_launch) : RES_SETUP_US;
             const double t = setup + us * steps + cost[s1];
@@ -1799,9 +1806,9 @@ bool res_allowed(Ctx* c, const Plan& plan, const eio_shot* shots, ResKind kind) 
 //   FP64, 280 x 472   6.9   5.3     8.2   5.15   21.6  13.3    26.5  13.0
 // Whole calls, resident against launched: 280 x 472, 0.60 ms both at 100 fine steps, 0.78 against 0.84 at 160;
 // 600 x 1592, 0.26 against 0.25 at 10, 0.31 against 0.35 at 18; a checkpointed forward and gradient of four shots of
-// 280 x 472 in segments of 46 steps, 24.4 against 28.2.  Where an FP32 forward has 17 tiles or more and up to 90,000 cells
-// the launched form is the faster one (200 x 200: 1.05 against 0.97 at 238 steps, 3.7 against 3.5 at 1000); on fewer tiles
-// the two are within 5 % of one another, and one launch a call leaves the host free.
+// 280 x 472 in segments of 46 steps, 24.4 against 28.2.  Where the tiles of an FP32 forward trade across XCDs both ways and it has up
+// to 90,000 cells the launched form is the faster one (200 x 200: 1.05 against 0.97 at 238 steps, 3.7 against 3.5 at 1000); on
+// 16 tiles and fewer the two are within 10 % of one another, and one launch a call leaves the host free.
 // `between`: the pass runs beside resident ones (a Born source pass before them, a recompute between the
 // segments of a receiver pass), where a launched one takes this much longer a step.  Born adjoint, FP32, 139 x 90: 2.00 ms a
 // call with the source pass resident against 1.99 launched at 192 fine steps, 6.62 against 6.93 at 768; FWI forward and

@@ -213,6 +213,8 @@ def test_born_batch_runs_resident():
     (np.float32, 139, 61, 1, 51, True),      # 12 tiles, two an XCD
     (np.float32, 200, 200, 1, 120, False),   # 36 tiles that all trade across XCDs: launched steps are faster
     (np.float32, 200, 200, 4, 120, True),    # four of them: most of a shot on one XCD
+    (np.float32, 200, 200, 2, 120, True),    # two: nine tiles an XCD, three whole columns
+    (np.float32, 200, 330, 1, 120, False),   # 63 tiles, not whole columns, 66,000 cells
     (np.float32, 500, 480, 1, 120, True),    # enough cells for a step of its own length
     (np.float64, 200, 200, 1, 120, False), (np.float64, 200, 200, 4, 120, True), (np.float64, 280, 472, 1, 120, True)])
 def test_forward_takes_the_faster_form(dtype, nz, nx, nshot, nts, resident):
